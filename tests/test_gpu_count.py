@@ -196,3 +196,17 @@ def test_count_above_2_30_arcs(lstc):
         assert sup.shape[0] == m and bool((sup == k - 2).all()), split
         assert pv.shape[0] == n and bool((pv == (k - 1) * (k - 2) // 2).all()), split
         del sup, pv
+
+
+@pytest.mark.parametrize("n", [2, 3, 63, 65, 1023, 1025, 4095, 4096, 4097, 9001])
+def test_count_plan_sizes(lstc, oracle, n):
+    """Row counts on both sides of the one-workgroup plan's and its rounds' limits: plain, split and
+    with a partner in a batch (the batch's rows add up)."""
+    gn, s, d = oracle.gen_er(n, min(20.0, n - 1.0), seed=n)
+    sym, g = oracle.clean_orient(gn, s, d)
+    want = oracle.count(g)
+    plain = _upload(lstc, g)
+    split = lstc.in_lists(_upload(lstc, g))
+    k30 = lstc.in_lists(_upload(lstc, _oracle_graph(oracle, G.complete(30))[1]))
+    assert lstc.count(plain) == want and lstc.count(split) == want
+    assert lstc.count_batch([k30, split, plain]) == [30 * 29 * 28 // 6, want, want]

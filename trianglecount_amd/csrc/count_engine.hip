@@ -62,9 +62,21 @@ static constexpr int kTinyBin = kBins;                // the lane-per-arc rows
 static constexpr int kSlots = kBins + 1;              // queue regions
 static constexpr uint32_t kBigGroup = 2;              // big items per ticket
 
+// Tickets are dealt in classes: ticket t belongs to class t % classes, and each
+// class has its own head, on a 128-byte line of its own.  Workgroup b starts with
+// ticket b (no atomic) and goes on with its class, then with the others' leftovers.
+// A launch of a few hundred tickets then costs few atomics where every one of the
+// resident workgroups used to ask the one head (1009-vertex uniform graph: k_count
+// 39.5 -> 20 us), and launches of short items do not queue on one address (mixed
+// batch of 66 graphs: 3.02 ms with one class, 2.84 with eight; 64 served requests
+// 9.93 -> 9.31 ms).  Without in-lists the items are long and one class balances
+// them better (RMAT s21: 5.38 ms against 5.50).
+static constexpr uint32_t kHeads = 8;
+static constexpr uint32_t kHeadStride = 32;  // words between heads
+
 // ctl (uint32) layout
-enum { C_CNT = 0, C_HEAD = 12, C_NBIG = 13, C_NSMALL = 14, C_NTICK = 15, C_NTINY = 16, C_TINY0 = 17, C_NSMALLT = 18,
-       C_SGROUP = 19, C_WORDS = 20 };
+enum { C_CNT = 0, C_NBIG = 13, C_NSMALL = 14, C_NTICK = 15, C_NTINY = 16, C_TINY0 = 17, C_NSMALLT = 18,
+       C_SGROUP = 19, C_CLASSES = 20, C_HEADS = 32, C_WORDS = C_HEADS + kHeads * kHeadStride };
 
 // work item: row (bits 0-31) | chunk (32-51) | kind (52) | graph (53-63).
 // A row's in-degree is below 2^32 (m < 2^32), so its chunk index fits 20 bits.
@@ -180,9 +192,38 @@ __device__ __forceinline__ uint32_t table_log2_for(uint32_t keys, uint32_t scale
 __device__ __forceinline__ uint64_t umin64(uint64_t a, uint64_t b) { return a < b ? a : b; }
 
 // ------------------------------------------------------------------ planning
-__global__ void k_plan_init(uint32_t *ctl, unsigned long long *counts, uint32_t G) {
-    for (uint32_t i = threadIdx.x; i < C_WORDS; i += blockDim.x) ctl[i] = 0;
-    for (uint32_t i = threadIdx.x; i < G; i += blockDim.x) counts[i] = 0;
+// The ticket counts of a plan whose regions hold n_big, n_small and n_tiny items
+// (in this order in the queue), and what the count starts from: the heads behind
+// the first `grid` tickets (the workgroups' own) and zero counts.  Run by one
+// workgroup.
+// small_group 0: the planner picks the small items per ticket, the largest
+// power of two up to (small items per workgroup) / 32, within [16, 64]: about
+// 32-64 small tickets per workgroup (measured on RMAT s21 and s23: fewer,
+// larger tickets leave a ragged tail, more of them queue on the ticket heads).
+// A launch with less than 16 small items per workgroup takes one per wave, so
+// that its items spread over the chip (a 1009-vertex uniform graph has 2000).
+__device__ __forceinline__ void plan_tickets(uint32_t *ctl, uint32_t n_big, uint32_t n_small, uint32_t n_tiny,
+                                             uint32_t small_group, uint32_t grid, uint32_t waves, uint32_t classes,
+                                             uint32_t tid) {
+    if (tid < classes) ctl[C_HEADS + tid * kHeadStride] = (grid + classes - 1 - tid) / classes;
+    if (tid != 0) return;
+    ctl[C_CLASSES] = classes;
+    uint32_t sg = small_group;
+    if (sg == 0) {
+        const uint32_t per_wg = n_small / (grid ? grid : 1u);
+        sg = 16;
+        while (sg < 64 && 2 * sg <= per_wg / 32) sg *= 2;
+        if (per_wg < 16) sg = waves;
+    }
+    ctl[C_SGROUP] = sg;
+    const uint32_t small_t = (n_small + sg - 1) / sg;
+    const uint32_t tiny_t = (n_tiny + waves * 64 - 1) / (waves * 64);  // 64 rows per wave
+    ctl[C_NBIG] = n_big;
+    ctl[C_NSMALL] = n_small;
+    ctl[C_NSMALLT] = small_t;
+    ctl[C_NTINY] = n_tiny;
+    ctl[C_TINY0] = n_big + n_small;
+    ctl[C_NTICK] = (n_big + kBigGroup - 1) / kBigGroup + small_t + tiny_t;
 }
 
 // The plan splits the owned rows of the launch (graph after graph) into
@@ -191,12 +232,64 @@ __global__ void k_plan_init(uint32_t *ctl, unsigned long long *counts, uint32_t 
 // exclusive queue positions (slot-major: bins 5,4,3 = big, largest first, then
 // 2,1,0 = small); pass 1 writes the items, in row order within a bin and range.
 // No atomics: the queue is the same on every run.
-static constexpr uint32_t kPlanBlocks = 1024;
+static constexpr uint32_t kPlanBlocks = 1012;
 static constexpr uint32_t kPlanWaves = kPlanBlocks * 4;
 static constexpr uint32_t kPlanEntries = kSlots * kPlanWaves;
 
 // queue region of a bin: hash bins 5..0 in slots 0..5, the tiny rows in slot 6
 __device__ __forceinline__ int slot_of(int b) { return b < kBins ? kBins - 1 - b : kTinyBin; }
+
+// What one planned row puts into the queue.
+struct RowPlan {
+    int bin = -1;  // -1: nothing
+    uint32_t g = 0, u = 0, n_a = 0, n_b = 0, tiny_kind = 0;
+    __device__ __forceinline__ uint32_t items() const { return bin < 0 ? 0u : bin == kTinyBin ? 1u : n_a + n_b; }
+    __device__ __forceinline__ void write(unsigned long long *q) const {
+        if (bin == kTinyBin) {
+            q[0] = make_item(g, tiny_kind, 0, u);
+        } else {
+            if (n_a) *q++ = make_item(g, 0, 0, u);
+            for (uint32_t j = 0; j < n_b; ++j) q[j] = make_item(g, 1, j, u);
+        }
+    }
+};
+
+// Planned row r of the launch (r < total_rows).
+__device__ __forceinline__ RowPlan plan_row(const GraphSet &gs, const Bounds &bd, uint64_t r) {
+    RowPlan p;
+    if (gs.table) {  // last g with row_base[g] <= r
+        uint32_t lo = 0, hi = gs.G;
+        while (hi - lo > 1) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (gload(gs.row_base + mid) <= r) lo = mid; else hi = mid;
+        }
+        p.g = lo;
+        p.u = (uint32_t)(r - gload(gs.row_base + lo));
+    } else {
+        p.u = (uint32_t)r;
+    }
+    const GraphDev G = graph_at(gs, p.g);
+    const bool owned = p.u < G.n_owned;  // rows past n_owned are visited only for split counting
+    const uint64_t k = gload(G.off + p.u + 1) - gload(G.off + p.u);
+    const uint64_t kb = G.in_off ? gload(G.in_off + p.u + 1) - gload(G.in_off + p.u) : 0;
+    if (k >= 2 && G.in_off && k <= bd.tiny_max) {
+        // one entry; kind 1 = in side only (a halo row owns no out side)
+        if (owned || kb) {
+            p.bin = kTinyBin;
+            p.tiny_kind = owned ? 0u : 1u;
+        }
+    } else if (k >= 2) {
+        const uint32_t sb = in_chunk(kb);
+        p.n_a = owned ? 1u : 0u;
+        p.n_b = (uint32_t)((kb + sb - 1) / sb);
+        if (p.n_a + p.n_b) {
+            p.bin = kBins - 1;
+            for (int i = kBins - 2; i >= 0; --i)
+                if (k <= bd.hi[i]) p.bin = i;
+        }
+    }
+    return p;
+}
 
 template <int PASS>
 __global__ __launch_bounds__(256) void k_plan_rows(GraphSet gs, Bounds bd, uint32_t *__restrict__ wcnt,
@@ -211,59 +304,18 @@ __global__ __launch_bounds__(256) void k_plan_rows(GraphSet gs, Bounds bd, uint3
     for (int i = 0; i < kSlots; ++i) run[i] = PASS == 1 ? wcnt[slot_of(i) * kPlanWaves + wave] : 0u;
     for (uint64_t r0 = r_begin; r0 < r_end; r0 += 64) {
         const uint64_t r = r0 + lane;
-        int b = -1;
-        uint32_t g = 0, u = 0, n_a = 0, n_b = 0, tiny_kind = 0;
-        if (r < r_end) {
-            if (gs.table) {  // last g with row_base[g] <= r
-                uint32_t lo = 0, hi = gs.G;
-                while (hi - lo > 1) {
-                    const uint32_t mid = (lo + hi) >> 1;
-                    if (gload(gs.row_base + mid) <= r) lo = mid; else hi = mid;
-                }
-                g = lo;
-                u = (uint32_t)(r - gload(gs.row_base + g));
-            } else {
-                u = (uint32_t)r;
-            }
-            const GraphDev G = graph_at(gs, g);
-            const bool owned = u < G.n_owned;  // rows past n_owned are visited only for split counting
-            const uint64_t k = gload(G.off + u + 1) - gload(G.off + u);
-            const uint64_t kb = G.in_off ? gload(G.in_off + u + 1) - gload(G.in_off + u) : 0;
-            if (k >= 2 && G.in_off && k <= bd.tiny_max) {
-                // one entry; kind 1 = in side only (a halo row owns no out side)
-                if (owned || kb) {
-                    b = kTinyBin;
-                    tiny_kind = owned ? 0u : 1u;
-                }
-            } else if (k >= 2) {
-                const uint32_t sb = in_chunk(kb);
-                n_a = owned ? 1u : 0u;
-                n_b = (uint32_t)((kb + sb - 1) / sb);
-                if (n_a + n_b) {
-                    b = kBins - 1;
-                    for (int i = kBins - 2; i >= 0; --i)
-                        if (k <= bd.hi[i]) b = i;
-                }
-            }
-        }
-        const uint32_t n_items = b == kTinyBin ? 1u : n_a + n_b;
+        RowPlan p;
+        if (r < r_end) p = plan_row(gs, bd, r);
+        const int b = p.bin;
 #pragma unroll
         for (int i = 0; i < kSlots; ++i) {
             if (ballot(b == i) == 0) continue;
-            const uint32_t c = (b == i) ? n_items : 0u;
+            const uint32_t c = (b == i) ? p.items() : 0u;
             if (PASS == 0) {
                 run[i] += c;
             } else {
                 const uint32_t incl = wave_incl_scan(c, lane);
-                if (b == i) {
-                    unsigned long long *q = queue + run[i] + (incl - c);
-                    if (b == kTinyBin) {
-                        q[0] = make_item(g, tiny_kind, 0, u);
-                    } else {
-                        if (n_a) *q++ = make_item(g, 0, 0, u);
-                        for (uint32_t j = 0; j < n_b; ++j) q[j] = make_item(g, 1, j, u);
-                    }
-                }
+                if (b == i) p.write(queue + run[i] + (incl - c));
                 run[i] += read_lane(incl, 63);
             }
         }
@@ -278,24 +330,26 @@ __global__ __launch_bounds__(256) void k_plan_rows(GraphSet gs, Bounds bd, uint3
 }
 
 // One workgroup of 1024: exclusive scan of wcnt in place (kPlanEntries values,
-// 24 per thread), then the ticket counts.  Item totals stay below 2^32
+// 28 per thread), then the ticket counts.  Item totals stay below 2^32
 // (checked on the host against the queue capacity).
-// small_group 0: the planner picks the small items per ticket, the largest
-// power of two up to (small items per workgroup) / 32, within [16, 64]: about
-// 32-64 small tickets per workgroup (measured on RMAT s21 and s23: fewer,
-// larger tickets leave a ragged tail, more of them queue on the ticket head).
 __global__ __launch_bounds__(1024) void k_plan_scan(uint32_t *__restrict__ wcnt, uint32_t *__restrict__ ctl,
-                                                    uint32_t small_group, uint32_t grid, uint32_t waves) {
-    constexpr uint32_t kPer = kPlanEntries / 1024;
-    static_assert(kPlanEntries % 1024 == 0, "plan entries per thread");
+                                                    unsigned long long *__restrict__ counts, uint32_t G,
+                                                    uint32_t small_group, uint32_t grid, uint32_t waves, uint32_t classes) {
+    constexpr uint32_t kPer = (kPlanEntries + 4095) / 4096 * 4;  // 16-byte loads and stores
+    static_assert(kPlanEntries % 4 == 0, "plan entries come in whole 16-byte words");
     __shared__ uint32_t s_wave[16];
     __shared__ uint32_t s_slot[kSlots + 1];
     const uint32_t tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     uint32_t v[kPer];
+#pragma unroll
+    for (uint32_t i = 0; i < kPer; i += 4) {
+        const uint32_t e = tid * kPer + i;
+        const uint4 q = e < kPlanEntries ? *(const uint4 *)(wcnt + e) : uint4{0, 0, 0, 0};
+        v[i] = q.x, v[i + 1] = q.y, v[i + 2] = q.z, v[i + 3] = q.w;
+    }
     uint32_t sum = 0;
 #pragma unroll
     for (uint32_t i = 0; i < kPer; ++i) {
-        v[i] = wcnt[tid * kPer + i];
         sum += v[i];
     }
     const uint32_t incl = wave_incl_scan(sum, lane);
@@ -307,35 +361,77 @@ __global__ __launch_bounds__(1024) void k_plan_scan(uint32_t *__restrict__ wcnt,
 #pragma unroll
     for (uint32_t i = 0; i < kPer; ++i) {
         const uint32_t e = tid * kPer + i;
-        if (e % kPlanWaves == 0) s_slot[e / kPlanWaves] = run;
-        wcnt[e] = run;
-        run += v[i];
+        if (e < kPlanEntries && e % kPlanWaves == 0) s_slot[e / kPlanWaves] = run;
+        const uint32_t x = v[i];
+        v[i] = run;
+        run += x;
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < kPer; i += 4) {
+        const uint32_t e = tid * kPer + i;
+        if (e < kPlanEntries) *(uint4 *)(wcnt + e) = uint4{v[i], v[i + 1], v[i + 2], v[i + 3]};
     }
     if (tid == 1023) s_slot[kSlots] = run;
     __syncthreads();
-    if (tid == 0) {
-        // slots 0..2 hold bins 5,4,3 (big), slots 3..5 bins 2,1,0 (small), slot 6 the tiny rows
-        const uint32_t n_big = s_slot[3] - s_slot[0];
-        const uint32_t n_small = s_slot[6] - s_slot[3];
-        const uint32_t n_tiny = s_slot[7] - s_slot[6];
-        for (int b = 0; b < kBins; ++b) ctl[C_CNT + b] = s_slot[kBins - b] - s_slot[kBins - 1 - b];
-        uint32_t sg = small_group;
-        if (sg == 0) {
-            const uint32_t per_wg = n_small / (grid ? grid : 1u) / 32u;
-            sg = 16;
-            while (sg < 64 && 2 * sg <= per_wg) sg *= 2;
-        }
-        ctl[C_SGROUP] = sg;
-        const uint32_t small_t = (n_small + sg - 1) / sg;
-        const uint32_t tiny_t = (n_tiny + waves * 64 - 1) / (waves * 64);  // 64 rows per wave
-        ctl[C_NBIG] = n_big;
-        ctl[C_NSMALL] = n_small;
-        ctl[C_NSMALLT] = small_t;
-        ctl[C_NTINY] = n_tiny;
-        ctl[C_TINY0] = s_slot[6];
-        ctl[C_NTICK] = (n_big + kBigGroup - 1) / kBigGroup + small_t + tiny_t;
-        ctl[C_HEAD] = 0;
+    for (uint32_t i = tid; i < G; i += 1024) counts[i] = 0;
+    // slots 0..2 hold bins 5,4,3 (big), slots 3..5 bins 2,1,0 (small), slot 6 the tiny rows
+    plan_tickets(ctl, s_slot[3], s_slot[6] - s_slot[3], s_slot[7] - s_slot[6], small_group, grid, waves, classes, tid);
+}
+
+// The whole plan of a launch of at most kSmallPlan rows in one workgroup: the
+// same queue regions (rows in another order within a bin), one launch instead of
+// three, each of which would cost more than the work of this one.
+static constexpr uint32_t kSmallPlanPer = 4;
+static constexpr uint32_t kSmallPlan = 1024 * kSmallPlanPer;
+
+__global__ __launch_bounds__(1024) void k_plan_small(GraphSet gs, Bounds bd, uint32_t *__restrict__ ctl,
+                                                     unsigned long long *__restrict__ queue,
+                                                     unsigned long long *__restrict__ counts, uint32_t small_group,
+                                                     uint32_t grid, uint32_t waves, uint32_t classes) {
+    __shared__ uint32_t s_wave[kSlots][16];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    RowPlan p[kSmallPlanPer];
+#pragma unroll
+    for (uint32_t i = 0; i < kSmallPlanPer; ++i) {
+        const uint64_t r = (uint64_t)i * 1024 + tid;
+        if (r < gs.total_rows) p[i] = plan_row(gs, bd, r);
     }
+    uint32_t mine[kSlots], excl[kSlots];  // this thread's items per slot, and its place within the wave
+#pragma unroll
+    for (int s = 0; s < kSlots; ++s) {
+        uint32_t c = 0;
+#pragma unroll
+        for (uint32_t i = 0; i < kSmallPlanPer; ++i) c += p[i].bin >= 0 && slot_of(p[i].bin) == s ? p[i].items() : 0u;
+        const uint32_t incl = wave_incl_scan(c, lane);
+        mine[s] = c;
+        excl[s] = incl - c;
+        if (lane == 63) s_wave[s][wv] = incl;
+    }
+    __syncthreads();
+    uint32_t base = 0, n_big = 0, n_small = 0;  // first queue position of the slot
+#pragma unroll
+    for (int s = 0; s < kSlots; ++s) {
+        uint32_t before = 0, total = 0;
+        for (uint32_t w = 0; w < 16; ++w) {
+            const uint32_t v = s_wave[s][w];
+            before += w < wv ? v : 0u;
+            total += v;
+        }
+        uint32_t pos = base + before + excl[s];
+        if (mine[s]) {
+#pragma unroll
+            for (uint32_t i = 0; i < kSmallPlanPer; ++i) {
+                if (p[i].bin < 0 || slot_of(p[i].bin) != s) continue;
+                p[i].write(queue + pos);
+                pos += p[i].items();
+            }
+        }
+        base += total;
+        if (s == 2) n_big = base;
+        if (s == 5) n_small = base - n_big;
+    }
+    for (uint32_t i = tid; i < gs.G; i += 1024) counts[i] = 0;
+    plan_tickets(ctl, n_big, n_small, base - n_big - n_small, small_group, grid, waves, classes, tid);
 }
 
 // ------------------------------------------------------------------ table build
@@ -698,6 +794,31 @@ __device__ __forceinline__ uint32_t tiny_walk(const GraphDev &G, bool mine, bool
     return wave_sum32(lane_hits);
 }
 
+// ------------------------------------------------------------------ tickets
+// One thread's view of the ticket heads: its class's next ticket, and when that
+// class has run out, the other classes' leftovers, each class left for good once
+// it is empty (kEmpty when none is left).  Asking before the current ticket's work
+// rather than after it was slower (s23 17.06 against 16.90 ms): the loads of the
+// asking wave wait behind the atomic.
+struct Tickets {
+    uint32_t *heads;
+    uint32_t n, classes, cls;
+    __device__ __forceinline__ Tickets(uint32_t *ctl, uint32_t n_tickets)
+        : heads(ctl + C_HEADS), n(n_tickets), classes(sload(ctl + C_CLASSES)), cls(blockIdx.x % classes) {}
+    // A head never passes its class's ticket count by more than the workgroups
+    // asking, so a ticket number stays below 2^32.
+    __device__ __forceinline__ uint32_t next() {
+        uint64_t t = (uint64_t)atomicAdd(heads + cls * kHeadStride, 1u) * classes + cls;
+        for (uint32_t left = classes - 1; t >= n && left; --left) {
+            cls = cls + 1 == classes ? 0 : cls + 1;
+            uint32_t *head = heads + cls * kHeadStride;
+            const uint32_t h = __hip_atomic_load(head, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if ((uint64_t)h * classes + cls < n) t = (uint64_t)atomicAdd(head, 1u) * classes + cls;
+        }
+        return t < n ? (uint32_t)t : kEmpty;
+    }
+};
+
 // ------------------------------------------------------------------ persistent count kernel
 // NARROW: every graph of the launch has m <= 2^30 arcs (and a streaming copy of at
 // most 2^30 entries).
@@ -714,7 +835,7 @@ __global__ __launch_bounds__(WAVES * 64, UNROLL == 4 ? 8 : 6) void k_count(Graph
     __shared__ uint32_t s_end[WAVES][64];
     __shared__ __align__(16) uint32_t s_flag[WAVES][16];  // 64 position flags per wave (tiny rows)
     __shared__ uint8_t s_src[WAVES][64];
-    __shared__ uint32_t s_ticket;
+    __shared__ uint32_t s_ticket[2];
     __shared__ unsigned long long s_acc[WAVES];
     __shared__ uint32_t s_g[WAVES];
 
@@ -729,12 +850,9 @@ __global__ __launch_bounds__(WAVES * 64, UNROLL == 4 ? 8 : 6) void k_count(Graph
     uint32_t cur_g = kEmpty;
     unsigned long long acc = 0;
 
-    for (;;) {
-        if (tid == 0) s_ticket = atomicAdd(ctl + C_HEAD, 1u);
-        __syncthreads();
-        const uint32_t t = uniform(s_ticket);
-        __syncthreads();
-        if (t >= n_tickets) break;
+    Tickets tk(ctl, n_tickets);
+    uint32_t turn = 0;
+    for (uint32_t t = blockIdx.x; t < n_tickets;) {
         if (t < n_bigt) {
           // big items (kBigGroup per ticket): the whole workgroup shares one table
           for (uint32_t bi = t * kBigGroup, be = min(bi + kBigGroup, n_big); bi < be; ++bi) {
@@ -820,6 +938,12 @@ __global__ __launch_bounds__(WAVES * 64, UNROLL == 4 ? 8 : 6) void k_count(Graph
                 if (G.per_row && lane == 0) G.per_row[u] = hits;
             }
         }
+        // two slots in turn: a slot is written again only after the barrier that
+        // every wave passes with its last reading of it behind
+        if (tid == 0) s_ticket[turn] = tk.next();
+        __syncthreads();
+        t = uniform(s_ticket[turn]);
+        turn ^= 1u;
     }
     // one atomic per graph per workgroup for what the waves still hold
     if (lane == 0) { s_acc[wv] = acc; s_g[wv] = cur_g; }
@@ -857,7 +981,7 @@ static uint64_t queue_cap(uint64_t total_rows, uint64_t total_m) { return 2 * to
 size_t count_ws_bytes(uint32_t G, uint64_t total_rows, uint64_t total_m) {
     (void)G;
     Carver c(nullptr, 0);
-    c.take<uint32_t>(64);
+    c.take<uint32_t>(C_WORDS);
     c.take<uint32_t>(kPlanEntries);
     c.take<unsigned long long>(queue_cap(total_rows, total_m));
     return c.need();
@@ -880,7 +1004,7 @@ lstc_status count_launch(const HostGraph *hosts, uint32_t G, const GraphDev *d_t
     Carver c(ws, ws_bytes);
     if (queue_cap(total, total_m) >= 0xFFFFFFFFull)
         return fail(LSTC_ERR_INVALID, "count: more than 2^32-1 work items in one launch");
-    uint32_t *ctl = c.take<uint32_t>(64);
+    uint32_t *ctl = c.take<uint32_t>(C_WORDS);
     uint32_t *wcnt = c.take<uint32_t>(kPlanEntries);
     unsigned long long *queue = c.take<unsigned long long>(queue_cap(total, total_m));
     if (!ws || !c.ok()) return fail(LSTC_ERR_WORKSPACE, "count: workspace %zu < %zu bytes", ws_bytes, c.need());
@@ -896,35 +1020,41 @@ lstc_status count_launch(const HostGraph *hosts, uint32_t G, const GraphDev *d_t
     }
     for (uint32_t g = 0; g < G; ++g)
         if (hosts[g].per_row) LSTC_TRY(fill_u64(hosts[g].per_row, 0, hosts[g].n_owned, st));
-    hipLaunchKernelGGL(k_plan_init, dim3(1), dim3(256), 0, st, ctl, d_counts, G);
-    LSTC_LAUNCHED("k_plan_init");
+    if (total == 0) return fill_u64((uint64_t *)d_counts, 0, G, st);
     const int cus = device_cus();
     Bounds bd{{16, 64, tr.small_max, 1024, 2048, 0xFFFFFFFFu}, tr.tiny_max};
-    if (total) {
+    bool narrow = true;
+    for (uint32_t g = 0; g < G; ++g)
+        narrow = narrow && hosts[g].m <= (1ull << 30) && hosts[g].scol_len <= (1ull << 30);
+    using Kern = void (*)(GraphSet, const unsigned long long *, uint32_t *, unsigned long long *, uint32_t);
+    // [unroll 4/8][narrow][waves 2/4/8]
+    static const Kern kerns[2][2][3] = {
+        {{k_count<4, false, 2>, k_count<4, false, 4>, k_count<4, false, 8>},
+         {k_count<4, true, 2>, k_count<4, true, 4>, k_count<4, true, 8>}},
+        {{k_count<8, false, 2>, k_count<8, false, 4>, k_count<8, false, 8>},
+         {k_count<8, true, 2>, k_count<8, true, 4>, k_count<8, true, 8>}}};
+    const Kern kern = kerns[tr.unroll == 8][narrow][tr.waves == 2 ? 0 : tr.waves == 4 ? 1 : 2];
+    // a persistent grid beyond what fits at once would only wait for the queue to drain
+    uint32_t grid = (uint32_t)cus * tr.grid_per_cu;
+    const uint32_t fit = resident_blocks((const void *)kern, tr.waves * 64);
+    if (fit && grid > (uint32_t)cus * fit) grid = (uint32_t)cus * fit;
+    bool split = false;
+    for (uint32_t g = 0; g < G; ++g) split = split || split_ok(hosts[g]);
+    const uint32_t classes = split ? kHeads : 1u;
+    if (total <= kSmallPlan) {
+        hipLaunchKernelGGL(k_plan_small, dim3(1), dim3(1024), 0, st, gs, bd, ctl, queue, d_counts, tr.small_group, grid,
+                           tr.waves, classes);
+        LSTC_LAUNCHED("k_plan_small");
+    } else {
         hipLaunchKernelGGL(k_plan_rows<0>, dim3(kPlanBlocks), dim3(256), 0, st, gs, bd, wcnt, queue);
         LSTC_LAUNCHED("k_plan_rows<0>");
-        hipLaunchKernelGGL(k_plan_scan, dim3(1), dim3(1024), 0, st, wcnt, ctl, tr.small_group,
-                           (uint32_t)cus * tr.grid_per_cu, tr.waves);
+        hipLaunchKernelGGL(k_plan_scan, dim3(1), dim3(1024), 0, st, wcnt, ctl, d_counts, G, tr.small_group, grid,
+                           tr.waves, classes);
         LSTC_LAUNCHED("k_plan_scan");
         hipLaunchKernelGGL(k_plan_rows<1>, dim3(kPlanBlocks), dim3(256), 0, st, gs, bd, wcnt, queue);
         LSTC_LAUNCHED("k_plan_rows<1>");
     }
-    if (total) {
-        uint32_t grid = (uint32_t)cus * tr.grid_per_cu;
-        bool narrow = true;
-        for (uint32_t g = 0; g < G; ++g)
-            narrow = narrow && hosts[g].m <= (1ull << 30) && hosts[g].scol_len <= (1ull << 30);
-        using Kern = void (*)(GraphSet, const unsigned long long *, uint32_t *, unsigned long long *, uint32_t);
-        // [unroll 4/8][narrow][waves 2/4/8]
-        static const Kern kerns[2][2][3] = {
-            {{k_count<4, false, 2>, k_count<4, false, 4>, k_count<4, false, 8>},
-             {k_count<4, true, 2>, k_count<4, true, 4>, k_count<4, true, 8>}},
-            {{k_count<8, false, 2>, k_count<8, false, 4>, k_count<8, false, 8>},
-             {k_count<8, true, 2>, k_count<8, true, 4>, k_count<8, true, 8>}}};
-        const Kern kern = kerns[tr.unroll == 8][narrow][tr.waves == 2 ? 0 : tr.waves == 4 ? 1 : 2];
-        // a persistent grid beyond what fits at once would only wait for the queue to drain
-        const uint32_t fit = resident_blocks((const void *)kern, tr.waves * 64);
-        if (fit && grid > (uint32_t)cus * fit) grid = (uint32_t)cus * fit;
+    {
         const TimingMark tm = timed ? timing_begin(st) : TimingMark{nullptr, nullptr};
         hipLaunchKernelGGL(kern, dim3(grid), dim3(tr.waves * 64), 0, st, gs, queue, ctl, d_counts, tr.table_scale);
         LSTC_LAUNCHED("k_count");
