@@ -210,3 +210,71 @@ def test_count_plan_sizes(lstc, oracle, n):
     k30 = lstc.in_lists(_upload(lstc, _oracle_graph(oracle, G.complete(30))[1]))
     assert lstc.count(plain) == want and lstc.count(split) == want
     assert lstc.count_batch([k30, split, plain]) == [30 * 29 * 28 // 6, want, want]
+
+
+def _hub_graphs(O):
+    """Graphs that are counted from hub codes when they carry a streaming copy, and neighbours of the rule:
+    more vertices than codes (tails), fewer (no tails), rows all of bitmaps, many chunks per row, a uniform
+    graph whose hubs cover too little (counted from ids), and one with too few arcs per row."""
+    return {
+        "rmat_s17": lambda: O.gen_rmat(17, 16, seed=5),
+        "rmat_s16_dense": lambda: O.gen_rmat(16, 40, seed=2),
+        "chung_lu": lambda: O.gen_chung_lu(100_000, 2.1, 50, 5e3, seed=3),
+        "er_dense": lambda: O.gen_er(2311, 1200.0, seed=4),
+        "K1501": lambda: G.complete(1501),
+        "hub_lists": lambda: _hub_lists(70_001, 300, 30),
+        "er_uniform": lambda: O.gen_er(130_001, 40.0, seed=6),
+        "er_sparse": lambda: O.gen_er(150_001, 20.0, seed=7),
+    }
+
+
+def _hub_lists(n, hubs, deg):
+    """`hubs` vertices joined to each other and to everyone by random edges: in-lists of thousands of rows."""
+    rng = np.random.default_rng(11)
+    src = np.repeat(np.arange(n, dtype=np.uint32), deg)
+    dst = rng.integers(0, hubs, n * deg).astype(np.uint32)
+    iu, ju = np.triu_indices(hubs, 1)
+    return n, np.concatenate([src, iu.astype(np.uint32)]), np.concatenate([dst, ju.astype(np.uint32)])
+
+
+@pytest.mark.parametrize("name", ["rmat_s17", "rmat_s16_dense", "chung_lu", "er_dense", "K1501", "hub_lists", "er_uniform",
+                                  "er_sparse"])
+def test_count_from_hub_codes(lstc, oracle, name):
+    n, s, d = _hub_graphs(oracle)[name]()
+    want = oracle.count(oracle.clean_orient(n, s, d)[1])
+    up = lambda a: torch.from_numpy(np.ascontiguousarray(a).view(np.int32)).cuda()  # noqa: E731
+    g = lstc.clean_orient(n, up(s), up(d), in_lists=True, stream_copy=True)
+    assert [lstc.count(g) for _ in range(2)] == [want, want]
+    assert lstc.count(g, tune=lstc.Tune(tiny_max=1)) == want and lstc.count(g, tune=lstc.Tune(small_group=200)) == want
+    plan = lstc.BatchPlan([g])
+    try:
+        for _ in range(3):
+            plan.counts.fill_(7)
+            plan.launch_graph()
+            assert plan.results() == [want]
+    finally:
+        plan.close()
+    # a workspace without room for the codes: counted from the ids
+    small = torch.empty(16 * g.n + g.m // 64 + (1 << 18), dtype=torch.uint8, device="cuda")
+    out = torch.zeros(1, dtype=torch.int64, device="cuda")
+    p = lambda t: t.data_ptr()  # noqa: E731
+    lstc.check(lstc.load().lstc_count_split_stream(p(g.off), p(g.col), p(g.in_off), p(g.in_col), p(g.col_seg), p(g.in_seg),
+                                                   p(g.scol), g.scol.numel(), g.n, g.n, g.m, p(out), None, p(small),
+                                                   small.numel(), None), "lstc_count_split_stream")
+    torch.cuda.synchronize()
+    assert int(out.item()) == want
+
+
+def test_count_halo_part_from_hub_codes(lstc, oracle):
+    """Halo rows own no arcs but stream and are streamed: a part of RMAT s18 with its streaming copy."""
+    n, s, d = lstc.generate_rmat(18, 16, seed=9)
+    g = lstc.clean_orient(n, s, d, keep_symmetric=True)
+    part = lstc.partition_random(g.n, 2, seed=4)
+    total = 0
+    for p in range(2):
+        h = lstc.stream_copy(lstc.halo_extract(g, part, p, split=True))
+        assert h.owned < h.n and h.m >= max(1 << 20, 16 * h.n)
+        c = lstc.count(h)
+        assert c == lstc.count(h, split=False)
+        total += c
+    assert total == lstc.count(g)

@@ -13,7 +13,7 @@ extern "C" lstc_status lstc_count_workspace(uint32_t n_rows, uint32_t n_owned, u
                                             const lstc_tune *tune, size_t *bytes) {
     (void)n_owned; (void)tune;
     if (!bytes) return fail(LSTC_ERR_INVALID, "lstc_count_workspace: bytes is NULL");
-    *bytes = count_ws_bytes(1, n_rows, m);  // split counting plans every row
+    *bytes = count_ws_bytes(n_rows, m);  // split counting plans every row
     return LSTC_OK;
 }
 

@@ -94,9 +94,12 @@ TuneR effective_tune(const lstc_tune *t, uint64_t total_m);
 
 lstc_status validate_graph(const HostGraph &h, const char *who);
 
-// Workspace for a launch over G graphs with total_rows owned rows and total_m
-// arcs (excludes the batch descriptor table, which the caller places).
-size_t count_ws_bytes(uint32_t G, uint64_t total_rows, uint64_t total_m);
+// Workspace for a launch over graphs with total_rows planned rows and total_m
+// arcs (excludes the batch descriptor table, which the caller places): what every
+// launch needs, and with the arrays that the count over 16-bit codes takes besides
+// (hubcode.h).  count_launch runs with either; with the second it may use codes.
+size_t count_ws_base(uint64_t total_rows, uint64_t total_m);
+size_t count_ws_bytes(uint64_t total_rows, uint64_t total_m);
 // Largest batch one launch can address (graph ids are packed into work items).
 constexpr uint32_t kMaxGraphs = 2047;
 

@@ -42,6 +42,8 @@
 #include <unordered_map>
 
 #include "count_engine.h"
+#include "hubplan.h"
+#include "hubwalk.h"
 #include "segwalk.h"
 #include "wave.h"
 
@@ -293,7 +295,8 @@ __device__ __forceinline__ RowPlan plan_row(const GraphSet &gs, const Bounds &bd
 
 template <int PASS>
 __global__ __launch_bounds__(256) void k_plan_rows(GraphSet gs, Bounds bd, uint32_t *__restrict__ wcnt,
-                                                   unsigned long long *__restrict__ queue) {
+                                                   unsigned long long *__restrict__ queue, HubSet hs) {
+    if (hs.hctl && sload(hs.hctl + HC_ON)) return hub_plan_rows<PASS>(gs.one, hs, bd.tiny_max);
     const uint32_t lane = lane_id();
     const uint32_t wave = blockIdx.x * 4 + (threadIdx.x >> 6);
     const uint64_t total = gs.total_rows;
@@ -334,7 +337,9 @@ __global__ __launch_bounds__(256) void k_plan_rows(GraphSet gs, Bounds bd, uint3
 // (checked on the host against the queue capacity).
 __global__ __launch_bounds__(1024) void k_plan_scan(uint32_t *__restrict__ wcnt, uint32_t *__restrict__ ctl,
                                                     unsigned long long *__restrict__ counts, uint32_t G,
-                                                    uint32_t small_group, uint32_t grid, uint32_t waves, uint32_t classes) {
+                                                    uint32_t small_group, uint32_t grid, uint32_t waves, uint32_t classes,
+                                                    HubSet hs, uint32_t hub_grid) {
+    if (hs.hctl && sload(hs.hctl + HC_ON)) return hub_plan_scan(hs, counts, hub_grid);
     constexpr uint32_t kPer = (kPlanEntries + 4095) / 4096 * 4;  // 16-byte loads and stores
     static_assert(kPlanEntries % 4 == 0, "plan entries come in whole 16-byte words");
     __shared__ uint32_t s_wave[16];
@@ -621,11 +626,11 @@ __device__ __forceinline__ uint32_t walk(const uint64_t *__restrict__ off, const
         {
             const uint32_t sg = first_segment(0, myend);
             if (RB > total)
-                index_walk<UNROLL, false, NARROW>(0, total, mybase, myend, sg, lane, idx);
+                index_walk<UNROLL, false, col_shift<NARROW>()>(0, total, mybase, myend, sg, lane, idx);
             else if (one_segment<UNROLL>(0, myend))
-                index_single<UNROLL, NARROW>((uint32_t)__builtin_amdgcn_readlane((int)mybase, (int)sg), lane, idx);
+                index_single<UNROLL, col_shift<NARROW>()>((uint32_t)__builtin_amdgcn_readlane((int)mybase, (int)sg), lane, idx);
             else
-                index_walk<UNROLL, true, NARROW>(0, total, mybase, myend, sg, lane, idx);
+                index_walk<UNROLL, true, col_shift<NARROW>()>(0, total, mybase, myend, sg, lane, idx);
         }
         load_round<UNROLL, NARROW>(col, idx, xa);
         uint32_t B = 0;
@@ -633,17 +638,17 @@ __device__ __forceinline__ uint32_t walk(const uint64_t *__restrict__ off, const
             // rounds B + RB and B + 2 * RB are full
             uint32_t sg = first_segment(B + RB, myend);
             if (one_segment<UNROLL>(B + RB, myend))
-                index_single<UNROLL, NARROW>((uint32_t)__builtin_amdgcn_readlane((int)mybase, (int)sg) + B + RB, lane, idx);
+                index_single<UNROLL, col_shift<NARROW>()>((uint32_t)__builtin_amdgcn_readlane((int)mybase, (int)sg) + B + RB, lane, idx);
             else
-                index_walk<UNROLL, true, NARROW>(B + RB, total, mybase, myend, sg, lane, idx);
+                index_walk<UNROLL, true, col_shift<NARROW>()>(B + RB, total, mybase, myend, sg, lane, idx);
             load_round<UNROLL, NARROW>(col, idx, xb);
             probe_round<UNROLL, true>(xa, B, total, tab, qmask, qshift, lane, lane_hits, s_base, qn);
             sg = first_segment(B + 2 * RB, myend);
             if (one_segment<UNROLL>(B + 2 * RB, myend))
-                index_single<UNROLL, NARROW>((uint32_t)__builtin_amdgcn_readlane((int)mybase, (int)sg) + B + 2 * RB, lane,
+                index_single<UNROLL, col_shift<NARROW>()>((uint32_t)__builtin_amdgcn_readlane((int)mybase, (int)sg) + B + 2 * RB, lane,
                                      idx);
             else
-                index_walk<UNROLL, true, NARROW>(B + 2 * RB, total, mybase, myend, sg, lane, idx);
+                index_walk<UNROLL, true, col_shift<NARROW>()>(B + 2 * RB, total, mybase, myend, sg, lane, idx);
             load_round<UNROLL, NARROW>(col, idx, xa);
             probe_round<UNROLL, true>(xb, B + RB, total, tab, qmask, qshift, lane, lane_hits, s_base, qn);
         }
@@ -652,11 +657,11 @@ __device__ __forceinline__ uint32_t walk(const uint64_t *__restrict__ off, const
         if (B + RB >= total) {
             probe_round<UNROLL, false>(xa, B, total, tab, qmask, qshift, lane, lane_hits, s_base, qn);
         } else {
-            index_walk<UNROLL, false, NARROW>(B + RB, total, mybase, myend, first_segment(B + RB, myend), lane, idx);
+            index_walk<UNROLL, false, col_shift<NARROW>()>(B + RB, total, mybase, myend, first_segment(B + RB, myend), lane, idx);
             load_round<UNROLL, NARROW>(col, idx, xb);
             probe_round<UNROLL, true>(xa, B, total, tab, qmask, qshift, lane, lane_hits, s_base, qn);
             if (B + 2 * RB < total) {
-                index_walk<UNROLL, false, NARROW>(B + 2 * RB, total, mybase, myend, first_segment(B + 2 * RB, myend), lane,
+                index_walk<UNROLL, false, col_shift<NARROW>()>(B + 2 * RB, total, mybase, myend, first_segment(B + 2 * RB, myend), lane,
                                           idx);
                 load_round<UNROLL, NARROW>(col, idx, xa);
                 probe_round<UNROLL, true>(xb, B + RB, total, tab, qmask, qshift, lane, lane_hits, s_base, qn);
@@ -819,6 +824,24 @@ struct Tickets {
     }
 };
 
+// One atomic per graph per workgroup for what its waves still hold.
+template <int WAVES>
+__device__ __forceinline__ void flush_counts(unsigned long long *counts, unsigned long long *s_acc, uint32_t *s_g,
+                                             unsigned long long acc, uint32_t cur_g, uint32_t tid, uint32_t wv,
+                                             uint32_t lane) {
+    if (lane == 0) { s_acc[wv] = acc; s_g[wv] = cur_g; }
+    __syncthreads();
+    if (tid == 0) {
+        for (int i = 0; i < WAVES; ++i) {
+            if (s_g[i] == kEmpty) continue;
+            unsigned long long sum = s_acc[i];
+            for (int j = i + 1; j < WAVES; ++j)
+                if (s_g[j] == s_g[i]) { sum += s_acc[j]; s_g[j] = kEmpty; }
+            if (sum) atomicAdd(counts + s_g[i], sum);
+        }
+    }
+}
+
 // ------------------------------------------------------------------ persistent count kernel
 // NARROW: every graph of the launch has m <= 2^30 arcs (and a streaming copy of at
 // most 2^30 entries).
@@ -827,7 +850,8 @@ struct Tickets {
 template <int UNROLL, bool NARROW, int WAVES>
 __global__ __launch_bounds__(WAVES * 64, UNROLL == 4 ? 8 : 6) void k_count(GraphSet gs, const unsigned long long *__restrict__ queue,
                                                        uint32_t *__restrict__ ctl,
-                                                       unsigned long long *__restrict__ counts, uint32_t scale) {
+                                                       unsigned long long *__restrict__ counts, uint32_t scale,
+                                                       const uint32_t *__restrict__ skip) {
     constexpr uint32_t kTab = tab_slots<WAVES>();
     __shared__ __align__(16) uint32_t s_tab[kTab];
     __shared__ uint32_t s_ovf[kTab / 128];  // overflow bits, one per 4-slot bucket
@@ -841,6 +865,7 @@ __global__ __launch_bounds__(WAVES * 64, UNROLL == 4 ? 8 : 6) void k_count(Graph
 
     // item and graph fields are wave-uniform: they live in scalar registers
     const uint32_t tid = threadIdx.x, wv = uniform(tid >> 6), lane = tid & 63;
+    if (skip && sload(skip)) return;  // the launch is counted by k_count_hub
     if (lane < 16) s_flag[wv][lane] = 0;
     const uint32_t n_big = sload(ctl + C_NBIG), n_small = sload(ctl + C_NSMALL), n_tickets = sload(ctl + C_NTICK);
     const uint32_t n_bigt = (n_big + kBigGroup - 1) / kBigGroup;  // big tickets
@@ -945,18 +970,86 @@ __global__ __launch_bounds__(WAVES * 64, UNROLL == 4 ? 8 : 6) void k_count(Graph
         t = uniform(s_ticket[turn]);
         turn ^= 1u;
     }
-    // one atomic per graph per workgroup for what the waves still hold
-    if (lane == 0) { s_acc[wv] = acc; s_g[wv] = cur_g; }
-    __syncthreads();
-    if (tid == 0) {
-        for (int i = 0; i < WAVES; ++i) {
-            if (s_g[i] == kEmpty) continue;
-            unsigned long long sum = s_acc[i];
-            for (int j = i + 1; j < WAVES; ++j)
-                if (s_g[j] == s_g[i]) { sum += s_acc[j]; s_g[j] = kEmpty; }
-            if (sum) atomicAdd(counts + s_g[i], sum);
+    flush_counts<WAVES>(counts, s_acc, s_g, acc, cur_g, tid, wv, lane);
+}
+
+// ------------------------------------------------------------------ hub count kernel
+// The split count over hub codes (hubcode.h): every item is one wave's, one wave per
+// workgroup (9.1 KB of LDS: 16 waves per CU).
+//
+// What bounds it (RMAT s23, 8.8 ms; k_count took 16.9): the fabric behind the L2,
+// which delivers 7.2-7.8 TB/s here wherever the lines come from, so bytes and L2
+// hits are what counts.  k_count fetched 121 GB a launch.  16-bit codes and bitmaps
+// of the top hubs: 75 GB.  Parts of heavy rows per XCD and step (hubcode.h), so that
+// lists are met again while they are in L2: 62 GB; the same share of a row's own arcs
+// and in-list in each part, lists from 128-byte boundaries, words and ids read
+// non-temporally: 56 GB (10.3, 9.8, 8.8 ms).  48 steps' parts instead of 32, 8 parts
+// from 256 lists or 32 from 1024 on: no faster.  A round of 4 chunks of codes: 2 or 3
+// chunks 11.0 / 10.7 against 10.7 ms a call.
+// The headers of a ticket's items (queue entry, row offsets, record: three
+// dependent loads) are loaded by the lanes together, and what an item starts from
+// (its row's block, its first 64 lists) while the item before it is walked.
+template <int U>
+__global__ __launch_bounds__(64, 4) void k_count_hub(GraphDev G, HubSet hs, unsigned long long *__restrict__ counts) {
+    __shared__ __align__(16) HubLds s;
+    __shared__ __align__(16) uint32_t s_flag[16];
+    __shared__ uint8_t s_src[64];
+
+    if (!sload(hs.hctl + HC_ON)) return;  // counted by k_count
+    const uint32_t lane = threadIdx.x;
+    if (lane < 16) s_flag[lane] = 0;
+    const uint32_t tiny_end = sload(hs.hctl + HC_TINY0) + sload(hs.hctl + HC_TINY);
+    const uint64_t *units = hs.units;
+    unsigned long long acc = 0;
+
+    HubTickets tk(hs.hctl);
+    for (HubTicket t = tk.first(); uniform(t.n); t = tk.next(lane)) {
+        t = HubTicket{uniform(t.at), uniform(t.n), uniform(t.tiny) != 0};
+        if (t.tiny) {
+            const uint32_t e = t.at + lane;
+            const uint64_t q = e < tiny_end ? gload(hs.queue + e) : 0;
+            acc += tiny_walk(G, e < tiny_end, e < tiny_end && !(q >> 32), (uint32_t)q, s.bits, s.base, s.end, s_src,
+                             (uint8_t *)s_flag, lane);
+            continue;
+        }
+        // lane i: item i's header
+        uint32_t len = 0, own = 0, n_own = 0, in = 0, n_l = 0;
+        uint64_t rec = 0;
+        if (lane < t.n) {
+            const uint64_t q = gload(hs.queue + t.at + lane);
+            const uint32_t row = (uint32_t)q, chunk = (uint32_t)(q >> 32);
+            rec = gload(hs.rec + row);
+            const uint64_t r0 = gload(G.off + row), i0 = gload(G.in_off + row);
+            len = (uint32_t)(gload(G.off + row + 1) - r0);
+            const uint32_t k = row < G.n_owned ? len : 0u, kb = (uint32_t)(gload(G.in_off + row + 1) - i0);
+            const uint32_t chunks = hub_split(k + kb).chunks();
+            // the chunk's share of both, so that equal parts of rows cover much the same ids
+            const uint32_t a0 = (uint32_t)((uint64_t)k * chunk / chunks), b0 = (uint32_t)((uint64_t)kb * chunk / chunks);
+            own = (uint32_t)r0 + a0;
+            in = (uint32_t)i0 + b0;
+            n_own = (uint32_t)((uint64_t)k * (chunk + 1) / chunks) - a0;
+            n_l = n_own + (uint32_t)((uint64_t)kb * (chunk + 1) / chunks) - b0;
+        }
+        auto item = [&](uint32_t i) {
+            return HubItem{read_lane(len, i), read_lane(own, i), read_lane(n_own, i), read_lane(in, i), read_lane(n_l, i),
+                           split_rec(read_lane64(rec, i))};
+        };
+        HubItem it = item(0);
+        HubAhead ahead = hub_ahead(G, it, units, lane);
+        for (uint32_t i = 0; i < t.n; ++i) {
+            const HubItem cur = it;
+            HubAhead a = ahead;
+            const bool kept = list_kept(cur, lane, a.word);
+            const uint64_t lrec = gload(hs.rec + (kept ? a.id : 0u));
+            hub_insert(cur, a, units, s, lane);
+            if (i + 1 < t.n) {
+                it = item(i + 1);
+                ahead = hub_ahead(G, it, units, lane);
+            }
+            acc += hub_walk<U>(G, hs.rec, cur, a, lrec, kept, units, s, lane);
         }
     }
+    if (acc != 0 && lane == 0) atomicAdd(counts, acc);
 }
 
 // ------------------------------------------------------------------ host side
@@ -975,15 +1068,23 @@ static uint32_t resident_blocks(const void *kern, int threads) {
     return (uint32_t)blocks;
 }
 
+static constexpr int kHubU = 4;
+
 // queue entries: per row one kind A item and at most 1 + in-degree / kInChunk kind B items
 static uint64_t queue_cap(uint64_t total_rows, uint64_t total_m) { return 2 * total_rows + total_m / kInChunk + 1; }
 
-size_t count_ws_bytes(uint32_t G, uint64_t total_rows, uint64_t total_m) {
-    (void)G;
+size_t count_ws_base(uint64_t total_rows, uint64_t total_m) {
     Carver c(nullptr, 0);
     c.take<uint32_t>(C_WORDS);
     c.take<uint32_t>(kPlanEntries);
     c.take<unsigned long long>(queue_cap(total_rows, total_m));
+    return c.need();
+}
+
+size_t count_ws_bytes(uint64_t rows, uint64_t m) {
+    Carver c(nullptr, 0);
+    c.take<char>(count_ws_base(rows, m));
+    if (hub_fits(rows, m)) (void)hub_layout(c, rows, m);
     return c.need();
 }
 
@@ -1026,7 +1127,7 @@ lstc_status count_launch(const HostGraph *hosts, uint32_t G, const GraphDev *d_t
     bool narrow = true;
     for (uint32_t g = 0; g < G; ++g)
         narrow = narrow && hosts[g].m <= (1ull << 30) && hosts[g].scol_len <= (1ull << 30);
-    using Kern = void (*)(GraphSet, const unsigned long long *, uint32_t *, unsigned long long *, uint32_t);
+    using Kern = void (*)(GraphSet, const unsigned long long *, uint32_t *, unsigned long long *, uint32_t, const uint32_t *);
     // [unroll 4/8][narrow][waves 2/4/8]
     static const Kern kerns[2][2][3] = {
         {{k_count<4, false, 2>, k_count<4, false, 4>, k_count<4, false, 8>},
@@ -1041,22 +1142,43 @@ lstc_status count_launch(const HostGraph *hosts, uint32_t G, const GraphDev *d_t
     bool split = false;
     for (uint32_t g = 0; g < G; ++g) split = split || split_ok(hosts[g]);
     const uint32_t classes = split ? kHeads : 1u;
-    if (total <= kSmallPlan) {
+    // Codes: one graph with a streaming copy (and so in-lists and segment words),
+    // and a workspace that holds their arrays (count_ws_base is still enough for
+    // k_count).  Whether its hubs cover its columns well enough is decided on the
+    // device: both count kernels are launched and one of them leaves at once.
+    HubSet hs{};
+    uint32_t hub_grid = 0;
+    if (G == 1 && seg_ok(hosts[0]) && hosts[0].scol && hub_fits(total, total_m)) {
+        const HubSet h = hub_layout(c, total, total_m);
+        if (c.ok()) {
+            hs = h;
+            const uint32_t hfit = resident_blocks((const void *)k_count_hub<kHubU>, 64);
+            hub_grid = (uint32_t)cus * (hfit ? hfit : 1u);
+            LSTC_TRY(hub_build(gs.one, total_m, hs, st));
+        }
+    }
+    const uint32_t *hub_on = hub_grid ? hs.hctl + HC_ON : nullptr;
+    if (total <= kSmallPlan && !hub_grid) {
         hipLaunchKernelGGL(k_plan_small, dim3(1), dim3(1024), 0, st, gs, bd, ctl, queue, d_counts, tr.small_group, grid,
                            tr.waves, classes);
         LSTC_LAUNCHED("k_plan_small");
     } else {
-        hipLaunchKernelGGL(k_plan_rows<0>, dim3(kPlanBlocks), dim3(256), 0, st, gs, bd, wcnt, queue);
+        hipLaunchKernelGGL(k_plan_rows<0>, dim3(kPlanBlocks), dim3(256), 0, st, gs, bd, wcnt, queue, hs);
         LSTC_LAUNCHED("k_plan_rows<0>");
         hipLaunchKernelGGL(k_plan_scan, dim3(1), dim3(1024), 0, st, wcnt, ctl, d_counts, G, tr.small_group, grid,
-                           tr.waves, classes);
+                           tr.waves, classes, hs, hub_grid);
         LSTC_LAUNCHED("k_plan_scan");
-        hipLaunchKernelGGL(k_plan_rows<1>, dim3(kPlanBlocks), dim3(256), 0, st, gs, bd, wcnt, queue);
+        hipLaunchKernelGGL(k_plan_rows<1>, dim3(kPlanBlocks), dim3(256), 0, st, gs, bd, wcnt, queue, hs);
         LSTC_LAUNCHED("k_plan_rows<1>");
     }
     {
         const TimingMark tm = timed ? timing_begin(st) : TimingMark{nullptr, nullptr};
-        hipLaunchKernelGGL(kern, dim3(grid), dim3(tr.waves * 64), 0, st, gs, queue, ctl, d_counts, tr.table_scale);
+        if (hub_grid) {
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_count_hub<kHubU>), dim3(hub_grid), dim3(64), 0, st, gs.one, hs, d_counts);
+            LSTC_LAUNCHED("k_count_hub");
+        }
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(tr.waves * 64), 0, st, gs, queue, ctl, d_counts, tr.table_scale,
+                           hub_on);
         LSTC_LAUNCHED("k_count");
         timing_end(tm, st);
     }

@@ -57,7 +57,7 @@ extern "C" lstc_status lstc_count_split_static(const uint64_t *d_off, const uint
     if (!d_in_off || !d_in_col) return fail(LSTC_ERR_INVALID, "lstc_count_split_static: NULL in-lists");
     HostGraph h{d_off, d_col, nullptr, n_rows, n_owned, m, d_in_off, d_in_col, d_col_seg, d_in_seg};
     LSTC_TRY(validate_graph(h, "lstc_count_split_static"));
-    const size_t need = count_ws_bytes(1, n_rows, m);
+    const size_t need = count_ws_base(n_rows, m);
     if (need > kStaticScratch)
         return fail(LSTC_ERR_INVALID,
                     "lstc_count_split_static: this graph needs %zu bytes of scratch, the static scratch holds %zu "

@@ -1,0 +1,362 @@
+// hubcode.hip -- selects a graph's hub vertices and writes its rows as 16-bit
+// codes, hub bitmaps and tails (hubcode.h).  No counterpart in the reference,
+// whose count reads 32-bit columns (ShareKernelTCV62_update_v1.cu:43-191).
+//
+//   k_hub_init   : clears the selection words and the occurrences
+//   k_hub_sample : occurrences of each vertex in every stride-th 64-entry chunk of the columns
+//   k_hub_pick   : vertices and occurrences per occurrence bin (8 bins per octave); the bins
+//                  whose vertices become hubs, their first codes, and whether the hubs cover
+//                  enough of the sample for codes to pay
+//   k_hub_assign : every vertex's code
+//   k_hub_short  : the blocks of rows below kLongRow entries, 16 lanes per row
+//   k_hub_long   : the others, a wave per row
+#include "hubcode.h"
+#include "wave.h"
+
+namespace lstc {
+
+// Sampled entries (RMAT s23, ms a count: 11.1 with 2^20, 10.7 with 2^21, 10.8 with
+// 2^22), and at most one in 16: the hubs' counters are hot addresses.
+static constexpr uint64_t kSamples = 2u << 20, kMinStride = 16;
+// The hubs have to cover half of the sample.  Calls from codes against ids: RMAT s21
+// 2.21 / 3.24 ms, Chung-Lu of 1M vertices (gamma 2.1, mean degree 50) 1.87 / 2.10; a
+// uniform graph of 1M vertices and mean degree 40, whose hubs cover a twentieth,
+// 1.66 / 1.01.
+static constexpr uint32_t kCoverPct = 50;
+// Smaller graphs and shorter rows keep ids: the build is worth 0.1 ms (RMAT s17,
+// 1.9M arcs: 0.30 against 0.39 ms; a uniform graph of 3M vertices and 15 arcs a row,
+// found out by its sample, 2.36 against 2.24).
+static constexpr uint64_t kMinArcs = 1ull << 20, kMinPerRow = 16;
+static constexpr uint32_t kAbsent = 0xFFFFFFFFu;  // past the end of a row (ids are below 2^32 - 2)
+
+__device__ __forceinline__ uint32_t occ_bin(uint32_t c) {
+    if (c < 16) return c;
+    const uint32_t lg = 31 - __clz(c);
+    return 8 * (lg - 2) + ((c >> (lg - 3)) & 7u);
+}
+
+// The code of id x in a graph of n rows whose codes start at `code`; an id
+// without a row (halo ids outside the part) has none.
+__device__ __forceinline__ uint32_t code_of(const uint16_t *code, uint32_t n, uint32_t x) {
+    return x < n ? gload(code + x) : kNoCode;
+}
+
+// First unit of the block of row r, whose columns start at o.
+__device__ __forceinline__ uint32_t block_of(uint64_t r, uint64_t o) { return (uint32_t)((o >> 1) + 2 * r); }
+
+__global__ __launch_bounds__(256) void k_hub_init(HubSet hs, uint32_t n) {
+    if (blockIdx.x == 0)
+        for (uint32_t i = threadIdx.x; i < HC_WORDS; i += 256) hs.hctl[i] = 0;
+    for (uint64_t v = (uint64_t)blockIdx.x * 256 + threadIdx.x; v < n; v += (uint64_t)gridDim.x * 256) hs.cnt[v] = 0;
+}
+
+// A wave takes four chunks at a time.
+__global__ __launch_bounds__(256) void k_hub_sample(GraphDev G, uint64_t m, uint32_t stride, uint32_t *__restrict__ cnt) {
+    constexpr uint32_t kPer = 4;
+    const uint32_t lane = threadIdx.x & 63;
+    const uint64_t waves = (uint64_t)gridDim.x * 4, wave = (uint64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    for (uint64_t c0 = wave; c0 * 64 * stride < m; c0 += waves * kPer) {
+        uint32_t x[kPer];
+#pragma unroll
+        for (uint32_t q = 0; q < kPer; ++q) {
+            const uint64_t j = (c0 + q * waves) * 64 * stride + lane;
+            x[q] = kAbsent;
+            if (j < m) x[q] = gload(G.col + j);
+        }
+#pragma unroll
+        for (uint32_t q = 0; q < kPer; ++q)
+            if (x[q] < G.n_rows) atomicAdd(cnt + x[q], 1u);
+    }
+}
+
+// Every workgroup adds its share to the bins; the last one to do so picks.  Bins
+// above HC_CUT are hubs; of bin HC_CUT the first HC_REST vertices that ask.
+__global__ __launch_bounds__(256) void k_hub_pick(const uint32_t *__restrict__ cnt, uint32_t n,
+                                                  uint32_t *__restrict__ hctl) {
+    __shared__ uint32_t s_n[257], s_add[256];
+    __shared__ unsigned long long s_sum[257];
+    __shared__ uint32_t s_last;
+    const uint32_t b = threadIdx.x;
+    s_n[b] = 0;
+    s_add[b] = 0;
+    __syncthreads();
+    constexpr uint32_t kPer = 8;
+    const uint64_t step = (uint64_t)gridDim.x * 256;
+    for (uint64_t v = (uint64_t)blockIdx.x * 256 + b; v < n; v += step * kPer) {
+        uint32_t c[kPer];
+#pragma unroll
+        for (uint32_t q = 0; q < kPer; ++q) c[q] = v + q * step < n ? cnt[v + q * step] : 0u;
+#pragma unroll
+        for (uint32_t q = 0; q < kPer; ++q) {
+            if (c[q] == 0) continue;
+            atomicAdd(&s_n[occ_bin(c[q])], 1u);
+            atomicAdd(&s_add[occ_bin(c[q])], c[q]);
+        }
+    }
+    __syncthreads();
+    if (s_n[b]) {
+        atomicAdd(hctl + HC_HIST + b, s_n[b]);
+        atomicAdd(hctl + HC_SUM + b, s_add[b]);
+    }
+    __threadfence();
+    __syncthreads();
+    if (b == 0) s_last = atomicAdd(hctl + HC_DONE, 1u) == gridDim.x - 1 ? 1u : 0u;
+    __syncthreads();
+    if (!s_last) return;
+    auto read = [](uint32_t *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+    const uint32_t own_n = read(hctl + HC_HIST + b);
+    const unsigned long long own_sum = read(hctl + HC_SUM + b);
+    uint32_t sn = own_n;  // over bins b, b + 1, ...
+    unsigned long long ssum = own_sum;
+    if (b == 0) s_n[256] = 0, s_sum[256] = 0;
+    for (uint32_t d = 1; d < 256; d <<= 1) {
+        s_n[b] = sn;
+        s_sum[b] = ssum;
+        __syncthreads();
+        if (b + d < 256) sn += s_n[b + d], ssum += s_sum[b + d];
+        __syncthreads();
+    }
+    s_n[b] = sn;
+    s_sum[b] = ssum;
+    __syncthreads();
+    hctl[HC_BASE + b] = s_n[b + 1];
+    const unsigned long long all = s_sum[0];
+    unsigned long long covered = all;
+    if (s_n[0] > kHubs) {
+        if (!(sn > kHubs && s_n[b + 1] <= kHubs)) return;  // the cut bin's thread goes on
+        const uint32_t rest = kHubs - s_n[b + 1];
+        covered = s_sum[b + 1] + own_sum * rest / own_n;
+        hctl[HC_CUT] = b;
+        hctl[HC_REST] = rest;
+    } else if (b != 0) {
+        return;
+    }
+    hctl[HC_ON] = all && covered * 100 >= all * kCoverPct ? 1u : 0u;
+}
+
+// A workgroup takes 4096 vertices at a time and one place per bin among all of them.
+__global__ __launch_bounds__(256) void k_hub_assign(const uint32_t *__restrict__ cnt, uint32_t n,
+                                                    uint32_t *__restrict__ hctl, uint16_t *__restrict__ code) {
+    __shared__ uint32_t s_n[256], s_at[256];
+    if (!sload(hctl + HC_ON)) return;
+    const uint32_t cut = sload(hctl + HC_CUT), rest = sload(hctl + HC_REST), tid = threadIdx.x;
+    for (uint64_t v0 = (uint64_t)blockIdx.x * 4096; v0 < n; v0 += (uint64_t)gridDim.x * 4096) {
+        s_n[tid] = 0;
+        __syncthreads();
+        uint32_t c[16], at[16];
+#pragma unroll
+        for (uint32_t i = 0; i < 16; ++i) {
+            const uint64_t v = v0 + i * 256 + tid;
+            c[i] = v < n ? cnt[v] : 0u;
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < 16; ++i) {
+            const uint32_t b = occ_bin(c[i]);
+            at[i] = c[i] != 0 && b >= cut ? atomicAdd(&s_n[b], 1u) : 0u;
+        }
+        __syncthreads();
+        s_at[tid] = s_n[tid] ? atomicAdd(hctl + HC_USED + tid, s_n[tid]) : 0u;
+        __syncthreads();
+#pragma unroll
+        for (uint32_t i = 0; i < 16; ++i) {
+            const uint64_t v = v0 + i * 256 + tid;
+            const uint32_t b = occ_bin(c[i]), p = s_at[b] + at[i];
+            const bool hub = c[i] != 0 && (b > cut || (b == cut && p < rest));
+            if (v < n) code[v] = (uint16_t)(hub ? hctl[HC_BASE + b] + p : kNoCode);
+        }
+        __syncthreads();
+    }
+}
+
+// One wave per 64 rows: four short rows at a time, 16 lanes each, their entries in
+// registers (at most six per lane).  Long rows are listed for k_hub_long; a row
+// longer than a record can say takes the launch back to k_count.
+__global__ __launch_bounds__(256) void k_hub_short(GraphDev G, HubSet hs) {
+    constexpr uint32_t kPer = kLongRow / 16;
+    static_assert(kLongRow % 16 == 0, "a short row's entries per lane");
+    __shared__ uint32_t s_n, s_at;
+    if (!sload(hs.hctl + HC_ON)) return;
+    const uint32_t lane = threadIdx.x & 63, sub = lane & 15, grp = lane >> 4;
+    const uint64_t r0 = ((uint64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * 64, r = r0 + lane;
+    const bool valid = r < G.n_rows;
+    const uint64_t o = valid ? gload(G.off + r) : 0, e = valid ? gload(G.off + r + 1) : 0;
+    if (e - o >= kMaxHubRow) hs.hctl[HC_ON] = 0;
+    const uint32_t d = (uint32_t)min(e - o, (uint64_t)kMaxHubRow);
+    const uint32_t start = block_of(r, o);
+    if (threadIdx.x == 0) s_n = 0;
+    __syncthreads();
+    const bool lng = d >= kLongRow;
+    uint32_t place = 0;
+    if (lng) place = atomicAdd(&s_n, 1u);
+    __syncthreads();
+    if (threadIdx.x == 0 && s_n) s_at = atomicAdd(hs.hctl + HC_LONG_ROWS, s_n);
+    __syncthreads();
+    if (lng) hs.long_rows[s_at + place] = (uint32_t)r;
+    uint16_t *codes = (uint16_t *)hs.units;
+    uint32_t *tails = (uint32_t *)hs.units;
+    uint64_t mine = 0;  // this lane's row's record
+    const uint64_t some = ballot(!lng && d != 0);
+    for (uint32_t k = 0; k < 16; ++k) {
+        if ((some >> (4 * k) & 15u) == 0) continue;
+        const uint32_t src = 4 * k + grp;
+        const uint32_t rd = gather(lng ? 0u : d, src);
+        const uint32_t rs = gather(start, src);
+        const uint32_t *pc = G.col + gather64(o, src);
+        uint32_t x[kPer], c[kPer];
+#pragma unroll
+        for (uint32_t q = 0; q < kPer; ++q) {
+            const uint32_t i = 16 * q + sub;
+            x[q] = kAbsent;
+            if (i < rd) x[q] = gload(pc + i);
+        }
+#pragma unroll
+        for (uint32_t q = 0; q < kPer; ++q) {
+            c[q] = kNoCode;
+            if (x[q] != kAbsent) c[q] = code_of(hs.code, G.n_rows, x[q]);
+        }
+        const uint32_t sh = 16 * grp;
+        uint32_t nh = 0;
+#pragma unroll
+        for (uint32_t q = 0; q < kPer; ++q) nh += (uint32_t)__popc((uint32_t)(ballot(c[q] != kNoCode) >> sh) & 0xFFFFu);
+        const uint32_t units = (nh + 3) / 4, nt = rd - nh;
+        uint32_t ph = rs * 4, pt = (rs + units) * 2;
+        const uint32_t below = (1u << sub) - 1u;
+#pragma unroll
+        for (uint32_t q = 0; q < kPer; ++q) {
+            const bool h = c[q] != kNoCode, t = !h && x[q] != kAbsent;
+            const uint32_t hm = (uint32_t)(ballot(h) >> sh) & 0xFFFFu, tm = (uint32_t)(ballot(t) >> sh) & 0xFFFFu;
+            if (h) codes[ph + __popc(hm & below)] = (uint16_t)c[q];
+            if (t) tails[pt + __popc(tm & below)] = x[q];
+            ph += __popc(hm);
+            pt += __popc(tm);
+        }
+        if (sub < ((0u - nh) & 3u)) codes[ph + sub] = (uint16_t)kNoCode;
+        if (sub == 0 && (nt & 1u)) tails[pt] = kTailPad;
+        // lane src of the wave takes the record of its row (held by lanes of group src & 3)
+        const uint64_t rec = make_rec(rs, units, (nt + 1) / 2, 0);
+        const uint64_t got = gather64(rec, 16 * (lane & 3));
+        if (lane >> 2 == k) mine = got;
+    }
+    if (valid && !lng) hs.rec[r] = mine;
+}
+
+// A wave per long row, 512 entries in registers at a time (read twice if there
+// are more).  A wave takes kBatch rows together: their headers (four dependent
+// loads) come in by lane at once.
+__global__ __launch_bounds__(256) void k_hub_long(GraphDev G, HubSet hs) {
+    constexpr uint32_t kRegs = 8, kStep = 64 * kRegs, kBatch = 8;
+    __shared__ __align__(8) uint32_t s_word[4][kTopWords];
+    if (!sload(hs.hctl + HC_ON)) return;
+    const uint32_t lane = threadIdx.x & 63, wv = uniform(threadIdx.x >> 6);
+    uint32_t *word = s_word[wv];
+    const uint32_t n_long = sload(hs.hctl + HC_LONG_ROWS);
+    uint16_t *codes = (uint16_t *)hs.units;
+    uint32_t *tails = (uint32_t *)hs.units;
+    for (uint32_t i0 = (blockIdx.x * 4 + wv) * kBatch; i0 < n_long; i0 += gridDim.x * 4 * kBatch) {
+      const uint32_t nb = min(kBatch, n_long - i0);
+      uint32_t l_row = 0, l_d = 0, l_start = 0;
+      uint64_t l_off = 0;
+      if (lane < nb) {
+          l_row = gload(hs.long_rows + i0 + lane);
+          l_off = gload(G.off + l_row);
+          l_d = (uint32_t)(gload(G.off + l_row + 1) - l_off);
+          l_start = block_of(l_row, l_off);
+      }
+      for (uint32_t ib = 0; ib < nb; ++ib) {
+        const uint32_t r = read_lane(l_row, ib), d = read_lane(l_d, ib), start = read_lane(l_start, ib);
+        const uint32_t *colr = G.col + read_lane64(l_off, ib);
+        uint32_t x[kRegs], c[kRegs];
+        auto fetch = [&](uint32_t p0) {
+#pragma unroll
+            for (uint32_t q = 0; q < kRegs; ++q) {
+                const uint32_t p = p0 + 64 * q + lane;
+                x[q] = kAbsent;
+                if (p < d) x[q] = gload(colr + p);
+            }
+#pragma unroll
+            for (uint32_t q = 0; q < kRegs; ++q) {
+                c[q] = kNoCode;
+                if (x[q] != kAbsent) c[q] = code_of(hs.code, G.n_rows, x[q]);
+            }
+        };
+        uint32_t top = 0, hub = 0;
+        for (uint32_t p0 = 0; p0 < d; p0 += kStep) {
+            fetch(p0);
+#pragma unroll
+            for (uint32_t q = 0; q < kRegs; ++q) {
+                top += (uint32_t)__popcll(ballot(c[q] < kTop));
+                hub += (uint32_t)__popcll(ballot(c[q] != kNoCode));
+            }
+        }
+        const bool bm = top >= kTopMin;
+        const uint32_t floor = bm ? kTop : 0u;  // codes below go to the bitmap
+        const uint32_t nh = bm ? hub - top : hub, units = (nh + 3) / 4, nt = d - hub;
+        // from a 128-byte boundary: with a bitmap there is always room for that, else if there is
+        const uint32_t aligned = (start + 15u) & ~15u;
+        const bool fits = aligned - start + units + (nt + 1) / 2 <= (d + 1) / 2 + 1;
+        const uint32_t first = bm ? aligned + kTopUnits : fits ? aligned : start;
+        word[lane] = word[64 + lane] = 0;
+        uint32_t ph = first * 4, pt = (first + units) * 2;
+        for (uint32_t p0 = 0; p0 < d; p0 += kStep) {
+            if (d > kStep) fetch(p0);
+#pragma unroll
+            for (uint32_t q = 0; q < kRegs; ++q) {
+                const bool in = x[q] != kAbsent, h = c[q] != kNoCode && c[q] >= floor, t = in && c[q] == kNoCode;
+                const uint64_t hm = ballot(h), tm = ballot(t);
+                if (h) codes[ph + mask_rank(hm)] = (uint16_t)c[q];
+                else if (t) tails[pt + mask_rank(tm)] = x[q];
+                else if (in) atomicOr(&word[c[q] >> 5], 1u << (c[q] & 31u));
+                ph += (uint32_t)__popcll(hm);
+                pt += (uint32_t)__popcll(tm);
+            }
+        }
+        if (lane < ((0u - nh) & 3u)) codes[ph + lane] = (uint16_t)kNoCode;
+        if (lane == 0 && (nt & 1u)) tails[pt] = kTailPad;
+        if (bm) hs.units[first - kTopUnits + lane] = *(const uint64_t *)(word + 2 * lane);
+        if (lane == 0) hs.rec[r] = make_rec(first, units, (nt + 1) / 2, bm ? 1u : 0u);
+      }
+    }
+}
+
+static uint64_t hub_units(uint64_t rows, uint64_t m) { return m / 2 + 2 * rows + 64; }
+
+bool hub_fits(uint64_t rows, uint64_t m) {
+    return m >= kMinArcs && m >= kMinPerRow * rows && rows < (1ull << 32) && hub_units(rows, m) < (1ull << 29);
+}
+
+HubSet hub_layout(Carver &c, uint64_t rows, uint64_t m) {
+    HubSet h{};
+    h.hctl = c.take<uint32_t>(HC_WORDS);
+    h.cnt = c.take<uint32_t>(rows + 1);
+    h.code = c.take<uint16_t>(rows + 1);
+    h.rec = c.take<uint64_t>(rows + 1);
+    h.long_rows = c.take<uint32_t>(m / kLongRow + 1);
+    h.units = c.take<uint64_t>(hub_units(rows, m));
+    h.plan_cnt = c.take<uint32_t>((size_t)kHubSlots * kHubPlanWaves);
+    // a row of n >= kHeavy lists has at most n / 64 items, any other one; all rows have at most 2 m lists
+    h.queue = c.take<uint64_t>(rows + m / 32 + 1);
+    return h;
+}
+
+lstc_status hub_build(const GraphDev &g, uint64_t m, const HubSet &hs, hipStream_t st) {
+    const uint32_t n = g.n_rows, cus = (uint32_t)device_cus();
+    const uint32_t stride = (uint32_t)hmax<uint64_t>(kMinStride, m / kSamples);
+    const uint32_t blocks = ceil_div_u32(n, 256);  // a wave per 64 rows
+    const uint32_t flat = hmin(blocks, cus * 4);
+    hipLaunchKernelGGL(k_hub_init, dim3(flat), dim3(256), 0, st, hs, n);
+    LSTC_LAUNCHED("k_hub_init");
+    hipLaunchKernelGGL(k_hub_sample, dim3(cus * 8), dim3(256), 0, st, g, m, stride, hs.cnt);
+    LSTC_LAUNCHED("k_hub_sample");
+    hipLaunchKernelGGL(k_hub_pick, dim3(hmin(blocks, cus)), dim3(256), 0, st, (const uint32_t *)hs.cnt, n, hs.hctl);
+    LSTC_LAUNCHED("k_hub_pick");
+    hipLaunchKernelGGL(k_hub_assign, dim3(hmin(ceil_div_u32(n, 4096), cus * 8)), dim3(256), 0, st,
+                       (const uint32_t *)hs.cnt, n, hs.hctl, hs.code);
+    LSTC_LAUNCHED("k_hub_assign");
+    hipLaunchKernelGGL(k_hub_short, dim3(blocks), dim3(256), 0, st, g, hs);
+    LSTC_LAUNCHED("k_hub_short");
+    hipLaunchKernelGGL(k_hub_long, dim3(cus * 8), dim3(256), 0, st, g, hs);
+    LSTC_LAUNCHED("k_hub_long");
+    return LSTC_OK;
+}
+
+}  // namespace lstc

@@ -38,20 +38,19 @@ __device__ __forceinline__ bool one_segment(uint32_t B, uint32_t myend) {
     return ballot(myend > B && myend < B + 64u * UNROLL) == 0;
 }
 
-// Column positions are element indices, or with NARROW (every index below
-// 2^30) byte offsets, which the loads take as they are.
+// Positions are element indices (SHIFT 0), or byte offsets that the loads take
+// as they are: SHIFT 2 for 32-bit columns (every index below 2^30), 3 for 8-byte
+// units of codes (every index below 2^29).
 template <bool NARROW>
-__device__ __forceinline__ uint32_t col_pos(uint32_t i) {
-    return NARROW ? i << 2 : i;
-}
+constexpr int col_shift() { return NARROW ? 2 : 0; }
 
 // A full round that lies wholly in one segment: its column index at position
 // B + 64k is c0 + 64k (uniform, below m), so only the lane offset is per lane.
-template <int UNROLL, bool NARROW>
+template <int UNROLL, int SHIFT>
 __device__ __forceinline__ void index_single(uint32_t c0, uint32_t lane, uint32_t (&idx)[UNROLL]) {
-    const uint32_t i0 = col_pos<NARROW>(c0 + lane);
+    const uint32_t i0 = (c0 + lane) << SHIFT;
 #pragma unroll
-    for (int k = 0; k < UNROLL; ++k) idx[k] = i0 + col_pos<NARROW>(64u * k);
+    for (int k = 0; k < UNROLL; ++k) idx[k] = i0 + ((64u * k) << SHIFT);
 }
 
 // A round in which segments end: they are the consecutive segments sg, sg + 1,
@@ -63,7 +62,7 @@ __device__ __forceinline__ void index_single(uint32_t c0, uint32_t lane, uint32_
 // window's segment count.  FULL: the round lies wholly before `total` (every
 // round of a window but the last), so no position needs the past-the-end
 // handling (index 0 otherwise).
-template <int UNROLL, bool FULL, bool NARROW>
+template <int UNROLL, bool FULL, int SHIFT>
 __device__ __forceinline__ void index_walk(uint32_t B, uint32_t total, uint32_t mybase, uint32_t myend, uint32_t sg,
                                            uint32_t lane, uint32_t (&idx)[UNROLL]) {
     uint32_t j = sg;
@@ -82,7 +81,7 @@ __device__ __forceinline__ void index_walk(uint32_t B, uint32_t total, uint32_t 
             ej = (uint32_t)__builtin_amdgcn_readlane((int)myend, (int)j);
             vb = t >= e ? bj : vb;
         }
-        idx[k] = FULL || t < total ? col_pos<NARROW>(vb + t) : 0u;
+        idx[k] = FULL || t < total ? (vb + t) << SHIFT : 0u;
     }
 }
 

@@ -567,7 +567,7 @@ static lstc_status launch_batch(lstc_server *S) {
         Req *r = S->ready.front();
         const uint32_t G1 = (uint32_t)batch.size() + 1;
         if (!batch.empty() &&
-            batch_head_bytes(G1) + count_ws_bytes(G1, rows + r->n_rows, arcs + r->m_cap) > S->reserve_bytes)
+            batch_head_bytes(G1) + count_ws_base(rows + r->n_rows, arcs + r->m_cap) > S->reserve_bytes)
             break;
         batch.push_back(r);
         rows += r->n_rows;
@@ -756,7 +756,7 @@ extern "C" lstc_status lstc_server_submit(lstc_server *S, const lstc_request *re
     if (r.kind == LSTC_REQ_CSR) {
         HostGraph h{r.off, r.col, nullptr, r.n_rows, r.n_rows, r.m};
         LSTC_TRY(validate_graph(h, "lstc_server_submit"));
-        if (batch_head_bytes(1) + count_ws_bytes(1, r.n_rows, r.m) > S->reserve_bytes)
+        if (batch_head_bytes(1) + count_ws_base(r.n_rows, r.m) > S->reserve_bytes)
             return fail(LSTC_ERR_OVER_BUDGET, "lstc_server_submit: CSR rows exceed the batch reserve");
     } else {
         if (r.m_raw >= 0x7FFFF000ull) return fail(LSTC_ERR_INVALID, "lstc_server_submit: too many edges");
@@ -764,7 +764,7 @@ extern "C" lstc_status lstc_server_submit(lstc_server *S, const lstc_request *re
         const uint32_t n = request_rows(r);
         size_t ws = 0;
         const size_t need = prep_bytes(n, r.m_raw, &ws) + resident_bytes(n, r.m_raw);
-        const size_t qneed = batch_head_bytes(1) + count_ws_bytes(1, n, r.m_raw);
+        const size_t qneed = batch_head_bytes(1) + count_ws_base(n, r.m_raw);
         if (need > S->pool.total() || qneed > S->reserve_bytes) {
             std::lock_guard<std::mutex> lk(S->mu);
             S->n_rejected++;

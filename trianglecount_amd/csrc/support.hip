@@ -211,11 +211,11 @@ __device__ __forceinline__ uint64_t sup_index(uint32_t B, uint32_t total, uint32
     constexpr uint32_t RB = 64u * U;
     const uint32_t sg = first_segment(B, myend);
     if (B + RB > total)
-        index_walk<U, false, NARROW>(B, total, mybase, myend, sg, lane, idx);
+        index_walk<U, false, col_shift<NARROW>()>(B, total, mybase, myend, sg, lane, idx);
     else if (one_segment<U>(B, myend))
-        index_single<U, NARROW>(read_lane(mybase, sg) + B, lane, idx);
+        index_single<U, col_shift<NARROW>()>(read_lane(mybase, sg) + B, lane, idx);
     else
-        index_walk<U, true, NARROW>(B, total, mybase, myend, sg, lane, idx);
+        index_walk<U, true, col_shift<NARROW>()>(B, total, mybase, myend, sg, lane, idx);
     return ballot(myend > B && myend <= B + RB);
 }
 
