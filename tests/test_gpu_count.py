@@ -278,3 +278,18 @@ def test_count_halo_part_from_hub_codes(lstc, oracle):
         assert c == lstc.count(h, split=False)
         total += c
     assert total == lstc.count(g)
+
+
+@pytest.mark.parametrize("owned", [None, 100_003, 1])
+def test_count_plain_from_hub_codes(lstc, owned):
+    """A bare CSR of RMAT s19 (7.7M arcs), whole and with the first rows owned, against the per-row partials
+    (counted from ids)."""
+    g = lstc.clean_orient(*lstc.generate_rmat(19, 16, seed=1))
+    want, per_row = lstc.count(g, per_row=True, split=False)
+    no = g.n if owned is None else owned
+    assert lstc.count(g, n_owned=no) == int(per_row[:no].sum())
+    if owned is None:
+        import json
+        with open(G.GOLDEN + "/rmat_counts.json") as f:
+            assert want == json.load(f)["19"]["triangles"]
+        assert lstc.count(lstc.in_lists(g)) == want  # split, lists read from the columns

@@ -989,7 +989,7 @@ __global__ __launch_bounds__(WAVES * 64, UNROLL == 4 ? 8 : 6) void k_count(Graph
 // The headers of a ticket's items (queue entry, row offsets, record: three
 // dependent loads) are loaded by the lanes together, and what an item starts from
 // (its row's block, its first 64 lists) while the item before it is walked.
-template <int U>
+template <int U, bool SPLIT>
 __global__ __launch_bounds__(64, 4) void k_count_hub(GraphDev G, HubSet hs, unsigned long long *__restrict__ counts) {
     __shared__ __align__(16) HubLds s;
     __shared__ __align__(16) uint32_t s_flag[16];
@@ -1005,7 +1005,7 @@ __global__ __launch_bounds__(64, 4) void k_count_hub(GraphDev G, HubSet hs, unsi
     HubTickets tk(hs.hctl);
     for (HubTicket t = tk.first(); uniform(t.n); t = tk.next(lane)) {
         t = HubTicket{uniform(t.at), uniform(t.n), uniform(t.tiny) != 0};
-        if (t.tiny) {
+        if (SPLIT && t.tiny) {
             const uint32_t e = t.at + lane;
             const uint64_t q = e < tiny_end ? gload(hs.queue + e) : 0;
             acc += tiny_walk(G, e < tiny_end, e < tiny_end && !(q >> 32), (uint32_t)q, s.bits, s.base, s.end, s_src,
@@ -1019,9 +1019,10 @@ __global__ __launch_bounds__(64, 4) void k_count_hub(GraphDev G, HubSet hs, unsi
             const uint64_t q = gload(hs.queue + t.at + lane);
             const uint32_t row = (uint32_t)q, chunk = (uint32_t)(q >> 32);
             rec = gload(hs.rec + row);
-            const uint64_t r0 = gload(G.off + row), i0 = gload(G.in_off + row);
+            const uint64_t r0 = gload(G.off + row), i0 = SPLIT ? gload(G.in_off + row) : 0;
             len = (uint32_t)(gload(G.off + row + 1) - r0);
-            const uint32_t k = row < G.n_owned ? len : 0u, kb = (uint32_t)(gload(G.in_off + row + 1) - i0);
+            const uint32_t k = row < G.n_owned ? len : 0u;
+            const uint32_t kb = SPLIT ? (uint32_t)(gload(G.in_off + row + 1) - i0) : 0u;
             const uint32_t chunks = hub_split(k + kb).chunks();
             // the chunk's share of both, so that equal parts of rows cover much the same ids
             const uint32_t a0 = (uint32_t)((uint64_t)k * chunk / chunks), b0 = (uint32_t)((uint64_t)kb * chunk / chunks);
@@ -1035,18 +1036,18 @@ __global__ __launch_bounds__(64, 4) void k_count_hub(GraphDev G, HubSet hs, unsi
                            split_rec(read_lane64(rec, i))};
         };
         HubItem it = item(0);
-        HubAhead ahead = hub_ahead(G, it, units, lane);
+        HubAhead ahead = hub_ahead<SPLIT>(G, it, units, lane);
         for (uint32_t i = 0; i < t.n; ++i) {
             const HubItem cur = it;
             HubAhead a = ahead;
-            const bool kept = list_kept(cur, lane, a.word);
+            const bool kept = list_kept<SPLIT>(G, cur, lane, a.word, a.id);
             const uint64_t lrec = gload(hs.rec + (kept ? a.id : 0u));
             hub_insert(cur, a, units, s, lane);
             if (i + 1 < t.n) {
                 it = item(i + 1);
-                ahead = hub_ahead(G, it, units, lane);
+                ahead = hub_ahead<SPLIT>(G, it, units, lane);
             }
-            acc += hub_walk<U>(G, hs.rec, cur, a, lrec, kept, units, s, lane);
+            acc += hub_walk<U, SPLIT>(G, hs.rec, cur, a, lrec, kept, units, s, lane);
         }
     }
     if (acc != 0 && lane == 0) atomicAdd(counts, acc);
@@ -1142,17 +1143,19 @@ lstc_status count_launch(const HostGraph *hosts, uint32_t G, const GraphDev *d_t
     bool split = false;
     for (uint32_t g = 0; g < G; ++g) split = split || split_ok(hosts[g]);
     const uint32_t classes = split ? kHeads : 1u;
-    // Codes: one graph with a streaming copy (and so in-lists and segment words),
-    // and a workspace that holds their arrays (count_ws_base is still enough for
-    // k_count).  Whether its hubs cover its columns well enough is decided on the
-    // device: both count kernels are launched and one of them leaves at once.
+    // Codes: one graph with in-lists and segment words, or counted without in-lists
+    // and without per-row output, and a workspace that holds their arrays (count_ws_base is
+    // still enough for k_count).  Whether its hubs cover its columns well enough is
+    // decided on the device: both count kernels are launched and one leaves at once.
     HubSet hs{};
     uint32_t hub_grid = 0;
-    if (G == 1 && seg_ok(hosts[0]) && hosts[0].scol && hub_fits(total, total_m)) {
-        const HubSet h = hub_layout(c, total, total_m);
+    using HubKern = void (*)(GraphDev, HubSet, unsigned long long *);
+    const HubKern hub_kern = split ? (HubKern)k_count_hub<kHubU, true> : (HubKern)k_count_hub<kHubU, false>;
+    if (G == 1 && (split ? seg_ok(hosts[0]) : !hosts[0].per_row) && hub_fits(hosts[0].n_rows, total_m, split)) {
+        const HubSet h = hub_layout(c, hosts[0].n_rows, total_m);
         if (c.ok()) {
             hs = h;
-            const uint32_t hfit = resident_blocks((const void *)k_count_hub<kHubU>, 64);
+            const uint32_t hfit = resident_blocks((const void *)hub_kern, 64);
             hub_grid = (uint32_t)cus * (hfit ? hfit : 1u);
             LSTC_TRY(hub_build(gs.one, total_m, hs, st));
         }
@@ -1174,7 +1177,7 @@ lstc_status count_launch(const HostGraph *hosts, uint32_t G, const GraphDev *d_t
     {
         const TimingMark tm = timed ? timing_begin(st) : TimingMark{nullptr, nullptr};
         if (hub_grid) {
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_count_hub<kHubU>), dim3(hub_grid), dim3(64), 0, st, gs.one, hs, d_counts);
+            hipLaunchKernelGGL(hub_kern, dim3(hub_grid), dim3(64), 0, st, gs.one, hs, d_counts);
             LSTC_LAUNCHED("k_count_hub");
         }
         hipLaunchKernelGGL(kern, dim3(grid), dim3(tr.waves * 64), 0, st, gs, queue, ctl, d_counts, tr.table_scale,

@@ -25,8 +25,10 @@ static constexpr uint64_t kSamples = 2u << 20, kMinStride = 16;
 static constexpr uint32_t kCoverPct = 50;
 // Smaller graphs and shorter rows keep ids: the build is worth 0.1 ms (RMAT s17,
 // 1.9M arcs: 0.30 against 0.39 ms; a uniform graph of 3M vertices and 15 arcs a row,
-// found out by its sample, 2.36 against 2.24).
-static constexpr uint64_t kMinArcs = 1ull << 20, kMinPerRow = 16;
+// found out by its sample, 2.36 against 2.24).  Without in-lists k_count has less to
+// lose to (Chung-Lu of 4.4M arcs 0.464 from codes, 0.441 from ids; of 6.8M arcs 0.620 /
+// 0.616; RMAT s19, 7.7M arcs, 0.65 / 0.92; s21 2.57 / 5.42).
+static constexpr uint64_t kMinArcs = 1ull << 20, kMinArcsPlain = 6ull << 20, kMinPerRow = 16;
 static constexpr uint32_t kAbsent = 0xFFFFFFFFu;  // past the end of a row (ids are below 2^32 - 2)
 
 __device__ __forceinline__ uint32_t occ_bin(uint32_t c) {
@@ -320,8 +322,8 @@ __global__ __launch_bounds__(256) void k_hub_long(GraphDev G, HubSet hs) {
 
 static uint64_t hub_units(uint64_t rows, uint64_t m) { return m / 2 + 2 * rows + 64; }
 
-bool hub_fits(uint64_t rows, uint64_t m) {
-    return m >= kMinArcs && m >= kMinPerRow * rows && rows < (1ull << 32) && hub_units(rows, m) < (1ull << 29);
+bool hub_fits(uint64_t rows, uint64_t m, bool split) {
+    return m >= (split ? kMinArcs : kMinArcsPlain) && m >= kMinPerRow * rows && rows < (1ull << 32) && hub_units(rows, m) < (1ull << 29);
 }
 
 HubSet hub_layout(Carver &c, uint64_t rows, uint64_t m) {

@@ -25,9 +25,9 @@ __device__ __forceinline__ void hub_plan_rows(const GraphDev &G, const HubSet &h
         bool tiny = false;
         if (r < end) {
             const uint32_t k = (uint32_t)(gload(G.off + r + 1) - gload(G.off + r));
-            const uint32_t kb = (uint32_t)(gload(G.in_off + r + 1) - gload(G.in_off + r));
+            const uint32_t kb = G.in_off ? (uint32_t)(gload(G.in_off + r + 1) - gload(G.in_off + r)) : 0u;
             in_only = r >= G.n_owned;
-            tiny = k >= 2 && k <= tiny_max;
+            tiny = G.in_off && k >= 2 && k <= tiny_max;
             n = k < 2 ? 0u : (in_only ? 0u : k) + kb;
         }
         for (uint64_t heavy = ballot(n >= kHeavy); heavy; heavy &= heavy - 1) {

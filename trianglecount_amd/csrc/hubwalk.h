@@ -47,13 +47,20 @@ struct HubAhead {
 };
 static constexpr uint32_t kEmptyId = 0xFFFFFFFFu;
 
+// SPLIT: the graph has in-lists and segment words (`word` is list j's); without
+// them every own arc is counted here, and only rows have lists.
+template <bool SPLIT>
 __device__ __forceinline__ void list_load(const GraphDev &G, const HubItem &it, uint32_t j, uint64_t &word, uint32_t &id) {
+    word = 0;
+    id = 0xFFFFFFFFu;
+    if (!SPLIT) {
+        if (j < it.n) id = __builtin_nontemporal_load((const LSTC_GLOBAL_AS uint32_t *)(G.col + it.own + j));
+        return;
+    }
     const bool own = j < it.n_own, in = j < it.n;
     const uint32_t at = own ? it.own + j : it.in + (j - it.n_own);
     const uint64_t *w = own ? G.col_seg : G.in_seg;
     const uint32_t *c = own ? G.col : G.in_col;
-    word = 0;
-    id = 0;
     if (in) {
         // read once per count: kept out of the way of the lists in L2
         word = __builtin_nontemporal_load((const LSTC_GLOBAL_AS uint64_t *)(w + at));
@@ -62,14 +69,17 @@ __device__ __forceinline__ void list_load(const GraphDev &G, const HubItem &it, 
 }
 // Whether list j of the item is streamed: it has entries, and one of the row's own
 // arcs is counted here only if its list is shorter than the row.
-__device__ __forceinline__ bool list_kept(const HubItem &it, uint32_t j, uint64_t word) {
+template <bool SPLIT>
+__device__ __forceinline__ bool list_kept(const GraphDev &G, const HubItem &it, uint32_t j, uint64_t word, uint32_t id) {
+    if (!SPLIT) return id < G.n_rows;
     const uint32_t d = (uint32_t)(word >> 32);
     return d != 0 && (j >= it.n_own || d < it.len);
 }
 
+template <bool SPLIT>
 __device__ __forceinline__ HubAhead hub_ahead(const GraphDev &G, const HubItem &it, const uint64_t *__restrict__ units, uint32_t lane) {
     HubAhead a;
-    list_load(G, it, lane, a.word, a.id);
+    list_load<SPLIT>(G, it, lane, a.word, a.id);
     a.codes = ~0ull;
     a.top = 0;
     a.tail = kEmptyId;
@@ -253,7 +263,7 @@ __device__ __forceinline__ uint32_t lay_out(uint32_t start, uint32_t len, HubLds
 }
 
 // The matches of the item's lists, summed over the wave.
-template <int U>
+template <int U, bool SPLIT>
 __device__ __forceinline__ uint32_t hub_walk(const GraphDev &G, const uint64_t *__restrict__ recs, const HubItem &it,
                                              const HubAhead &a, uint64_t rec, bool kept,
                                              const uint64_t *__restrict__ units, HubLds &s, uint32_t lane) {
@@ -264,7 +274,7 @@ __device__ __forceinline__ uint32_t hub_walk(const GraphDev &G, const uint64_t *
         const RowRec R = split_rec(kept ? rec : 0);
         uint64_t word;
         uint32_t id;
-        list_load(G, it, j0 + 64 + lane, word, id);  // the next window's
+        list_load<SPLIT>(G, it, j0 + 64 + lane, word, id);  // the next window's
         // the first round of tails and of codes
         uint32_t tbase = 0, tend = 0, ttotal = 0, ti[1] = {0};
         uint64_t tx[1] = {0};
@@ -297,7 +307,7 @@ __device__ __forceinline__ uint32_t hub_walk(const GraphDev &G, const uint64_t *
             for (int k = 0; k < 8; ++k)
                 hits += (uint32_t)__popc((uint32_t)v[k] & top0) + (uint32_t)__popc((uint32_t)(v[k] >> 32) & top1);
         }
-        kept = list_kept(it, j0 + 64 + lane, word);
+        kept = list_kept<SPLIT>(G, it, j0 + 64 + lane, word, id);
         rec = gload(recs + (kept ? id : 0u));
         uint32_t B = 0;
         if (total) {
