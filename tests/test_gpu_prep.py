@@ -220,3 +220,23 @@ def test_stream_copy_bit_exact(lstc, oracle, name, builder):
     assert lstc.count_batch([g]) == [want]
     lstc.in_lists(g)  # words into col again: the copy is dropped
     assert g.scol is None and lstc.count(g) == want
+
+
+@pytest.mark.parametrize("n,m", [(16384, 40_000), (16385, 40_000), (3, 5), (5003, 1 << 21), (5003, (1 << 21) - 1),
+                                 (17_000_003, 3000)])
+def test_clean_orient_path_edges(lstc, oracle, n, m):
+    """Both sides of the one-workgroup vertex steps (16384 vertices, 2^22 keys), of the sort's block size
+    (2^22 keys) and of the scan's levels (4096 tiles of 4096): symmetric, and split with the streaming copy."""
+    rng = np.random.default_rng(n + m)
+    s, d = rng.integers(0, n, m).astype(np.uint32), rng.integers(0, n, m).astype(np.uint32)
+    _check_clean_orient(lstc, oracle, n, s, d, compact=m % 2 == 0)
+    up = lambda a: torch.from_numpy(a.view(np.int32)).cuda()  # noqa: E731
+    g = lstc.clean_orient(n, up(s), up(d), in_lists=True, stream_copy=n < 1_000_000)
+    og = oracle.clean_orient(n, s, d, True)[1]
+    off, col = g.to_numpy()
+    assert np.array_equal(off, og.off) and np.array_equal(col, og.col)
+    bare = lstc.in_lists(lstc.Graph.from_numpy(og.off, og.col))  # in-lists built by the other path
+    k = g.meta["in_entries"]
+    assert k == bare.meta["in_entries"] and torch.equal(g.in_off[: g.n + 1], bare.in_off[: g.n + 1])
+    assert torch.equal(g.in_col[:k], bare.in_col[:k])
+    assert lstc.count(g) == oracle.count(og)

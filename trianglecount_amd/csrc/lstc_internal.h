@@ -98,13 +98,15 @@ size_t radix_sort_ws_bytes(uint64_t n);
 lstc_status radix_sort_u64(uint64_t *keys, uint64_t *alt, uint64_t n, int key_bits,
                            uint64_t **result, void *ws, size_t ws_bytes, hipStream_t s,
                            bool first_counts_ready = false);
-// The sort's passes work on blocks of kRadixBlock consecutive keys.  A kernel
-// that writes the keys block by block can count the first digit (the low 8
+// The sort's passes work on blocks of radix_sub(n) * kRadixTile consecutive keys.
+// A kernel that writes the keys block by block can count the first digit (the low 8
 // bits) itself: the count of digit d in block t goes to
 // radix_first_counts(ws, n)[d * radix_blocks(n) + t], and the sort is then
 // called with first_counts_ready, which skips its first counting pass.
-constexpr uint64_t kRadixBlock = 16384;
-inline uint64_t radix_blocks(uint64_t n) { return (n + kRadixBlock - 1) / kRadixBlock; }
+constexpr uint64_t kRadixTile = 4096;
+constexpr uint64_t kRadixFew = 1ull << 22;  // below: one sub-tile per block (1024 blocks at most)
+inline uint32_t radix_sub(uint64_t n) { return n < kRadixFew ? 1u : 4u; }
+inline uint64_t radix_blocks(uint64_t n) { return (n + radix_sub(n) * kRadixTile - 1) / (radix_sub(n) * kRadixTile); }
 uint32_t *radix_first_counts(void *ws, uint64_t n);
 
 // (a) clean + orient without synchronising (prep.hip); sizes stay on the device:

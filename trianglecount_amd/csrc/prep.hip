@@ -26,6 +26,7 @@
 #include "lookback.h"
 #include "lstc_internal.h"
 #include "wave.h"
+#include "wgscan.h"
 
 namespace lstc {
 
@@ -45,19 +46,18 @@ static int bits_for(uint64_t n) {  // bits to represent values < n
 // workgroup: the workgroup also counts its block's first digit (the low 8
 // bits) into counts[d * blocks + blockIdx.x], the sort's first histogram.
 // The raw pairs are read once (non-temporal hint).
-static constexpr uint32_t kKeyPairs = (uint32_t)(kRadixBlock / 2);  // raw pairs per workgroup
 static constexpr uint32_t kKeyBatch = 8;                             // rounds whose loads go out together
 
 __global__ __launch_bounds__(256) void k_make_keys(const uint32_t *__restrict__ src, const uint32_t *__restrict__ dst,
                                                    uint64_t m_raw, uint32_t n, uint32_t b, uint64_t *__restrict__ keys,
-                                                   uint32_t blocks, uint32_t *__restrict__ counts,
+                                                   uint32_t pairs, uint32_t blocks, uint32_t *__restrict__ counts,
                                                    uint32_t *__restrict__ bad) {
     __shared__ uint32_t cnt[256];
     cnt[threadIdx.x] = 0;
     __syncthreads();
-    const uint64_t p0 = (uint64_t)blockIdx.x * kKeyPairs;
+    const uint64_t p0 = (uint64_t)blockIdx.x * pairs;  // pairs: raw pairs per workgroup
     bool out_of_range = false;
-    for (uint32_t r0 = 0; r0 < kKeyPairs / 256; r0 += kKeyBatch) {
+    for (uint32_t r0 = 0; r0 < pairs / 256; r0 += kKeyBatch) {
         uint32_t s[kKeyBatch], d[kKeyBatch];
 #pragma unroll
         for (uint32_t r = 0; r < kKeyBatch; ++r) {
@@ -420,15 +420,15 @@ static lstc_status compact_pass(const Op &op, uint64_t n_max, uint32_t *tile_cnt
     return LSTC_OK;
 }
 
-// Row lengths from the unique pass's row bounds (the symmetric degree).
+// Row lengths from the unique pass's row bounds (the symmetric degree; rows that
+// the pass met no key of have both bounds zero), and whether the vertex is kept.
 __global__ void k_row_lengths(const uint64_t *__restrict__ first, const uint64_t *__restrict__ last, uint32_t n,
-                              uint32_t *__restrict__ len) {
-    GRID_STRIDE(v, n) len[v] = (uint32_t)(last[v] - first[v]);
-}
-
-__global__ void k_nonzero(const uint32_t *__restrict__ deg, uint32_t n, int compact,
-                          uint32_t *__restrict__ f) {
-    GRID_STRIDE(v, n) f[v] = (!compact || deg[v] != 0) ? 1u : 0u;
+                              int compact, uint32_t *__restrict__ len, uint32_t *__restrict__ keep) {
+    GRID_STRIDE(v, n) {
+        const uint32_t d = (uint32_t)(last[v] - first[v]);
+        len[v] = d;
+        keep[v] = (!compact || d != 0) ? 1u : 0u;
+    }
 }
 
 // nid[v] = new id (from the exclusive scan of the keep flags); writes compacted offsets.
@@ -474,6 +474,93 @@ __global__ void k_vrec(const uint32_t *__restrict__ nid, const uint32_t *__restr
                        const uint64_t *__restrict__ doscan, const uint32_t *__restrict__ deg, uint32_t n,
                        VRec *__restrict__ rec) {
     GRID_STRIDE(v, n) rec[v] = VRec{nid[v], dout[v], (uint32_t)doscan[v], deg[v]};
+}
+
+// ------------------------------------------------------------------ small graphs
+// The per-vertex steps between the passes over the keys, fused for graphs of at
+// most kSmallN vertices and kSmallKeys keys: one workgroup scans all vertices, three
+// launches instead of the nine to twelve above, which cost 4-5 us each whatever
+// they do (RMAT s12 through lstc_clean_orient_split: 34 launches before, 18 now).
+static constexpr uint32_t kSmallN = 16384;
+static constexpr uint64_t kSmallKeys = 1ull << 22;
+
+// deg, keep flags, new ids and symmetric offsets from the unique pass's row bounds.
+__global__ __launch_bounds__(1024) void k_small_vertices(const uint64_t *__restrict__ first, const uint64_t *__restrict__ last,
+                                                         uint32_t n, int compact, uint32_t *__restrict__ deg,
+                                                         uint32_t *__restrict__ keepv, uint32_t *__restrict__ nid,
+                                                         uint64_t *__restrict__ sym_off, uint64_t *__restrict__ scal) {
+    // degree | keep << 32: the degrees add up to at most kSmallKeys
+    const uint64_t total = wg_scan(
+        n,
+        [&](uint64_t v) {
+            const uint64_t d = last[v] - first[v];
+            return d | (uint64_t)(!compact || d != 0 ? 1u : 0u) << 32;
+        },
+        [&](uint64_t v, uint64_t run, uint64_t own) {
+            const bool keep = own >> 32;
+            deg[v] = (uint32_t)own;
+            keepv[v] = keep;
+            nid[v] = keep ? (uint32_t)(run >> 32) : 0xFFFFFFFFu;
+            if (keep && sym_off) sym_off[run >> 32] = (uint32_t)run;
+        });
+    if (threadIdx.x == 0) {
+        scal[1] = total >> 32;
+        if (sym_off) sym_off[total >> 32] = scal[0];
+    }
+}
+
+// Tile offsets of the oriented arcs, oriented offsets, streaming-copy row starts (padded), records.
+__global__ __launch_bounds__(1024) void k_small_rows(const uint32_t *__restrict__ tile_cnt, uint64_t *__restrict__ tile_off,
+                                                     uint64_t tiles, const uint32_t *__restrict__ dout, uint32_t n,
+                                                     const uint32_t *__restrict__ nid, const uint32_t *__restrict__ deg,
+                                                     bool padded, uint64_t *__restrict__ doscan, uint64_t *__restrict__ off,
+                                                     VRec *__restrict__ rec, uint64_t *__restrict__ scal) {
+    const uint64_t m = wg_scan(
+        tiles, [&](uint64_t t) { return (uint64_t)tile_cnt[t]; },
+        [&](uint64_t t, uint64_t run, uint64_t) { tile_off[t] = run; });
+    const uint64_t total = wg_scan(
+        n, [&](uint64_t v) { return (uint64_t)dout[v] | (uint64_t)((dout[v] + 31u) & ~31u) << 32; },
+        [&](uint64_t v, uint64_t run, uint64_t own) {
+            const uint32_t id = nid[v], start = (uint32_t)run;
+            doscan[v] = start;
+            rec[v] = VRec{id, (uint32_t)own, padded ? (uint32_t)(run >> 32) : start, deg[v]};
+            if (id != 0xFFFFFFFFu) off[id] = start;
+        });
+    if (threadIdx.x == 0) {
+        scal[2] = m;
+        if (padded) scal[4] = total >> 32;
+        off[scal[1]] = m;
+    }
+}
+
+__global__ __launch_bounds__(1024) void k_small_in_offsets(const uint32_t *__restrict__ din, uint32_t n,
+                                                           const uint32_t *__restrict__ nid, uint64_t *__restrict__ in_off,
+                                                           const uint64_t *__restrict__ scal) {
+    (void)wg_scan(
+        n, [&](uint64_t v) { return (uint64_t)din[v]; },
+        [&](uint64_t v, uint64_t run, uint64_t) {
+            if (nid[v] != 0xFFFFFFFFu) in_off[nid[v]] = run;
+        });
+    if (threadIdx.x == 0) in_off[scal[1]] = scal[3];
+}
+
+// One clear for all that the passes count into: tiles look-back words, and per
+// vertex the row bounds and the two counters.
+__global__ void k_prep_init(uint32_t n, uint64_t tiles, uint64_t *__restrict__ first, uint64_t *__restrict__ last,
+                            uint32_t *__restrict__ dout, uint32_t *__restrict__ din, uint64_t *__restrict__ tstat,
+                            uint64_t *__restrict__ scal, uint32_t *__restrict__ bad, uint32_t *__restrict__ ticket) {
+    if (blockIdx.x == 0 && threadIdx.x < 8) {
+        scal[threadIdx.x] = 0;
+        if (threadIdx.x < 2) bad[threadIdx.x] = 0;
+        if (threadIdx.x == 0) *ticket = 0;
+    }
+    GRID_STRIDE(v, (uint64_t)n + 1) {
+        first[v] = 0;
+        last[v] = 0;
+        dout[v] = 0;
+        din[v] = 0;
+    }
+    GRID_STRIDE(t, tiles) tstat[t] = 0;
 }
 
 struct PrepLayout {
@@ -522,7 +609,8 @@ static PrepLayout prep_layout(void *ws, size_t ws_bytes, uint32_t n, uint64_t m_
     L.plen = c.take<uint32_t>((size_t)n + 1);
     L.pscan = c.take<uint64_t>((size_t)n + 1);
     L.scal = c.take<uint64_t>(8);
-    L.bad = c.take<uint32_t>(4);
+    L.bad = L.scal ? (uint32_t *)(L.scal + 5) : nullptr;  // behind the sizes: one copy brings both
+    (void)c.take<uint32_t>(4);
     L.sort_bytes = radix_sort_ws_bytes(nk);
     L.sort_ws = c.take<char>(L.sort_bytes);
     L.scan_bytes = scan_ws_bytes(tiles > (uint64_t)n + 1 ? tiles : (uint64_t)n + 1);
@@ -542,8 +630,8 @@ extern "C" lstc_status lstc_clean_orient_workspace(uint32_t n, uint64_t m_raw, s
 }
 
 // Enqueues the whole pipeline without synchronising.  On return *d_sizes points
-// at device words {m2, n_out, m, in-list entries} and *d_bad at the out-of-range
-// flag; both are valid once the stream reaches this point.
+// at device words {m2, n_out, m, in-list entries, streaming copy entries, flag} and
+// *d_bad at the out-of-range flag in the last of them; both are valid once the stream reaches this point.
 lstc_status lstc::clean_orient_launch(const uint32_t *d_src, const uint32_t *d_dst, uint64_t m_raw, uint32_t n,
                                       int compact, uint64_t *d_sym_off, uint32_t *d_sym_col, uint64_t *d_off,
                                       uint32_t *d_col, uint64_t *d_in_off, uint32_t *d_in_col, uint64_t *d_col_seg,
@@ -567,35 +655,36 @@ lstc_status lstc::clean_orient_launch(const uint32_t *d_src, const uint32_t *d_d
     const uint32_t grid_k = (uint32_t)hmin<uint64_t>((nk + 255) / 256 + 1, (uint64_t)device_cus() * 32);
     const uint32_t grid_n = (uint32_t)hmin<uint64_t>(((uint64_t)n + 255) / 256 + 1, (uint64_t)device_cus() * 32);
 
-    LSTC_TRY(fill_u64(L.scal, 0, 8, st));
-    LSTC_TRY(fill_u32(L.bad, 0, 4, st));
-    LSTC_TRY(fill_u32(L.deg, 0, (uint64_t)n + 1, st));
-    LSTC_TRY(fill_u32(L.dout, 0, (uint64_t)n + 1, st));
-    LSTC_TRY(fill_u32(L.din, 0, (uint64_t)n + 1, st));
+    hipLaunchKernelGGL(k_prep_init, dim3(grid_n), dim3(256), 0, st, n, tiles, L.first, L.last, L.dout, L.din, L.tstat,
+                       L.scal, L.bad, L.ticket);
+    LSTC_LAUNCHED("k_prep_init");
     if (m_raw) {
         const uint64_t kblocks = radix_blocks(nk);
         if (kblocks > 0x7FFFFFFFull) return fail(LSTC_ERR_INVALID, "lstc_clean_orient: too many edges");
         hipLaunchKernelGGL(k_make_keys, dim3((uint32_t)kblocks), dim3(256), 0, st, d_src, d_dst, m_raw, n, b, L.keys,
-                           (uint32_t)kblocks, radix_first_counts(L.sort_ws, nk), L.bad);
+                           radix_sub(nk) * (uint32_t)(kRadixTile / 2), (uint32_t)kblocks, radix_first_counts(L.sort_ws, nk), L.bad);
         LSTC_LAUNCHED("k_make_keys");
         uint64_t *sorted = nullptr;
         LSTC_TRY(radix_sort_u64(L.keys, L.alt, nk, (int)(2 * b > 64 ? 64 : 2 * b), &sorted, L.sort_ws, L.sort_bytes, st,
                                 true));
         uint64_t *uk = (sorted == L.keys) ? L.alt : L.keys;
         // unique arcs and the symmetric row bounds (m2 -> scal[0])
-        LSTC_TRY(fill_u64(L.first, 0, (uint64_t)n + 1, st));
-        LSTC_TRY(fill_u64(L.last, 0, (uint64_t)n + 1, st));
         LSTC_TRY(compact_pass(UniqueOp{sorted, nk, b, uk, L.first, L.last}, nk, L.tile_cnt, L.tile_off, L.scal + 0,
                               L.scan_ws, L.scan_bytes, st));
-        hipLaunchKernelGGL(k_row_lengths, dim3(grid_n), dim3(256), 0, st, L.first, L.last, n, L.deg);
-        LSTC_LAUNCHED("k_row_lengths(deg)");
-        hipLaunchKernelGGL(k_nonzero, dim3(grid_n), dim3(256), 0, st, L.deg, n, compact, L.keepv);
-        LSTC_LAUNCHED("k_nonzero");
-        LSTC_TRY(scan_exclusive_u32_to_u64(L.keepv, L.nidscan, n, L.scal + 1, L.scan_ws, L.scan_bytes, st));
-        LSTC_TRY(scan_exclusive_u32_to_u64(L.deg, L.degscan, n, nullptr, L.scan_ws, L.scan_bytes, st));
-        hipLaunchKernelGGL(k_relabel_offsets, dim3(grid_n), dim3(256), 0, st, L.keepv, L.nidscan, L.degscan, n,
-                           L.scal + 1, L.scal + 0, L.nid, d_sym_off);
-        LSTC_LAUNCHED("k_relabel_offsets");
+        const bool small = n <= kSmallN && nk <= kSmallKeys;
+        if (small) {
+            hipLaunchKernelGGL(k_small_vertices, dim3(1), dim3(1024), 0, st, L.first, L.last, n, compact, L.deg, L.keepv,
+                               L.nid, d_sym_off, L.scal);
+            LSTC_LAUNCHED("k_small_vertices");
+        } else {
+            hipLaunchKernelGGL(k_row_lengths, dim3(grid_n), dim3(256), 0, st, L.first, L.last, n, compact, L.deg, L.keepv);
+            LSTC_LAUNCHED("k_row_lengths");
+            LSTC_TRY(scan_exclusive_u32_to_u64(L.keepv, L.nidscan, n, L.scal + 1, L.scan_ws, L.scan_bytes, st));
+            LSTC_TRY(scan_exclusive_u32_to_u64(L.deg, L.degscan, n, nullptr, L.scan_ws, L.scan_bytes, st));
+            hipLaunchKernelGGL(k_relabel_offsets, dim3(grid_n), dim3(256), 0, st, L.keepv, L.nidscan, L.degscan, n,
+                               L.scal + 1, L.scal + 0, L.nid, d_sym_off);
+            LSTC_LAUNCHED("k_relabel_offsets");
+        }
         if (d_sym_col) {
             hipLaunchKernelGGL(k_sym_cols, dim3(grid_k), dim3(256), 0, st, uk, L.scal + 0, mask, L.nid, d_sym_col);
             LSTC_LAUNCHED("k_sym_cols");
@@ -604,28 +693,35 @@ lstc_status lstc::clean_orient_launch(const uint32_t *d_src, const uint32_t *d_d
         hipLaunchKernelGGL(k_compact_count<OrientCountOp>, dim3((uint32_t)tiles), dim3(kCT), 0, st,
                            OrientCountOp{uk, L.scal + 0, b, mask, L.deg, L.dout}, L.tile_cnt);
         LSTC_LAUNCHED("k_compact_count<orient>");
-        LSTC_TRY(scan_exclusive_u32_to_u64(L.tile_cnt, L.tile_off, tiles, L.scal + 2, L.scan_ws, L.scan_bytes, st));
-        LSTC_TRY(scan_exclusive_u32_to_u64(L.dout, L.doscan, n, nullptr, L.scan_ws, L.scan_bytes, st));
-        hipLaunchKernelGGL(k_orient_offsets, dim3(grid_n), dim3(256), 0, st, L.keepv, L.nidscan, L.doscan, n,
-                           L.scal + 1, L.scal + 2, d_off);
-        LSTC_LAUNCHED("k_orient_offsets");
-        if (d_scol) {  // the streaming copy's row starts (entries -> scal[4]); the records carry them
-            hipLaunchKernelGGL(k_pad_rows, dim3(grid_n), dim3(256), 0, st, L.dout, n, L.plen);
-            LSTC_LAUNCHED("k_pad_rows");
-            LSTC_TRY(scan_exclusive_u32_to_u64(L.plen, L.pscan, n, L.scal + 4, L.scan_ws, L.scan_bytes, st));
+        if (small) {
+            hipLaunchKernelGGL(k_small_rows, dim3(1), dim3(1024), 0, st, L.tile_cnt, L.tile_off, tiles, L.dout, n, L.nid,
+                               L.deg, d_scol != nullptr, L.doscan, d_off, L.rec, L.scal);
+            LSTC_LAUNCHED("k_small_rows");
+        } else {
+            LSTC_TRY(scan_exclusive_u32_to_u64(L.tile_cnt, L.tile_off, tiles, L.scal + 2, L.scan_ws, L.scan_bytes, st));
+            LSTC_TRY(scan_exclusive_u32_to_u64(L.dout, L.doscan, n, nullptr, L.scan_ws, L.scan_bytes, st));
+            hipLaunchKernelGGL(k_orient_offsets, dim3(grid_n), dim3(256), 0, st, L.keepv, L.nidscan, L.doscan, n,
+                               L.scal + 1, L.scal + 2, d_off);
+            LSTC_LAUNCHED("k_orient_offsets");
+            if (d_scol) {  // the streaming copy's row starts (entries -> scal[4]); the records carry them
+                hipLaunchKernelGGL(k_pad_rows, dim3(grid_n), dim3(256), 0, st, L.dout, n, L.plen);
+                LSTC_LAUNCHED("k_pad_rows");
+                LSTC_TRY(scan_exclusive_u32_to_u64(L.plen, L.pscan, n, L.scal + 4, L.scan_ws, L.scan_bytes, st));
+            }
+            hipLaunchKernelGGL(k_vrec, dim3(grid_n), dim3(256), 0, st, L.nid, L.dout, d_scol ? L.pscan : L.doscan, L.deg,
+                               n, L.rec);
+            LSTC_LAUNCHED("k_vrec");
         }
-        hipLaunchKernelGGL(k_vrec, dim3(grid_n), dim3(256), 0, st, L.nid, L.dout, d_scol ? L.pscan : L.doscan, L.deg,
-                           n, L.rec);
-        LSTC_LAUNCHED("k_vrec");
         // scatter pass: columns (and segment words); in-lists (entries -> scal[3]) in the same pass
-        LSTC_TRY(fill_u64(L.tstat, 0, tiles, st));
-        LSTC_TRY(fill_u32(L.ticket, 0, 1, st));
         hipLaunchKernelGGL(k_orient_in_scatter, dim3((uint32_t)tiles), dim3(kCT), 0, st,
                            OrientInPass{uk, L.scal + 0, b, mask, L.rec, d_col, d_col_seg, d_in_col, d_in_seg, L.din,
                                         L.tstat, L.ticket, L.scal + 3, L.bad, d_scol, L.doscan},
                            (const uint64_t *)L.tile_off);
         LSTC_LAUNCHED("k_orient_in_scatter");
-        if (d_in_off) {
+        if (d_in_off && small) {
+            hipLaunchKernelGGL(k_small_in_offsets, dim3(1), dim3(1024), 0, st, L.din, n, L.nid, d_in_off, L.scal);
+            LSTC_LAUNCHED("k_small_in_offsets");
+        } else if (d_in_off) {
             LSTC_TRY(scan_exclusive_u32_to_u64(L.din, L.discan, n, nullptr, L.scan_ws, L.scan_bytes, st));
             hipLaunchKernelGGL(k_orient_offsets, dim3(grid_n), dim3(256), 0, st, L.keepv, L.nidscan, L.discan, n,
                                L.scal + 1, L.scal + 3, d_in_off);
@@ -633,8 +729,8 @@ lstc_status lstc::clean_orient_launch(const uint32_t *d_src, const uint32_t *d_d
         }
     } else {
         // no edges: every vertex is isolated
-        hipLaunchKernelGGL(k_nonzero, dim3(grid_n), dim3(256), 0, st, L.deg, n, compact, L.keepv);
-        LSTC_LAUNCHED("k_nonzero");
+        hipLaunchKernelGGL(k_row_lengths, dim3(grid_n), dim3(256), 0, st, L.first, L.last, n, compact, L.deg, L.keepv);
+        LSTC_LAUNCHED("k_row_lengths");
         LSTC_TRY(scan_exclusive_u32_to_u64(L.keepv, L.nidscan, n, L.scal + 1, L.scan_ws, L.scan_bytes, st));
         LSTC_TRY(fill_u64(L.doscan, 0, (uint64_t)n + 1, st));
         hipLaunchKernelGGL(k_relabel_offsets, dim3(grid_n), dim3(256), 0, st, L.keepv, L.nidscan, L.doscan, n,
@@ -669,11 +765,10 @@ static lstc_status clean_orient_split_impl(const char *who, const uint32_t *d_sr
     const uint32_t *d_bad = nullptr;
     LSTC_TRY(clean_orient_launch(d_src, d_dst, m_raw, n, compact, d_sym_off, d_sym_col, d_off, d_col, d_in_off,
                                  d_in_col, d_col_seg, d_in_seg, d_ws, ws_bytes, st, &d_sizes, &d_bad, d_scol));
-    uint64_t h[5];
-    uint32_t bad = 0;
+    uint64_t h[6];
     LSTC_HIP(hipMemcpyAsync(h, d_sizes, sizeof(h), hipMemcpyDeviceToHost, st));
-    LSTC_HIP(hipMemcpyAsync(&bad, d_bad, sizeof(bad), hipMemcpyDeviceToHost, st));
     LSTC_HIP(hipStreamSynchronize(st));
+    const uint32_t bad = (uint32_t)h[5];
     if (bad & 2u) return fail(LSTC_ERR_DEVICE, "%s: in-list look-back exceeded its bound", who);
     if (bad) return fail(LSTC_ERR_INVALID, "%s: vertex id >= n in input", who);
     *n_out = (uint32_t)h[1];
@@ -725,11 +820,10 @@ extern "C" lstc_status lstc_clean_orient(const uint32_t *d_src, const uint32_t *
         return fail(LSTC_ERR_INVALID, "lstc_clean_orient: give both in-list outputs or neither");
     LSTC_TRY(clean_orient_launch(d_src, d_dst, m_raw, n, compact, d_sym_off, d_sym_col, d_off, d_col, d_in_off,
                                  d_in_col, nullptr, nullptr, d_ws, ws_bytes, st, &d_sizes, &d_bad));
-    uint64_t h[4];
-    uint32_t bad = 0;
+    uint64_t h[6];
     LSTC_HIP(hipMemcpyAsync(h, d_sizes, sizeof(h), hipMemcpyDeviceToHost, st));
-    LSTC_HIP(hipMemcpyAsync(&bad, d_bad, sizeof(bad), hipMemcpyDeviceToHost, st));
     LSTC_HIP(hipStreamSynchronize(st));
+    const uint32_t bad = (uint32_t)h[5];
     if (bad & 2u) return fail(LSTC_ERR_DEVICE, "lstc_clean_orient: in-list look-back exceeded its bound");
     if (bad) return fail(LSTC_ERR_INVALID, "lstc_clean_orient: vertex id >= n in input");
     *n_out = (uint32_t)h[1];

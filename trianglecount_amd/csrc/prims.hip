@@ -6,6 +6,7 @@
 // :468-495, cp.cumsum at Med_dataset/without_part_preprocess.py:256).
 #include "lstc_internal.h"
 #include "wave.h"
+#include "wgscan.h"
 
 namespace lstc {
 
@@ -30,10 +31,14 @@ lstc_status fill_u32(uint32_t *p, uint32_t v, uint64_t n, hipStream_t s) { retur
 lstc_status fill_u8(uint8_t *p, uint8_t v, uint64_t n, hipStream_t s) { return fill_impl(p, v, n, s, "fill_u8"); }
 
 // ------------------------------------------------------------------ scan
-// Tile = 256 threads x 16 items.  reduce -> (recursive) scan of tile sums -> downsweep.
+// Tile = 256 threads x 16 items.  reduce -> downsweep, whose workgroups add up the
+// sums of the tiles before theirs (at most kScanRaw of them, 16 loads per thread: a
+// launch of its own for them costs more, 4 us, than that), or for more tiles a
+// (recursive) scan of the tile sums in between.
 static constexpr int kScanThreads = 256;
 static constexpr int kScanItems = 16;
 static constexpr uint64_t kScanTile = kScanThreads * kScanItems;
+static constexpr uint64_t kScanRaw = 4096;
 
 template <class TI>
 __device__ __forceinline__ uint64_t block_excl_scan(uint64_t v, uint64_t *s_w, uint64_t *total) {
@@ -74,7 +79,8 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_reduce(const TI *__restri
 // rows are padded by one item per 16 so the per-thread reads do not collide
 // on banks.  `in` may alias `out`: every read of the tile precedes the first
 // barrier and every write follows it.
-template <class TI>
+// RAW: tile_off holds the tiles' sums, else their exclusive prefixes.
+template <class TI, bool RAW>
 __global__ __launch_bounds__(kScanThreads) void k_scan_down(const TI *in, uint64_t *out, uint64_t n,
                                                             const uint64_t *__restrict__ tile_off,
                                                             uint64_t *__restrict__ d_total) {
@@ -95,8 +101,15 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_down(const TI *in, uint64
         x[r] = s_x[e + e / 16];
         v += x[r];
     }
-    uint64_t tot;
-    uint64_t run = block_excl_scan<TI>(v, s_w, &tot) + (tile_off ? tile_off[blockIdx.x] : 0);
+    uint64_t tot, before = 0;
+    if (RAW) {
+        for (uint32_t t = tid; t < blockIdx.x; t += kScanThreads) before += tile_off[t];
+        (void)block_excl_scan<TI>(before, s_w, &tot);
+        before = tot;
+    } else if (tile_off) {
+        before = tile_off[blockIdx.x];
+    }
+    uint64_t run = block_excl_scan<TI>(v, s_w, &tot) + before;
     // block_excl_scan's barriers order every thread's reads of s_x before these writes
 #pragma unroll
     for (int r = 0; r < kScanItems; ++r) {
@@ -111,6 +124,16 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_down(const TI *in, uint64
         const uint32_t e = r * kScanThreads + tid;
         if (tb + e < n) out[tb + e] = s_x[e + e / 16];
     }
+}
+
+// A few tiles by one workgroup: one launch instead of two.
+static constexpr uint64_t kScanOne = 4 * kScanTile;
+
+template <class TI>
+__global__ __launch_bounds__(1024) void k_scan_one(const TI *in, uint64_t *out, uint64_t n, uint64_t *__restrict__ d_total) {
+    const uint64_t total = wg_scan(
+        n, [&](uint64_t i) { return (uint64_t)in[i]; }, [&](uint64_t i, uint64_t run, uint64_t) { out[i] = run; });
+    if (d_total && threadIdx.x == 0) *d_total = total;
 }
 
 static size_t scan_ws_rec(uint64_t n) {
@@ -129,9 +152,14 @@ static lstc_status scan_impl(const TI *in, uint64_t *out, uint64_t n, uint64_t *
     }
     const uint64_t tiles = (n + kScanTile - 1) / kScanTile;
     if (tiles == 1) {
-        hipLaunchKernelGGL(k_scan_down<TI>, dim3(1), dim3(kScanThreads), 0, s, in, out, n,
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_scan_down<TI, false>), dim3(1), dim3(kScanThreads), 0, s, in, out, n,
                            (const uint64_t *)nullptr, d_total);
         LSTC_LAUNCHED("k_scan_down");
+        return LSTC_OK;
+    }
+    if (n <= kScanOne) {
+        hipLaunchKernelGGL(k_scan_one<TI>, dim3(1), dim3(1024), 0, s, in, out, n, d_total);
+        LSTC_LAUNCHED("k_scan_one");
         return LSTC_OK;
     }
     if (tiles > 0xFFFFFFFFull) return fail(LSTC_ERR_INVALID, "scan: too many items");
@@ -140,9 +168,14 @@ static lstc_status scan_impl(const TI *in, uint64_t *out, uint64_t n, uint64_t *
     uint64_t *sums = (uint64_t *)ws;
     hipLaunchKernelGGL(k_scan_reduce<TI>, dim3((uint32_t)tiles), dim3(kScanThreads), 0, s, in, n, sums);
     LSTC_LAUNCHED("k_scan_reduce");
-    LSTC_TRY(scan_impl<uint64_t>(sums, sums, tiles, nullptr, (char *)ws + need, ws_bytes - need, s));
-    hipLaunchKernelGGL(k_scan_down<TI>, dim3((uint32_t)tiles), dim3(kScanThreads), 0, s, in, out, n,
-                       (const uint64_t *)sums, d_total);
+    if (tiles <= kScanRaw) {
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_scan_down<TI, true>), dim3((uint32_t)tiles), dim3(kScanThreads), 0, s, in,
+                           out, n, (const uint64_t *)sums, d_total);
+    } else {
+        LSTC_TRY(scan_impl<uint64_t>(sums, sums, tiles, nullptr, (char *)ws + need, ws_bytes - need, s));
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_scan_down<TI, false>), dim3((uint32_t)tiles), dim3(kScanThreads), 0, s, in,
+                           out, n, (const uint64_t *)sums, d_total);
+    }
     LSTC_LAUNCHED("k_scan_down");
     return LSTC_OK;
 }
@@ -158,8 +191,9 @@ lstc_status scan_exclusive_u32_to_u64(const uint32_t *in, uint64_t *out, uint64_
 
 // ------------------------------------------------------------------ radix sort
 // LSD over 8-bit digits; per digit a histogram pass, one scan of the
-// digit-major block counts, and a scatter pass.  A block owns kSortSub
-// consecutive sub-tiles of 4 waves x 16 rounds x 64 lanes = 4096 keys; key i of
+// digit-major block counts, and a scatter pass.  A block owns radix_sub(n)
+// consecutive sub-tiles (four, or one when four would leave CUs without a block:
+// 131072 keys took 29 us a scatter pass in 8 blocks) of 4 waves x 16 rounds x 64 lanes = 4096 keys; key i of
 // a sub-tile sits at (wave, round, lane) = (i / 1024, (i / 64) % 16, i % 64), so
 // ranking in that lexicographic order, sub-tile after sub-tile, is stable.
 // Owning several sub-tiles keeps the count matrix (one count per block and
@@ -168,22 +202,20 @@ lstc_status scan_exclusive_u32_to_u64(const uint32_t *in, uint64_t *out, uint64_
 // they work on the current one.
 static constexpr int kSortWaves = 4;
 static constexpr int kSortRounds = 16;
-static constexpr uint32_t kSortSub = 4;
 static constexpr uint64_t kSortTile = kSortWaves * kSortRounds * 64;  // keys per sub-tile
-static constexpr uint64_t kSortBlock = kSortTile * kSortSub;          // keys per block
-static_assert(kSortBlock == kRadixBlock, "the sort's block is the one key producers count by");
+static_assert(kSortTile == kRadixTile, "the sort's sub-tile is the one key producers count by");
 
 // Digit counts of each block.  The keys are loaded with the non-temporal hint:
 // each is read once here, and the pass measured 12% faster with it (0.40 vs
 // 0.45 ms per pass on 268 M keys); the scatter's own loads and stores keep the
 // default policy, where the hint measured slower.
 __global__ __launch_bounds__(kSortWaves * 64) void k_radix_hist(const uint64_t *__restrict__ keys,
-                                                                uint64_t n, uint32_t shift,
+                                                                uint64_t n, uint32_t shift, uint32_t subs,
                                                                 uint32_t num_blocks,
                                                                 uint32_t *__restrict__ hist) {
     __shared__ uint32_t cnt[256];
     cnt[threadIdx.x] = 0;
-    const uint64_t base = (uint64_t)blockIdx.x * kSortBlock;
+    const uint64_t base = (uint64_t)blockIdx.x * subs * kSortTile;
     uint64_t k[kSortRounds];
 #pragma unroll
     for (int r = 0; r < kSortRounds; ++r) {
@@ -191,10 +223,10 @@ __global__ __launch_bounds__(kSortWaves * 64) void k_radix_hist(const uint64_t *
         k[r] = i < n ? __builtin_nontemporal_load(&keys[i]) : 0;
     }
     __syncthreads();
-    for (uint32_t sub = 0; sub < kSortSub; ++sub) {
+    for (uint32_t sub = 0; sub < subs; ++sub) {
         const uint64_t b0 = base + sub * kSortTile;
         uint64_t kn[kSortRounds];
-        if (sub + 1 < kSortSub) {
+        if (sub + 1 < subs) {
 #pragma unroll
             for (int r = 0; r < kSortRounds; ++r) {
                 const uint64_t i = b0 + kSortTile + (uint64_t)r * (kSortWaves * 64) + threadIdx.x;
@@ -205,7 +237,7 @@ __global__ __launch_bounds__(kSortWaves * 64) void k_radix_hist(const uint64_t *
         for (int r = 0; r < kSortRounds; ++r)
             if (b0 + (uint64_t)r * (kSortWaves * 64) + threadIdx.x < n)
                 atomicAdd(&cnt[(uint32_t)(k[r] >> shift) & 255u], 1u);
-        if (sub + 1 < kSortSub) {
+        if (sub + 1 < subs) {
 #pragma unroll
             for (int r = 0; r < kSortRounds; ++r) k[r] = kn[r];
         }
@@ -220,7 +252,7 @@ __global__ __launch_bounds__(kSortWaves * 64) void k_radix_hist(const uint64_t *
 // digit's run of the sub-tile leaves as contiguous stores; the block's running
 // offset of each digit advances by the sub-tile's count.
 __global__ __launch_bounds__(kSortWaves * 64) void k_radix_scatter(
-    const uint64_t *__restrict__ keys, uint64_t *__restrict__ out, uint64_t n, uint32_t shift,
+    const uint64_t *__restrict__ keys, uint64_t *__restrict__ out, uint64_t n, uint32_t shift, uint32_t subs,
     uint32_t num_blocks, const uint64_t *__restrict__ goff) {
     __shared__ uint32_t wcnt[kSortWaves][256];
     __shared__ uint32_t dstart[256];
@@ -231,19 +263,19 @@ __global__ __launch_bounds__(kSortWaves * 64) void k_radix_scatter(
     uint64_t run = goff[(uint64_t)tid * num_blocks + blockIdx.x];  // digit tid's next output position
     uint64_t k[kSortRounds];
     {
-        const uint64_t b = (uint64_t)blockIdx.x * kSortBlock + (uint64_t)wv * (kSortRounds * 64);
+        const uint64_t b = (uint64_t)blockIdx.x * subs * kSortTile + (uint64_t)wv * (kSortRounds * 64);
 #pragma unroll
         for (int r = 0; r < kSortRounds; ++r) {
             const uint64_t i = b + (uint64_t)r * 64 + lane;
             k[r] = i < n ? keys[i] : 0;
         }
     }
-    for (uint32_t sub = 0; sub < kSortSub; ++sub) {
-        const uint64_t tile0 = (uint64_t)blockIdx.x * kSortBlock + sub * kSortTile;
+    for (uint32_t sub = 0; sub < subs; ++sub) {
+        const uint64_t tile0 = ((uint64_t)blockIdx.x * subs + sub) * kSortTile;
         if (tile0 >= n) break;  // block-uniform
         const uint64_t base = tile0 + (uint64_t)wv * (kSortRounds * 64);
         uint64_t kn[kSortRounds];
-        if (sub + 1 < kSortSub) {
+        if (sub + 1 < subs) {
 #pragma unroll
             for (int r = 0; r < kSortRounds; ++r) {
                 const uint64_t i = base + kSortTile + (uint64_t)r * 64 + lane;
@@ -302,7 +334,7 @@ __global__ __launch_bounds__(kSortWaves * 64) void k_radix_scatter(
             const uint64_t key = stage[i];
             out[gbase[(uint32_t)(key >> shift) & 255u] + i] = key;
         }
-        if (sub + 1 < kSortSub) {
+        if (sub + 1 < subs) {
 #pragma unroll
             for (int r = 0; r < kSortRounds; ++r) k[r] = kn[r];
         }
@@ -312,7 +344,8 @@ __global__ __launch_bounds__(kSortWaves * 64) void k_radix_scatter(
 
 static size_t radix_layout(uint64_t n, uint32_t **hist, uint64_t **goff, void **scan_ws,
                            size_t *scan_bytes, void *ws, size_t ws_bytes) {
-    const uint64_t tiles = (n + kSortBlock - 1) / kSortBlock;
+    // (room for the most blocks of any smaller n, so the size grows with n)
+    const uint64_t tiles = hmax(radix_blocks(n), radix_blocks(hmin(n, kRadixFew - 1)));
     Carver c(ws, ws_bytes);
     *hist = c.take<uint32_t>(tiles * 256);
     *goff = c.take<uint64_t>(tiles * 256);
@@ -341,18 +374,19 @@ lstc_status radix_sort_u64(uint64_t *keys, uint64_t *alt, uint64_t n, int key_bi
     uint32_t *hist; uint64_t *goff; void *sws; size_t sb;
     size_t need = radix_layout(n, &hist, &goff, &sws, &sb, ws, ws_bytes);
     if (!ws || ws_bytes < need) return fail(LSTC_ERR_WORKSPACE, "radix sort: workspace too small");
-    const uint64_t tiles = (n + kSortBlock - 1) / kSortBlock;
+    const uint64_t tiles = radix_blocks(n);
+    const uint32_t subs = radix_sub(n);
     if (tiles > 0x7FFFFFFFull) return fail(LSTC_ERR_INVALID, "radix sort: too many keys");
     uint64_t *in = keys, *out = alt;
     for (int shift = 0; shift < key_bits; shift += 8) {
         if (shift > 0 || !first_counts_ready) {
             hipLaunchKernelGGL(k_radix_hist, dim3((uint32_t)tiles), dim3(kSortWaves * 64), 0, s, in, n,
-                               (uint32_t)shift, (uint32_t)tiles, hist);
+                               (uint32_t)shift, subs, (uint32_t)tiles, hist);
             LSTC_LAUNCHED("k_radix_hist");
         }
         LSTC_TRY(scan_exclusive_u32_to_u64(hist, goff, tiles * 256, nullptr, sws, sb, s));
         hipLaunchKernelGGL(k_radix_scatter, dim3((uint32_t)tiles), dim3(kSortWaves * 64), 0, s, in,
-                           out, n, (uint32_t)shift, (uint32_t)tiles, goff);
+                           out, n, (uint32_t)shift, subs, (uint32_t)tiles, goff);
         LSTC_LAUNCHED("k_radix_scatter");
         uint64_t *t = in; in = out; out = t;
     }
