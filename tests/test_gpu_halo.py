@@ -334,3 +334,20 @@ def test_halo_parts_build_reports_sizes_when_too_small(lstc, oracle):
     assert st == -1
     assert [(nl[p], no[p], ml[p]) for p in range(3)] == [(h.n, h.owned, h.m) for h in want]
     assert all(int(off[0].item()) == -7 for off, _ in keep)
+
+
+@pytest.mark.parametrize("degree", [2047, 2048, 2049, 5000])
+@pytest.mark.parametrize("k,mode", [(1, 0), (5, 1), (8, 0), (11, 0)])
+def test_halo_parts_long_rows(lstc, oracle, degree, k, mode):
+    """Hub rows on both sides of the length from which a workgroup walks them, joined to each other."""
+    rng = np.random.default_rng(degree)
+    n, hubs = 6000, 4
+    far = [rng.choice(np.arange(hubs, n), degree - (hubs - 1), replace=False) for _ in range(hubs)]
+    pairs = [(h, o) for h in range(hubs) for o in range(h)]
+    s = np.concatenate([np.full(len(f), h) for h, f in enumerate(far)] + [[a for a, _ in pairs], rng.integers(0, n, 3000)])
+    d = np.concatenate(far + [[b for _, b in pairs], rng.integers(0, n, 3000)])
+    s, d = s.astype(np.uint32), d.astype(np.uint32)
+    g = _device_graph(lstc, n, s, d)
+    sym, _ = oracle.clean_orient(n, s, d)
+    part = lstc.partition_random(g.n, k, seed=7)
+    _parts_equal_oracle(lstc, oracle, g, sym, part, oracle.partition_random(sym.n, k, seed=7), k, mode, degree)

@@ -62,9 +62,29 @@ __device__ __forceinline__ unsigned long long wave_or64(unsigned long long v) {
     return v;
 }
 
-__global__ void k_hp_init(const uint64_t *__restrict__ off, const uint32_t *__restrict__ part, uint32_t n,
-                          uint32_t k, VInfo *__restrict__ info) {
-    for (uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; v < n; v += (uint64_t)gridDim.x * blockDim.x) {
+// Rows of kLongArcs arcs or more are listed by k_hp_init and walked by a whole
+// workgroup, before it takes its share of the others, one wave each: a wave walks
+// 64 arcs per 1-2 us (two to three dependent loads), so that the hubs of RMAT s21
+// (10^5 arcs) alone kept every pass waiting.  s21, 8 parts: masks 1.31 -> 0.61 ms,
+// lengths 2.63 -> 1.09, fill 3.40 -> 2.86; the call 7.90 -> 4.79 (kLongArcs 512: 5.47,
+// 1024: 4.90; workgroups of 4 waves 5.23, of 16 5.23).  What is left are the gathers of
+// the neighbours' records and local ids, a 128-byte line each.
+static constexpr uint32_t kLongArcs = 2048;
+static constexpr uint32_t kHpWaves = 8;  // waves of a workgroup
+
+__global__ __launch_bounds__(256) void k_hp_init(const uint64_t *__restrict__ off, const uint32_t *__restrict__ part,
+                                                 uint32_t n, uint32_t k, VInfo *__restrict__ info,
+                                                 uint32_t *__restrict__ long_rows, uint32_t *__restrict__ n_long) {
+    constexpr uint32_t kPer = 8;  // vertices per thread: the workgroup takes its places in the list with one atomic
+    __shared__ uint32_t s_n, s_at;
+    if (threadIdx.x == 0) s_n = 0;
+    __syncthreads();
+    uint32_t at[kPer];
+    uint32_t lng = 0;  // bit i: vertex i of this thread has a long row
+#pragma unroll
+    for (uint32_t i = 0; i < kPer; ++i) {
+        const uint64_t v = ((uint64_t)blockIdx.x * kPer + i) * 256 + threadIdx.x;
+        if (v >= n) break;
         const uint32_t p = part[v];
         VInfo x;
         x.mem = 0;
@@ -73,31 +93,62 @@ __global__ void k_hp_init(const uint64_t *__restrict__ off, const uint32_t *__re
         x.part = p < k ? p : kNoLoc;
         x.pad[0] = x.pad[1] = 0;
         info[v] = x;
+        if (x.deg >= kLongArcs) {
+            at[i] = atomicAdd(&s_n, 1u);
+            lng |= 1u << i;
+        }
     }
+    __syncthreads();
+    if (threadIdx.x == 0 && s_n) s_at = atomicAdd(n_long, s_n);
+    __syncthreads();
+#pragma unroll
+    for (uint32_t i = 0; i < kPer; ++i)
+        if (lng >> i & 1u) long_rows[s_at + at[i]] = (uint32_t)(((uint64_t)blockIdx.x * kPer + i) * 256 + threadIdx.x);
 }
 
-// mem[v] = own part | parts of the neighbours d that put v into their halo:
-// every neighbour (mode 0) or the neighbours with an arc d -> v (mode 1).
-__global__ __launch_bounds__(256) void k_hp_mask(const uint64_t *__restrict__ off, const uint32_t *__restrict__ col,
-                                                 const uint32_t *__restrict__ part, uint32_t n, uint32_t k, int mode,
-                                                 VInfo *__restrict__ info) {
-    const uint32_t lane = threadIdx.x & 63;
-    const uint64_t nw = (uint64_t)gridDim.x * (blockDim.x >> 6);
-    for (uint64_t v = (uint64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); v < n; v += nw) {
-        const uint64_t b = off[v], e = off[v + 1];
-        const uint32_t dv = (uint32_t)(e - b);
-        unsigned long long m = 0;
-        for (uint64_t j = b + lane; j < e; j += 64) {
-            const uint32_t d = col[j];
-            if (mode == 0) {  // the 4-byte part id is all a neighbour needs
-                const uint32_t pd = part[d];
-                if (pd < k) m |= 1ull << pd;
-            } else {
-                const VInfo x = info[d];
-                if (x.part != kNoLoc && keep_arc(x.deg, dv, d, (uint32_t)v)) m |= 1ull << x.part;
-            }
+// The parts that arcs [b + first, e) of row v, every step-th, put v into.
+__device__ __forceinline__ unsigned long long hp_mask_of(const uint32_t *__restrict__ col, const uint32_t *__restrict__ part,
+                                                         const VInfo *__restrict__ info, uint32_t k, int mode, uint32_t v,
+                                                         uint64_t b, uint64_t e, uint32_t first, uint32_t step) {
+    const uint32_t dv = (uint32_t)(e - b);
+    unsigned long long m = 0;
+    for (uint64_t j = b + first; j < e; j += step) {
+        const uint32_t d = col[j];
+        if (mode == 0) {  // the 4-byte part id is all a neighbour needs
+            const uint32_t pd = part[d];
+            if (pd < k) m |= 1ull << pd;
+        } else {
+            const VInfo x = info[d];
+            if (x.part != kNoLoc && keep_arc(x.deg, dv, d, v)) m |= 1ull << x.part;
         }
-        m = wave_or64(m);
+    }
+    return wave_or64(m);
+}
+
+__global__ __launch_bounds__(kHpWaves * 64) void k_hp_mask(const uint64_t *__restrict__ off, const uint32_t *__restrict__ col,
+                                                 const uint32_t *__restrict__ part, uint32_t n, uint32_t k, int mode,
+                                                 VInfo *__restrict__ info, const uint32_t *__restrict__ long_rows,
+                                                 const uint32_t *__restrict__ n_long) {
+    __shared__ unsigned long long s_m[kHpWaves];
+    const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    for (uint32_t i = blockIdx.x; i < *n_long; i += gridDim.x) {
+        const uint32_t v = long_rows[i];
+        const unsigned long long m = hp_mask_of(col, part, info, k, mode, v, off[v], off[v + 1], threadIdx.x, blockDim.x);
+        if (lane == 0) s_m[wv] = m;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            unsigned long long all = 0;
+            for (uint32_t w = 0; w < kHpWaves; ++w) all |= s_m[w];
+            const uint32_t p = info[v].part;
+            info[v].mem = p == kNoLoc ? all : all | (1ull << p);
+        }
+        __syncthreads();
+    }
+    const uint64_t nw = (uint64_t)gridDim.x * kHpWaves;
+    for (uint64_t v = (uint64_t)blockIdx.x * kHpWaves + wv; v < n; v += nw) {
+        const uint64_t b = off[v], e = off[v + 1];
+        if (e - b >= kLongArcs) continue;
+        const unsigned long long m = hp_mask_of(col, part, info, k, mode, (uint32_t)v, b, e, lane, 64);
         if (lane == 0) {
             const uint32_t p = info[v].part;
             info[v].mem = p == kNoLoc ? m : m | (1ull << p);
@@ -227,98 +278,155 @@ __global__ void k_hp_l2g(const VInfo *__restrict__ info, const uint32_t *__restr
     }
 }
 
-// One wave per vertex s; FILL = 0 counts each part's kept arcs of row s
-// (rowlen[p][local row], and those into P_p: rowp[p][local row]); FILL = 1
-// writes them.
-// Lane p holds part p's state: counters, or the two write positions.
+// What a wave keeps of a row: lane p has part p's counters of kept arcs, all and
+// those into P_p (FILL = 0), or its two write positions (FILL = 1).
+struct HpRow {
+    uint32_t cnt, cntp;
+    uint64_t posp, posh;
+    uint32_t *ocol;
+};
+
+// One wave walks arcs [b, e) of row s (ds arcs in all, parts ms): counts each part's
+// kept arcs or writes them.
 template <int FILL>
-__global__ __launch_bounds__(256) void k_hp_rows(const uint64_t *__restrict__ off, const uint32_t *__restrict__ col,
+__device__ __forceinline__ void hp_walk(const uint32_t *__restrict__ col, uint32_t k, const VInfo *__restrict__ info,
+                                        const uint32_t *__restrict__ lids, uint32_t s, uint32_t ds, unsigned long long ms,
+                                        uint64_t b, uint64_t e, uint32_t lane, HpRow &R) {
+    uint32_t &cnt = R.cnt, &cntp = R.cntp;
+    uint64_t &posp = R.posp, &posh = R.posh;
+    uint32_t *const ocol = R.ocol;
+    for (uint64_t j0 = b; j0 < e; j0 += 64) {
+        const uint64_t j = j0 + lane;
+        uint32_t d = 0;
+        unsigned long long md = 0, dmem = 0, dbase = 0;
+        uint32_t pd = kNoLoc;
+        if (j < e) {
+            d = col[j];
+            const VInfo x = info[d];
+            if (keep_arc(ds, x.deg, (uint32_t)s, d)) {
+                md = x.mem & ms;
+                dmem = x.mem;
+                dbase = x.lbase;
+                pd = x.part;
+            }
+        }
+        // with at most 8 parts, the target's local ids in all its parts (side by side in
+        // lids) are loaded together here rather than one after another in the part loop
+        uint32_t l8[8];
+        if (FILL && k <= 8) {
+            const uint32_t np = (uint32_t)__popcll(md ? dmem : 0ull);
+#pragma unroll
+            for (uint32_t r = 0; r < 8; ++r) l8[r] = r < np ? lids[dbase + r] : 0u;
+        }
+        for (unsigned long long rest = ms; rest;) {
+            const uint32_t p = (uint32_t)__builtin_ctzll(rest);
+            rest &= rest - 1;
+            const bool in = (md >> p) & 1ull, inp = in && pd == p;
+            const uint64_t mP = ballot(inp), mA = ballot(in);
+            if (!FILL) {
+                if (lane == p) {
+                    cnt += (uint32_t)__popcll(mA);
+                    cntp += (uint32_t)__popcll(mP);
+                }
+            } else {
+                const uint64_t mH = mA & ~mP;
+                if (mA) {
+                    const uint64_t bp = read_lane64(posp, p), bh = read_lane64(posh, p);
+                    uint32_t *oc = (uint32_t *)read_lane64((uint64_t)ocol, p);
+                    if (in) {
+                        const uint32_t rk = lid_rank(dmem, p);
+                        uint32_t ld;
+                        if (k <= 8) {
+                            ld = l8[0];
+#pragma unroll
+                            for (uint32_t r = 1; r < 8; ++r) ld = rk == r ? l8[r] : ld;
+                        } else {
+                            ld = lids[dbase + rk];
+                        }
+                        if (inp) oc[bp + mask_rank(mP)] = ld;
+                        else oc[bh + mask_rank(mH)] = ld;
+                    }
+                    if (lane == p) {
+                        posp += (uint64_t)__popcll(mP);
+                        posh += (uint64_t)__popcll(mH);
+                    }
+                }
+            }
+        }
+    }
+}
+
+// FILL = 0: each part's kept arcs of every row (rowlen[p][local row], and those
+// into P_p: rowp[p][local row]); FILL = 1: the arcs themselves.  Long rows first, a
+// workgroup each, its waves on consecutive segments (which the fill counts first, to
+// know where each segment's arcs go); then a wave per row.
+template <int FILL>
+__global__ __launch_bounds__(kHpWaves * 64) void k_hp_rows(const uint64_t *__restrict__ off, const uint32_t *__restrict__ col,
                                                  uint32_t n, uint32_t k, const VInfo *__restrict__ info,
                                                  const uint32_t *__restrict__ lids, uint32_t *__restrict__ rowlen,
                                                  uint32_t *__restrict__ rowp, unsigned long long *__restrict__ m_tot,
-                                                 const PartOut *__restrict__ outs) {
-    const uint32_t lane = threadIdx.x & 63;
-    const uint64_t nw = (uint64_t)gridDim.x * (blockDim.x >> 6);
+                                                 const PartOut *__restrict__ outs, const uint32_t *__restrict__ long_rows,
+                                                 const uint32_t *__restrict__ n_long) {
+    __shared__ uint32_t s_all[kHpWaves][64], s_own[kHpWaves][64];
+    const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     unsigned long long arcs = 0;  // lane p: arcs of part p over this wave's rows (FILL = 0)
-    for (uint64_t s = (uint64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); s < n; s += nw) {
-        const unsigned long long ms = read_lane64(info[s].mem, 0);  // wave-uniform
-        if (ms == 0) continue;
-        const uint64_t sbase = read_lane64(info[s].lbase, 0);
+    // this lane's part's view of row s
+    auto start = [&](uint32_t s, unsigned long long ms, uint32_t &ls) {
+        HpRow R{0, 0, 0, 0, nullptr};
+        const bool mine = lane < k && ((ms >> lane) & 1ull);
+        ls = mine ? lids[info[s].lbase + lid_rank(ms, lane)] : 0u;  // s's local row in part `lane`
+        if (FILL && mine) {
+            R.posp = outs[lane].off[ls];
+            R.posh = R.posp + rowp[(uint64_t)lane * n + ls];
+            R.ocol = outs[lane].col;
+        }
+        return R;
+    };
+    for (uint32_t i = blockIdx.x; i < *n_long; i += gridDim.x) {
+        const uint32_t s = long_rows[i];
+        const unsigned long long ms = read_lane64(info[s].mem, 0);
+        if (ms == 0) continue;  // the same for the whole workgroup
         const uint64_t b = off[s], e = off[s + 1];
         const uint32_t ds = (uint32_t)(e - b);
-        const bool mine = lane < k && ((ms >> lane) & 1ull);
-        const uint32_t ls = mine ? lids[sbase + lid_rank(ms, lane)] : 0u;  // s's local row in part `lane`
-        uint32_t cnt = 0, cntp = 0;
-        uint64_t posp = 0, posh = 0;
-        uint32_t *ocol = nullptr;
-        if (FILL && mine) {
-            posp = outs[lane].off[ls];
-            posh = posp + rowp[(uint64_t)lane * n + ls];
-            ocol = outs[lane].col;
+        const uint64_t seg = ((uint64_t)ds + kHpWaves * 64 - 1) / (kHpWaves * 64) * 64;
+        const uint64_t sb = min(e, b + wv * seg), se = min(e, sb + seg);
+        uint32_t ls;
+        HpRow R = start(s, ms, ls);
+        hp_walk<0>(col, k, info, lids, s, ds, ms, sb, se, lane, R);
+        s_all[wv][lane] = R.cnt;
+        s_own[wv][lane] = R.cntp;
+        __syncthreads();
+        if (FILL) {
+            for (uint32_t w = 0; w < wv; ++w) {
+                R.posp += s_own[w][lane];
+                R.posh += s_all[w][lane] - s_own[w][lane];
+            }
+            hp_walk<1>(col, k, info, lids, s, ds, ms, sb, se, lane, R);
+        } else if (wv == 0 && lane < k && ((ms >> lane) & 1ull)) {
+            uint32_t all = 0, own = 0;
+            for (uint32_t w = 0; w < kHpWaves; ++w) {
+                all += s_all[w][lane];
+                own += s_own[w][lane];
+            }
+            rowlen[(uint64_t)lane * n + ls] = all;
+            rowp[(uint64_t)lane * n + ls] = own;
+            arcs += all;
         }
-        for (uint64_t j0 = b; j0 < e; j0 += 64) {
-            const uint64_t j = j0 + lane;
-            uint32_t d = 0;
-            unsigned long long md = 0, dmem = 0, dbase = 0;
-            uint32_t pd = kNoLoc;
-            if (j < e) {
-                d = col[j];
-                const VInfo x = info[d];
-                if (keep_arc(ds, x.deg, (uint32_t)s, d)) {
-                    md = x.mem & ms;
-                    dmem = x.mem;
-                    dbase = x.lbase;
-                    pd = x.part;
-                }
-            }
-            // with at most 8 parts, the target's local ids in all its parts (side by side in
-            // lids) are loaded together here rather than one after another in the part loop
-            uint32_t l8[8];
-            if (FILL && k <= 8) {
-                const uint32_t np = (uint32_t)__popcll(md ? dmem : 0ull);
-#pragma unroll
-                for (uint32_t r = 0; r < 8; ++r) l8[r] = r < np ? lids[dbase + r] : 0u;
-            }
-            for (unsigned long long rest = ms; rest;) {
-                const uint32_t p = (uint32_t)__builtin_ctzll(rest);
-                rest &= rest - 1;
-                const bool in = (md >> p) & 1ull, inp = in && pd == p;
-                const uint64_t mP = ballot(inp), mA = ballot(in);
-                if (!FILL) {
-                    if (lane == p) {
-                        cnt += (uint32_t)__popcll(mA);
-                        cntp += (uint32_t)__popcll(mP);
-                    }
-                } else {
-                    const uint64_t mH = mA & ~mP;
-                    if (mA) {
-                        const uint64_t bp = read_lane64(posp, p), bh = read_lane64(posh, p);
-                        uint32_t *oc = (uint32_t *)read_lane64((uint64_t)ocol, p);
-                        if (in) {
-                            const uint32_t rk = lid_rank(dmem, p);
-                            uint32_t ld;
-                            if (k <= 8) {
-                                ld = l8[0];
-#pragma unroll
-                                for (uint32_t r = 1; r < 8; ++r) ld = rk == r ? l8[r] : ld;
-                            } else {
-                                ld = lids[dbase + rk];
-                            }
-                            if (inp) oc[bp + mask_rank(mP)] = ld;
-                            else oc[bh + mask_rank(mH)] = ld;
-                        }
-                        if (lane == p) {
-                            posp += (uint64_t)__popcll(mP);
-                            posh += (uint64_t)__popcll(mH);
-                        }
-                    }
-                }
-            }
-        }
-        if (!FILL && mine) {
-            rowlen[(uint64_t)lane * n + ls] = cnt;
-            rowp[(uint64_t)lane * n + ls] = cntp;
-            arcs += cnt;
+        __syncthreads();
+    }
+    const uint64_t nw = (uint64_t)gridDim.x * kHpWaves;
+    for (uint64_t s = (uint64_t)blockIdx.x * kHpWaves + wv; s < n; s += nw) {
+        const unsigned long long ms = read_lane64(info[s].mem, 0);  // wave-uniform
+        if (ms == 0) continue;
+        const uint64_t b = off[s], e = off[s + 1];
+        if (e - b >= kLongArcs) continue;
+        uint32_t ls;
+        HpRow R = start((uint32_t)s, ms, ls);
+        hp_walk<FILL>(col, k, info, lids, (uint32_t)s, (uint32_t)(e - b), ms, b, e, lane, R);
+        if (!FILL && lane < k && ((ms >> lane) & 1ull)) {
+            rowlen[(uint64_t)lane * n + ls] = R.cnt;
+            rowp[(uint64_t)lane * n + ls] = R.cntp;
+            arcs += R.cnt;
         }
     }
     if (!FILL && lane < k && arcs) atomicAdd(m_tot + lane, arcs);
@@ -334,7 +442,8 @@ struct HPLayout {
     uint32_t *lids, *pc, *rowlen, *rowp, *cnt;
     uint64_t *lbase;
     uint64_t *tot;               // [2k]
-    unsigned long long *m_tot;   // [k]
+    unsigned long long *m_tot;   // [k], and behind them the number of long rows
+    uint32_t *long_rows, *n_long;
     PartOut *outs;               // [k]
     uint32_t **l2g;              // [k]
     void *scan_ws;
@@ -355,7 +464,9 @@ static HPLayout hp_layout(void *ws, size_t ws_bytes, uint32_t n, uint32_t k) {
     L.rowp = c.take<uint32_t>(kk * nn);
     L.cnt = c.take<uint32_t>((size_t)(L.tiles ? L.tiles : 1) * 2 * kk);
     L.tot = c.take<uint64_t>(2 * kk);
-    L.m_tot = c.take<unsigned long long>(kk);
+    L.m_tot = c.take<unsigned long long>(kk + 1);
+    L.n_long = L.m_tot ? (uint32_t *)(L.m_tot + k) : nullptr;
+    L.long_rows = c.take<uint32_t>(nn);
     L.outs = c.take<PartOut>(kk);
     L.l2g = c.take<uint32_t *>(kk);
     L.scan_bytes = scan_ws_bytes(nn);
@@ -374,16 +485,23 @@ static lstc_status hp_check(const uint64_t *off, const uint32_t *col, uint32_t n
     return LSTC_OK;
 }
 
+// Workgroups of the passes over the rows: a wave per row, up to 16 workgroups per CU.
+static uint32_t hp_grid(uint32_t n) {
+    return (uint32_t)hmin<uint64_t>(((uint64_t)n + kHpWaves - 1) / kHpWaves, (uint64_t)device_cus() * 16);
+}
+
 // membership, local ids and row lengths of every part; sizes stay on the device
 // (tot: |P_p|, |H_p|; m_tot: arcs of part p).
 static lstc_status hp_front(const uint64_t *off, const uint32_t *col, uint32_t n, const uint32_t *part, uint32_t k,
                             int mode, const HPLayout &L, hipStream_t st) {
     const int cus = device_cus();
     const uint32_t grid_n = (uint32_t)hmin<uint64_t>(((uint64_t)n + 255) / 256, (uint64_t)cus * 32);
-    const uint32_t grid_w = (uint32_t)hmin<uint64_t>(((uint64_t)n + 3) / 4, (uint64_t)cus * 32);
-    hipLaunchKernelGGL(k_hp_init, dim3(grid_n), dim3(256), 0, st, off, part, n, k, L.info);
+    const uint32_t grid_w = hp_grid(n);
+    LSTC_TRY(fill_u64((uint64_t *)L.m_tot, 0, k + 1, st));
+    hipLaunchKernelGGL(k_hp_init, dim3(ceil_div_u32(n, 2048)), dim3(256), 0, st, off, part, n, k, L.info, L.long_rows, L.n_long);
     LSTC_LAUNCHED("k_hp_init");
-    hipLaunchKernelGGL(k_hp_mask, dim3(grid_w), dim3(256), 0, st, off, col, part, n, k, mode, L.info);
+    hipLaunchKernelGGL(k_hp_mask, dim3(grid_w), dim3(kHpWaves * 64), 0, st, off, col, part, n, k, mode, L.info,
+                       (const uint32_t *)L.long_rows, (const uint32_t *)L.n_long);
     LSTC_LAUNCHED("k_hp_mask");
     hipLaunchKernelGGL(k_hp_popc, dim3(grid_n), dim3(256), 0, st, (const VInfo *)L.info, n, L.pc);
     LSTC_LAUNCHED("k_hp_popc");
@@ -396,9 +514,9 @@ static lstc_status hp_front(const uint64_t *off, const uint32_t *col, uint32_t n
     LSTC_LAUNCHED("k_hp_tilescan");
     hipLaunchKernelGGL(k_hp_local, dim3(L.tiles), dim3(256), 0, st, L.info, n, k, L.cnt, L.tot, L.lids);
     LSTC_LAUNCHED("k_hp_local");
-    LSTC_TRY(fill_u64((uint64_t *)L.m_tot, 0, k, st));
-    hipLaunchKernelGGL(k_hp_rows<0>, dim3(grid_w), dim3(256), 0, st, off, col, n, k, L.info, L.lids, L.rowlen, L.rowp,
-                       L.m_tot, (const PartOut *)nullptr);
+    hipLaunchKernelGGL(k_hp_rows<0>, dim3(grid_w), dim3(kHpWaves * 64), 0, st, off, col, n, k, L.info, L.lids, L.rowlen,
+                       L.rowp, L.m_tot, (const PartOut *)nullptr, (const uint32_t *)L.long_rows,
+                       (const uint32_t *)L.n_long);
     LSTC_LAUNCHED("k_hp_rows<0>");
     return LSTC_OK;
 }
@@ -511,9 +629,9 @@ static lstc_status hp_extract(const uint64_t *d_sym_off, const uint32_t *d_sym_c
                            (uint32_t *const *)L.l2g);
         LSTC_LAUNCHED("k_hp_l2g");
     }
-    const uint32_t grid_w = (uint32_t)hmin<uint64_t>(((uint64_t)n + 3) / 4, (uint64_t)cus * 32);
-    hipLaunchKernelGGL(k_hp_rows<1>, dim3(grid_w), dim3(256), 0, st, d_sym_off, d_sym_col, n, k, L.info, L.lids,
-                       L.rowlen, L.rowp, L.m_tot, (const PartOut *)L.outs);
+    hipLaunchKernelGGL(k_hp_rows<1>, dim3(hp_grid(n)), dim3(kHpWaves * 64), 0, st, d_sym_off, d_sym_col, n, k, L.info,
+                       L.lids, L.rowlen, L.rowp, L.m_tot, (const PartOut *)L.outs, (const uint32_t *)L.long_rows,
+                       (const uint32_t *)L.n_long);
     LSTC_LAUNCHED("k_hp_rows<1>");
     return LSTC_OK;
 }
