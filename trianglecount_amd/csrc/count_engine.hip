@@ -256,11 +256,12 @@ struct RowPlan {
     }
 };
 
-// Planned row r of the launch (r < total_rows).
-__device__ __forceinline__ RowPlan plan_row(const GraphSet &gs, const Bounds &bd, uint64_t r) {
+// Planned row r of the launch (r < total_rows); its graph is g0 or a later one.
+__device__ __forceinline__ RowPlan plan_row(const GraphSet &gs, const Bounds &bd, uint64_t r, uint32_t g0 = 0) {
     RowPlan p;
     if (gs.table) {  // last g with row_base[g] <= r
-        uint32_t lo = 0, hi = gs.G;
+        uint32_t lo = g0, hi = gs.G;
+        if (r < gload(gs.row_base + lo + 1)) hi = lo + 1;
         while (hi - lo > 1) {
             const uint32_t mid = (lo + hi) >> 1;
             if (gload(gs.row_base + mid) <= r) lo = mid; else hi = mid;
@@ -305,10 +306,12 @@ __global__ __launch_bounds__(256) void k_plan_rows(GraphSet gs, Bounds bd, uint3
     uint32_t run[kSlots];
 #pragma unroll
     for (int i = 0; i < kSlots; ++i) run[i] = PASS == 1 ? wcnt[slot_of(i) * kPlanWaves + wave] : 0u;
+    uint32_t g0 = 0;  // graph of the range's last row so far
     for (uint64_t r0 = r_begin; r0 < r_end; r0 += 64) {
         const uint64_t r = r0 + lane;
         RowPlan p;
-        if (r < r_end) p = plan_row(gs, bd, r);
+        if (r < r_end) p = plan_row(gs, bd, r, g0);
+        g0 = read_lane(p.g, 63);  // (0 behind the range's end, where no row follows)
         const int b = p.bin;
 #pragma unroll
         for (int i = 0; i < kSlots; ++i) {
@@ -813,6 +816,7 @@ struct Tickets {
     // A head never passes its class's ticket count by more than the workgroups
     // asking, so a ticket number stays below 2^32.
     __device__ __forceinline__ uint32_t next() {
+        if (n <= gridDim.x) return kEmpty;  // every ticket was some workgroup's first
         uint64_t t = (uint64_t)atomicAdd(heads + cls * kHeadStride, 1u) * classes + cls;
         for (uint32_t left = classes - 1; t >= n && left; --left) {
             cls = cls + 1 == classes ? 0 : cls + 1;

@@ -89,10 +89,13 @@ struct HubSet {
     uint64_t *rec;        // per row
     uint32_t *long_rows;  // rows of at least kTopMin entries
     uint64_t *units;
-    uint32_t *plan_cnt;   // [kHubSlots][kHubPlanWaves]
+    uint32_t *plan_cnt;   // [kHubSlots][plan_waves]
+    uint32_t plan_waves;
     uint64_t *queue;      // row | chunk << 32; tiny rows: 1 << 32 if only their in-list counts
 };
-static constexpr uint32_t kHubPlanBlocks = 512, kHubPlanWaves = kHubPlanBlocks * 4;
+// Waves of the plan: one per 512 rows, up to this many (the scan of their counters is
+// one workgroup's, 18 us for 2048 waves).
+static constexpr uint32_t kHubPlanWaves = 2048;
 // Items per ticket (at most 64), by region: a ticket of the small rows is worth one
 // item of the others, and the last tickets decide how long the chip waits for its
 // last wave.

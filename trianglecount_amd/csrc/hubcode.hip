@@ -335,6 +335,7 @@ HubSet hub_layout(Carver &c, uint64_t rows, uint64_t m) {
     h.long_rows = c.take<uint32_t>(m / kLongRow + 1);
     h.units = c.take<uint64_t>(hub_units(rows, m));
     h.plan_cnt = c.take<uint32_t>((size_t)kHubSlots * kHubPlanWaves);
+    h.plan_waves = (uint32_t)hmin<uint64_t>(kHubPlanWaves, (rows + 2047) / 2048 * 4);  // a multiple of four
     // a row of n >= kHeavy lists has at most n / 64 items, any other one; all rows have at most 2 m lists
     h.queue = c.take<uint64_t>(rows + m / 32 + 1);
     return h;

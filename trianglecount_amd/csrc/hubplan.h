@@ -6,20 +6,20 @@
 
 namespace lstc {
 
-// As the engine's plan, but each wave has every kHubPlanWaves-th group of 64 rows
+// As the engine's plan, but each wave has every plan_waves-th group of 64 rows
 // (heavy rows often lie together: 325 -> 64 us at RMAT s23 for the writing pass
 // against contiguous ranges): pass 0 counts its items per queue region,
 // hub_plan_scan turns that into positions, pass 1 writes the items.  Lane s keeps
 // the counter of region s.
 template <int PASS>
 __device__ __forceinline__ void hub_plan_rows(const GraphDev &G, const HubSet &hs, uint32_t tiny_max) {
-    if (blockIdx.x >= kHubPlanBlocks) return;
+    if (blockIdx.x * 4 >= hs.plan_waves) return;
     const uint32_t lane = threadIdx.x & 63, wave = blockIdx.x * 4 + (threadIdx.x >> 6);
     const uint64_t end = G.n_rows;
     uint32_t run = 0;
-    if (PASS == 1 && lane < kHubSlots) run = hs.plan_cnt[lane * kHubPlanWaves + wave];
+    if (PASS == 1 && lane < kHubSlots) run = hs.plan_cnt[lane * hs.plan_waves + wave];
     const uint32_t xcd = lane / kXcdSlots, step = lane % kXcdSlots;  // of lanes below kSlotLight
-    for (uint64_t r0 = wave * 64ull; r0 < end; r0 += kHubPlanWaves * 64ull) {
+    for (uint64_t r0 = wave * 64ull; r0 < end; r0 += hs.plan_waves * 64ull) {
         const uint64_t r = r0 + lane;
         uint32_t n = 0, in_only = 0;
         bool tiny = false;
@@ -54,21 +54,21 @@ __device__ __forceinline__ void hub_plan_rows(const GraphDev &G, const HubSet &h
             if (lane == slot) run += (uint32_t)__popcll(m);
         }
     }
-    if (PASS == 0 && lane < kHubSlots) hs.plan_cnt[lane * kHubPlanWaves + wave] = run;
+    if (PASS == 0 && lane < kHubSlots) hs.plan_cnt[lane * hs.plan_waves + wave] = run;
 }
 
 // One workgroup: exclusive scan of the counters in place, then the tickets.
 __device__ __forceinline__ void hub_plan_scan(const HubSet &hs, unsigned long long *counts, uint32_t grid) {
-    constexpr uint32_t kRound = 4096, kAll = kHubSlots * kHubPlanWaves;
-    static_assert(kHubPlanWaves % 4 == 0, "a slot starts on a 16-byte word");
+    constexpr uint32_t kRound = 4096;
+    const uint32_t all = kHubSlots * hs.plan_waves;  // (a slot starts on a 16-byte word)
     __shared__ uint32_t s_wave[16], s_slot[kHubSlots + 1];
     uint32_t *hctl = hs.hctl;
     const uint32_t tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     uint32_t before = 0;
-    for (uint32_t e0 = 0; e0 < kAll; e0 += kRound) {
+    for (uint32_t e0 = 0; e0 < all; e0 += kRound) {
         const uint32_t e = e0 + 4 * tid;
         uint4 *p = (uint4 *)(hs.plan_cnt + e);
-        uint4 v = e < kAll ? *p : uint4{0, 0, 0, 0};
+        uint4 v = e < all ? *p : uint4{0, 0, 0, 0};
         const uint32_t sum = v.x + v.y + v.z + v.w;
         const uint32_t incl = wave_incl_scan(sum, lane);
         __syncthreads();
@@ -79,8 +79,8 @@ __device__ __forceinline__ void hub_plan_scan(const HubSet &hs, unsigned long lo
             run += w < wv ? s_wave[w] : 0u;
             before += s_wave[w];
         }
-        if (e < kAll) {
-            if (e % kHubPlanWaves == 0) s_slot[e / kHubPlanWaves] = run;
+        if (e < all) {
+            if (e % hs.plan_waves == 0) s_slot[e / hs.plan_waves] = run;
             const uint4 q{run, run + v.x, run + v.x + v.y, run + v.x + v.y + v.z};
             *p = q;
         }
