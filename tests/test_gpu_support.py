@@ -85,3 +85,14 @@ def test_support_tiled_workgroup_rows(lstc, oracle):
         p = pv.cpu().numpy().view(np.uint64)
         assert s.shape == (n * (n - 1) // 2,) and bool((s == n - 2).all()), split
         assert bool((p == (n - 1) * (n - 2) // 2).all()), split
+
+
+@pytest.mark.parametrize("n", [3, 4, 9, 10, 257, 258, 259, 514])
+def test_support_split_item_edges(lstc, n):
+    """Complete graphs with fewer items than ticket classes, and with longest rows on both sides of a wave's
+    table (256 keys): every edge lies in n - 2 triangles, every vertex in (n - 1)(n - 2) / 2."""
+    _, s, d = G.complete(n)
+    up = lambda a: torch.from_numpy(a.view(np.int32)).cuda()  # noqa: E731
+    g = lstc.clean_orient(n, up(s), up(d), in_lists=True)
+    sup, pv = lstc.triangle_support(g, split=True)
+    assert (sup == n - 2).all() and (pv == (n - 1) * (n - 2) // 2).all()

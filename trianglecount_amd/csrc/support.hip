@@ -31,8 +31,8 @@
 
 namespace lstc {
 
-// A workgroup of WAVES waves (4 for the split rule, 8 for the plain walk: the
-// faster of the two for each at RMAT s23) holds one table of 2^kSupGroupLog2
+// A workgroup of WAVES waves (8 for both rules: at RMAT s21 17.6 ms against 18.7 with
+// 4 for the split rule) holds one table of 2^kSupGroupLog2
 // slots, or one slice of it per wave.
 static constexpr uint32_t kSupGroupLog2 = 12;                             // slots of a workgroup's table
 static constexpr uint32_t kSupGroupTile = (1u << kSupGroupLog2) / 2;      // keys per tile: load <= 1/2
@@ -40,7 +40,7 @@ template <int WAVES>
 constexpr uint32_t sup_wave_log2() { return kSupGroupLog2 - (WAVES == 8 ? 3 : 2); }  // slots of a wave's table
 template <int WAVES>
 constexpr uint32_t sup_wave_tile() { return (1u << sup_wave_log2<WAVES>()) / 2; }
-static constexpr int kSupSplitWaves = 4, kSupPlainWaves = 8;
+static constexpr int kSupSplitWaves = 8, kSupPlainWaves = 8;
 static constexpr int kSupUnroll = 4;                                       // chunks of 64 entries per round
 static constexpr uint32_t kSupEmpty = 0xFFFFFFFFu;     // empty slot; also the end of a lane without a list
 static constexpr uint32_t kSupNoId = 0xFFFFFFFEu;      // past-the-end positions: never a key (ids < 2^32 - 2)
@@ -440,7 +440,19 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 8 : 4) void k_support(cons
 // so a hub's long in-list is spread over waves.  Items of rows with d+ above a
 // wave tile ("group" items) are listed first and run by whole workgroups, then
 // the rest by single waves; both take items from a ticket.
+// (1024: RMAT s23 85 against 92 ms, but RMAT s19 6.0 against 5.7 and Chung-Lu of 300
+// thousand vertices 8.0 against 6.7, which wait for their longest items.)
 static constexpr uint32_t kSupChunk = 512;
+// Items are dealt in kSupHeads classes (item t to class t % kSupHeads), each with
+// its own head per kind on a line of its own; a workgroup starts with class blockIdx %
+// kSupHeads and goes on with the others' leftovers.  Waves take up to kSupMaxGroup
+// items at once while many are left, one at the end.  One head for all and one item a
+// ticket put a million tickets on one address: RMAT s21 23.4 ms (groups of 4 on one
+// head 19.5, of 16 22.5 and of 64 25.9: the long items at their ends), now 18.7, and
+// 17.6 with eight waves per workgroup instead of four, which the one head had kept from
+// paying; RMAT s23 123 -> 92 ms, a uniform graph of 300 thousand vertices 3.4 -> 0.43,
+// a 1000 x 1000 grid 9.3 -> 0.81.
+static constexpr uint32_t kSupHeads = 8, kSupHeadStride = 32, kSupMaxGroup = 8;
 
 // Items per row, group rows and wave rows counted apart.
 __global__ void k_sup_items(const uint64_t *__restrict__ off, const uint64_t *__restrict__ in_off, uint32_t n_rows,
@@ -465,6 +477,11 @@ __global__ void k_sup_item_rows(const uint32_t *__restrict__ items_g, const uint
         for (uint32_t c = 0; c < items_g[r]; ++c) item_row[off_g[r] + c] = (uint32_t)r;
         for (uint32_t c = 0; c < items_w[r]; ++c) item_row[n_g + off_w[r] + c] = (uint32_t)r;
     }
+}
+
+// A ticket head as it is now (it only grows, so an old value costs one atomic at most).
+__device__ __forceinline__ uint32_t sup_head(uint32_t *head) {
+    return __hip_atomic_load(head, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 template <bool NARROW, int NT, uint32_t TILE>
@@ -495,26 +512,44 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 8 : 4) void k_support_spli
     const uint32_t tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const SupWin W = sup_win(L, wv);
     const uint32_t n_g = (uint32_t)off_g[n_rows], n_w = (uint32_t)off_w[n_rows];
-    for (;;) {  // group items (every thread of the workgroup reaches the same break)
-        if (tid == 0) L.ticket = atomicAdd(ticket, 1u);
-        __syncthreads();
-        const uint32_t t = L.ticket;
-        __syncthreads();
-        if (t >= n_g) break;
-        const uint32_t r = item_row[t];
-        sup_split_item<NARROW, WAVES * 64, kSupGroupTile>(sup_group_tab(L), W, off, col, in_off, in_col, n_rows,
-                                                          n_owned, r, t - (uint32_t)off_g[r], support, per_vertex,
-                                                          &L.next, tid);
+    // group items (every thread of the workgroup leaves the loops together)
+    for (uint32_t c = 0; c < kSupHeads && n_g != 0; ++c) {
+        const uint32_t x = (blockIdx.x + c) % kSupHeads;
+        for (;;) {
+            if (tid == 0) {
+                uint32_t *head = ticket + x * kSupHeadStride;
+                L.ticket = c && (uint64_t)sup_head(head) * kSupHeads + x >= n_g ? n_g : atomicAdd(head, 1u);
+            }
+            __syncthreads();
+            const uint64_t t = (uint64_t)L.ticket * kSupHeads + x;
+            __syncthreads();
+            if (t >= n_g) break;
+            const uint32_t r = item_row[t];
+            sup_split_item<NARROW, WAVES * 64, kSupGroupTile>(sup_group_tab(L), W, off, col, in_off, in_col, n_rows,
+                                                              n_owned, r, (uint32_t)t - (uint32_t)off_g[r], support,
+                                                              per_vertex, &L.next, tid);
+        }
     }
     const SupTab Q = sup_wave_tab(L, wv);
-    for (;;) {  // wave items (every wave reaches this break once the items are taken)
-        uint32_t t = 0;
-        if (lane == 0) t = atomicAdd(ticket + 1, 1u);
-        t = read_lane(t, 0);
-        if (t >= n_w) break;
-        const uint32_t r = item_row[n_g + t];
-        sup_split_item<NARROW, 64, sup_wave_tile<WAVES>()>(Q, W, off, col, in_off, in_col, n_rows, n_owned, r,
-                                                           t - (uint32_t)off_w[r], support, per_vertex, nullptr, lane);
+    const uint32_t share = gridDim.x * WAVES / kSupHeads * 4;  // a quarter of what is left per wave of the class
+    for (uint32_t c = 0; c < kSupHeads; ++c) {  // wave items (every wave leaves once the items are taken)
+        const uint32_t x = (blockIdx.x + c) % kSupHeads;
+        const uint32_t n_x = n_w > x ? (n_w - x - 1) / kSupHeads + 1 : 0u;  // the class's items x, x + 8, ...
+        uint32_t *head = ticket + (kSupHeads + x) * kSupHeadStride;
+        for (uint32_t seen = c ? read_lane(sup_head(head), 0) : 0u; seen < n_x;) {
+            const uint32_t g = max(1u, min(kSupMaxGroup, (n_x - seen) / share));
+            uint32_t h = 0;
+            if (lane == 0) h = atomicAdd(head, g);
+            h = read_lane(h, 0);
+            if (h >= n_x) break;
+            for (uint32_t i = h, e = min(h + g, n_x); i < e; ++i) {
+                const uint32_t t = i * kSupHeads + x, r = item_row[n_g + t];
+                sup_split_item<NARROW, 64, sup_wave_tile<WAVES>()>(Q, W, off, col, in_off, in_col, n_rows, n_owned, r,
+                                                                   t - (uint32_t)off_w[r], support, per_vertex, nullptr,
+                                                                   lane);
+            }
+            seen = h + g;
+        }
     }
 }
 
@@ -533,7 +568,7 @@ static SupLayout sup_layout(void *ws, size_t ws_bytes, uint32_t n_rows, uint64_t
     L.off_g = c.take<uint64_t>((size_t)n_rows + 1);
     L.off_w = c.take<uint64_t>((size_t)n_rows + 1);
     L.item_row = c.take<uint32_t>(2 * (size_t)n_rows + m / kSupChunk + 1);
-    L.ticket = c.take<uint32_t>(4);
+    L.ticket = c.take<uint32_t>(2 * kSupHeads * kSupHeadStride);
     L.scan_bytes = scan_ws_bytes((uint64_t)n_rows + 1);
     L.scan_ws = c.take<char>(L.scan_bytes);
     L.bytes = c.need();
@@ -611,7 +646,7 @@ extern "C" lstc_status lstc_triangle_support_split(const uint64_t *d_off, const 
     hipLaunchKernelGGL(k_sup_item_rows, dim3(grid_n), dim3(256), 0, st, L.items_g, L.items_w, L.off_g, L.off_w,
                        n_rows, L.item_row);
     LSTC_LAUNCHED("k_sup_item_rows");
-    LSTC_TRY(fill_u32(L.ticket, 0, 2, st));
+    LSTC_TRY(fill_u32(L.ticket, 0, 2 * kSupHeads * kSupHeadStride, st));
     const uint32_t grid = (uint32_t)device_cus() * 4;  // persistent: four workgroups per CU (LDS)
     if (m < (1ull << 30))  // column positions as 32-bit byte offsets
         hipLaunchKernelGGL((k_support_split<true, kSupSplitWaves>), dim3(grid), dim3(kSupSplitWaves * 64), 0, st, d_off,
