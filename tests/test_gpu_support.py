@@ -3,6 +3,7 @@
 and per vertex, including rows longer than one LDS tile and halo parts (owned rows)."""
 import numpy as np
 import pytest
+import torch
 
 import graphs as G
 
