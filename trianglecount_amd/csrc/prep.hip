@@ -317,6 +317,8 @@ struct OrientInPass {
     uint32_t *flag;
     uint32_t *scol;           // streaming copy (NULL: none): row s from rec[s].off_lo, 128-byte aligned
     const uint64_t *doscan;   // row starts in col (old ids), for an arc's index in its row
+    uint32_t *sym_col;        // symmetric columns (NULL: none): every key's target, whose record is here anyway
+                              // (a pass of its own took 0.33 ms for 47M keys)
 };
 
 __global__ __launch_bounds__(kCT) void k_orient_in_scatter(OrientInPass op, const uint64_t *__restrict__ tile_off) {
@@ -360,6 +362,7 @@ __global__ __launch_bounds__(kCT) void k_orient_in_scatter(OrientInPass op, cons
             if (lane == 0) s_w[r & 1][wv] = (uint32_t)__popcll(km);
             inm[g + r] = ballot(ki);
             if (lane == 0) s_in[(g + r) * (kCT / 64) + wv] = (uint32_t)__popcll(inm[g + r]);
+            if (op.sym_col && valid) op.sym_col[i] = vd[r].nid;
             iv[g + r] = vd[r].nid;
             ilo[g + r] = vd[r].off_lo;
             idp[g + r] = vd[r].dplus;
@@ -446,12 +449,6 @@ __global__ void k_relabel_offsets(const uint32_t *__restrict__ keepv, const uint
         }
     }
     if (blockIdx.x == 0 && threadIdx.x == 0 && sym_off) sym_off[*d_n_out] = *d_m2;
-}
-
-__global__ void k_sym_cols(const uint64_t *__restrict__ uk, const uint64_t *__restrict__ d_m2,
-                           uint64_t mask, const uint32_t *__restrict__ nid, uint32_t *__restrict__ sym_col) {
-    const uint64_t m2 = *d_m2;
-    GRID_STRIDE(i, m2) sym_col[i] = nid[uk[i] & mask];
 }
 
 __global__ void k_orient_offsets(const uint32_t *__restrict__ keepv, const uint64_t *__restrict__ nidscan,
@@ -652,7 +649,6 @@ lstc_status lstc::clean_orient_launch(const uint32_t *d_src, const uint32_t *d_d
     const uint64_t mask = (b >= 64) ? ~0ull : ((1ull << b) - 1);
     const uint64_t nk = 2 * m_raw;
     const uint64_t tiles = (nk + kCTile - 1) / kCTile;
-    const uint32_t grid_k = (uint32_t)hmin<uint64_t>((nk + 255) / 256 + 1, (uint64_t)device_cus() * 32);
     const uint32_t grid_n = (uint32_t)hmin<uint64_t>(((uint64_t)n + 255) / 256 + 1, (uint64_t)device_cus() * 32);
 
     hipLaunchKernelGGL(k_prep_init, dim3(grid_n), dim3(256), 0, st, n, tiles, L.first, L.last, L.dout, L.din, L.tstat,
@@ -685,10 +681,6 @@ lstc_status lstc::clean_orient_launch(const uint32_t *d_src, const uint32_t *d_d
                                L.scal + 1, L.scal + 0, L.nid, d_sym_off);
             LSTC_LAUNCHED("k_relabel_offsets");
         }
-        if (d_sym_col) {
-            hipLaunchKernelGGL(k_sym_cols, dim3(grid_k), dim3(256), 0, st, uk, L.scal + 0, mask, L.nid, d_sym_col);
-            LSTC_LAUNCHED("k_sym_cols");
-        }
         // oriented arcs: count pass (tile counts, d+ per vertex; m -> scal[2]), offsets, per-vertex records
         hipLaunchKernelGGL(k_compact_count<OrientCountOp>, dim3((uint32_t)tiles), dim3(kCT), 0, st,
                            OrientCountOp{uk, L.scal + 0, b, mask, L.deg, L.dout}, L.tile_cnt);
@@ -715,7 +707,7 @@ lstc_status lstc::clean_orient_launch(const uint32_t *d_src, const uint32_t *d_d
         // scatter pass: columns (and segment words); in-lists (entries -> scal[3]) in the same pass
         hipLaunchKernelGGL(k_orient_in_scatter, dim3((uint32_t)tiles), dim3(kCT), 0, st,
                            OrientInPass{uk, L.scal + 0, b, mask, L.rec, d_col, d_col_seg, d_in_col, d_in_seg, L.din,
-                                        L.tstat, L.ticket, L.scal + 3, L.bad, d_scol, L.doscan},
+                                        L.tstat, L.ticket, L.scal + 3, L.bad, d_scol, L.doscan, d_sym_col},
                            (const uint64_t *)L.tile_off);
         LSTC_LAUNCHED("k_orient_in_scatter");
         if (d_in_off && small) {
