@@ -210,7 +210,15 @@ typedef struct lstc_tune {
  * m = d_off[n_rows] is the arc count (the reference kernel's `edge` argument),
  * limited to m < 2^32 - 4096 by the 32-bit work positions inside a row.
  * d_count (1 uint64) is overwritten.  d_per_row (n_owned uint64, may be NULL)
- * receives the reference's per-row partials g_sum[u].                         */
+ * receives the reference's per-row partials g_sum[u].
+ *
+ * The workspace of lstc_count_workspace also holds, for graphs of 2^20 arcs
+ * and 16 arcs per row on, their rows as 16-bit codes of frequent vertices, built
+ * by the call, which the count then reads instead of the ids (lstc_count without
+ * d_per_row from 6 * 2^20 arcs on; lstc_count_split with segment words,
+ * lstc_count_split_stream).  A workspace without room for them is accepted as
+ * long as it holds the engine's queue; the count then reads the ids.  Of the tune
+ * only tiny_max reaches the count from codes.                                  */
 lstc_status lstc_count_workspace(uint32_t n_rows, uint32_t n_owned, uint64_t m,
                                  const lstc_tune *tune, size_t *bytes);
 lstc_status lstc_count(const uint64_t *d_off, const uint32_t *d_col, uint32_t n_rows,
@@ -248,7 +256,8 @@ lstc_status lstc_stream_copy(const uint64_t *d_off, const uint32_t *d_col, uint3
 
 /* lstc_count_split over the outputs of lstc_clean_orient_stream: the lists
  * named by the segment words are read from the streaming copy d_scol
- * (scol_len entries), tables and everything else from d_off / d_col.  Same
+ * (scol_len entries), tables and everything else from d_off / d_col (a count
+ * from codes reads neither copy of the lists while it counts).  Same
  * count, same workspace (lstc_count_workspace).  Replaces the same reference
  * code as lstc_count_split.                                                  */
 lstc_status lstc_count_split_stream(const uint64_t *d_off, const uint32_t *d_col, const uint64_t *d_in_off,
@@ -262,7 +271,7 @@ lstc_status lstc_count_split_stream(const uint64_t *d_off, const uint32_t *d_col
  * harnesses that forbid allocation).  No counterpart in the reference.  The
  * engine's scratch is a static device array of lstc_count_split_static_limit()
  * bytes (32 MiB) per GPU, held until the process ends; a graph whose scratch
- * need (lstc_count_workspace) exceeds it is refused with LSTC_ERR_INVALID.
+ * need (the engine's queue: it reads ids, never codes) exceeds it is refused with LSTC_ERR_INVALID.
  * The call allocates nothing.  Calls that overlap on one GPU share the array
  * and race: keep them on one stream or serialise them.                      */
 size_t lstc_count_split_static_limit(void);
@@ -384,6 +393,8 @@ lstc_status lstc_batch_plan_destroy(lstc_batch_plan *plan);
  *   4 (hashed_keys + streamed) + 8 or 20 per segment + 20 per tiny_segment
  *   + 16 (items + chunk_items) + 32 tiny_rows + 16 (items + tiny_rows)
  *   + 32 or 16 per planned row (two planner passes over the row offsets).
+ * The figures are those of a count that reads ids; one from codes (see
+ * lstc_count_workspace) streams the same lists in about half the bytes.
  * out[G]; workspace from lstc_work_stats_workspace; synchronises the stream. */
 typedef struct lstc_work {
     uint64_t rows;          /* rows the planner visits                              */

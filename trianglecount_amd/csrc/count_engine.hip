@@ -21,20 +21,25 @@
 // instead.  Items of rows above small_max form "big" tickets (kBigGroup items each);
 // smaller ones form "small" tickets of small_group items (by default chosen by
 // the planner from the small items per workgroup).  k_count reads it from ctl.
+// Launches of at most kSmallPlan rows are planned by one workgroup (k_plan_small).
+//
+// One graph large enough for it is counted from 16-bit hub codes instead
+// (hubcode.h, hubplan.h, hubwalk.h; k_count_hub): its plan kernels write that
+// walk's queue.  Batches, and graphs whose hubs the device finds to cover too
+// few of their columns, are counted by k_count.
 //
 // Count (k_count, one persistent launch): each workgroup of WAVES waves (2, 4 or
-// 8: the workgroup size is a tuning knob) takes
-// tickets from an atomic head.
+// 8: the workgroup size is a tuning knob) starts with the ticket of its own number
+// and takes the next from the atomic heads (see kHeads).
 //   big item  : the whole workgroup builds one LDS hash table (up to 1024 slots
 //               per wave: 4096 with 4 waves; load <= 1/2, longer rows are tiled)
 //               and the waves split the 64-segment windows round-robin;
 //   small item: one wave, a private 1024-slot slice of the same LDS.
 // Walk of one window: one segment per lane (id, start, length), inclusive scan
 // of lengths, empty segments compacted out; then the flat sequence of entries
-// is consumed in rounds of UNROLL chunks of 64.  The segment ends inside a
-// round are marked in LDS once, then every chunk finds each lane's segment with
-// one LDS read + ballot + popcount (a chunk inside one segment takes its base
-// from a scalar).  Rounds are software-pipelined: round r+1 is addressed and
+// is consumed in rounds of UNROLL chunks of 64, whose segment ends the wave walks
+// with uniform lane reads (a chunk inside one segment takes its base from a
+// scalar; segwalk.h).  Rounds are software-pipelined: round r+1 is addressed and
 // loaded (global loads, never FLAT) before round r is probed, lockstep over its
 // UNROLL chunks.  Hits are counted per lane and reduced across the wave per
 // item; the workgroup issues one uint64 atomic per graph it counted.
