@@ -280,6 +280,26 @@ def test_count_halo_part_from_hub_codes(lstc, oracle):
     assert total == lstc.count(g)
 
 
+@pytest.mark.parametrize("longest", [(1 << 17) - 1, 1 << 17, (1 << 17) + 60])
+def test_count_hub_codes_longest_rows(lstc, longest):
+    """Rows around the longest that a code record can say, several in every wave of a workgroup of the build, all
+    with tails too long for codes: 52 rows that point at each other and at a path of L vertices."""
+    k, first = 52, 1000
+    L = longest - (k - 1)
+    rows = [np.zeros(0, np.uint32)] * first + [np.array([v + 1], np.uint32) for v in range(first, first + L - 1)]
+    rows.append(np.zeros(0, np.uint32))
+    heads = np.arange(0, 5 * k, 5, dtype=np.uint32)
+    for i, r in enumerate(heads):
+        rows[r] = np.concatenate([heads[i + 1:], np.arange(first, first + L, dtype=np.uint32)])
+    off = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int64)
+    col = torch.from_numpy(np.concatenate(rows).view(np.int32)).cuda()
+    g = lstc.Graph(len(rows), int(off[-1]), torch.from_numpy(off).cuda(), col)
+    want = k * (L - 1) + sum(j * (L + k - 1 - j) for j in range(k))  # head, v, v + 1; two heads and a vertex of both
+    assert [lstc.count(g) for _ in range(2)] == [want, want]
+    lstc.in_lists(g)
+    assert g.in_off is not None and [lstc.count(g) for _ in range(2)] == [want, want]
+
+
 @pytest.mark.parametrize("owned", [None, 100_003, 1])
 def test_count_plain_from_hub_codes(lstc, owned):
     """A bare CSR of RMAT s19 (7.7M arcs), whole and with the first rows owned, against the per-row partials

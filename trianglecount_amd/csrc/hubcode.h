@@ -31,6 +31,13 @@ static constexpr uint32_t kTopMin = 192;         // a row with this many of them
 static constexpr uint32_t kLongRow = 96;         // entries from which a row has a wave of its own in the build
 static constexpr uint32_t kTailPad = 0xFFFFFFFEu;  // fills a tail's last unit; never an id
 static constexpr uint32_t kMaxHubRow = 1u << 17;   // longest row whose lengths fit a record
+// Longest tail.  A streamed id that passes the 2048-bit filter is compared with every
+// id of the row's tail, so the cost per id grows with the tail twice.  Power-law graphs stay
+// far below (RMAT s23 has tails of at most 89, Chung-Lu graphs of 1M to 3M vertices 46); uniform
+// graphs are still faster from codes with tails of 350 (100 thousand vertices, mean degree
+// 1000: 8.1 ms against 9.3 from ids) and 546 (90 thousand, 2000: 28.6 / 31.0); with
+// tails of 65 thousand one list alone takes 0.2 s.
+static constexpr uint32_t kMaxTail = 512;
 
 // Work items.  A row's lists (its own arcs, then its in-list) are one sequence of n;
 // an item is a chunk of it.  A row of kHeavy lists or more is cut into 8 parts, one

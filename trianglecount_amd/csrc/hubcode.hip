@@ -176,8 +176,16 @@ __global__ __launch_bounds__(256) void k_hub_assign(const uint32_t *__restrict__
 __global__ __launch_bounds__(256) void k_hub_short(GraphDev G, HubSet hs) {
     constexpr uint32_t kPer = kLongRow / 16;
     static_assert(kLongRow % 16 == 0, "a short row's entries per lane");
-    __shared__ uint32_t s_n, s_at;
-    if (!sload(hs.hctl + HC_ON)) return;
+    __shared__ uint32_t s_n, s_at, s_on;
+    // one read per workgroup: its waves must agree while another one clears the flag (a
+    // scalar load: as an atomic one from every workgroup 1.10 ms for 0.43 at RMAT s23)
+    const uint32_t on = sload(hs.hctl + HC_ON);
+    if (threadIdx.x == 0) {
+        s_n = 0;
+        s_on = on;
+    }
+    __syncthreads();
+    if (!s_on) return;
     const uint32_t lane = threadIdx.x & 63, sub = lane & 15, grp = lane >> 4;
     const uint64_t r0 = ((uint64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * 64, r = r0 + lane;
     const bool valid = r < G.n_rows;
@@ -185,8 +193,6 @@ __global__ __launch_bounds__(256) void k_hub_short(GraphDev G, HubSet hs) {
     if (e - o >= kMaxHubRow) hs.hctl[HC_ON] = 0;
     const uint32_t d = (uint32_t)min(e - o, (uint64_t)kMaxHubRow);
     const uint32_t start = block_of(r, o);
-    if (threadIdx.x == 0) s_n = 0;
-    __syncthreads();
     const bool lng = d >= kLongRow;
     uint32_t place = 0;
     if (lng) place = atomicAdd(&s_n, 1u);
@@ -243,7 +249,7 @@ __global__ __launch_bounds__(256) void k_hub_short(GraphDev G, HubSet hs) {
 }
 
 // A wave per long row, 512 entries in registers at a time (read twice if there
-// are more).  A wave takes kBatch rows together: their headers (four dependent
+// are more).  A tail of more than kMaxTail ids takes the launch back to k_count.  A wave takes kBatch rows together: their headers (four dependent
 // loads) come in by lane at once.
 __global__ __launch_bounds__(256) void k_hub_long(GraphDev G, HubSet hs) {
     constexpr uint32_t kRegs = 8, kStep = 64 * kRegs, kBatch = 8;
@@ -293,6 +299,7 @@ __global__ __launch_bounds__(256) void k_hub_long(GraphDev G, HubSet hs) {
         const bool bm = top >= kTopMin;
         const uint32_t floor = bm ? kTop : 0u;  // codes below go to the bitmap
         const uint32_t nh = bm ? hub - top : hub, units = (nh + 3) / 4, nt = d - hub;
+        if (nt > kMaxTail && lane == 0) hs.hctl[HC_ON] = 0;  // (this launch's waves read it before their rows)
         // from a 128-byte boundary: with a bitmap there is always room for that, else if there is
         const uint32_t aligned = (start + 15u) & ~15u;
         const bool fits = aligned - start + units + (nt + 1) / 2 <= (d + 1) / 2 + 1;
