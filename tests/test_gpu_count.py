@@ -220,8 +220,8 @@ def _hub_graphs(O):
         "rmat_s17": lambda: O.gen_rmat(17, 16, seed=5),
         "rmat_s16_dense": lambda: O.gen_rmat(16, 40, seed=2),
         "chung_lu": lambda: O.gen_chung_lu(100_000, 2.1, 50, 5e3, seed=3),
-        "er_dense": lambda: O.gen_er(2311, 1200.0, seed=4),
-        "K1501": lambda: G.complete(1501),
+        "er_dense": lambda: O.gen_er(2811, 1200.0, seed=4),
+        "K1901": lambda: G.complete(1901),
         "hub_lists": lambda: _hub_lists(70_001, 300, 30),
         "er_uniform": lambda: O.gen_er(130_001, 40.0, seed=6),
         "er_sparse": lambda: O.gen_er(150_001, 20.0, seed=7),
@@ -237,7 +237,7 @@ def _hub_lists(n, hubs, deg):
     return n, np.concatenate([src, iu.astype(np.uint32)]), np.concatenate([dst, ju.astype(np.uint32)])
 
 
-@pytest.mark.parametrize("name", ["rmat_s17", "rmat_s16_dense", "chung_lu", "er_dense", "K1501", "hub_lists", "er_uniform",
+@pytest.mark.parametrize("name", ["rmat_s17", "rmat_s16_dense", "chung_lu", "er_dense", "K1901", "hub_lists", "er_uniform",
                                   "er_sparse"])
 def test_count_from_hub_codes(lstc, oracle, name):
     n, s, d = _hub_graphs(oracle)[name]()

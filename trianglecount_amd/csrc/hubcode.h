@@ -81,7 +81,9 @@ __device__ __forceinline__ RowRec split_rec(uint64_t r) {
 }
 
 // words of the selection (uint32)
-enum { HC_ON = 0, HC_LONG_ROWS = 1, HC_DONE = 2, HC_CUT = 3, HC_REST = 4, HC_HIST = 64, HC_SUM = HC_HIST + 256,
+enum { HC_ON = 0, HC_LONG_ROWS = 1, HC_DONE = 2, HC_CUT = 3, HC_REST = 4,
+       HC_LEN = 8, HC_LENS = 10, HC_SQ = 12,  // 64-bit sums
+       HC_HIST = 64, HC_SUM = HC_HIST + 256,
        HC_BASE = HC_SUM + 256, HC_USED = HC_BASE + 256,
        // the plan: first item and tickets of each XCD's own region; the light and the tiny rows
        HC_OWN0 = HC_USED + 256, HC_OWN_T = HC_OWN0 + 8, HC_OWN_END = HC_OWN_T + 8, HC_LIGHT0 = HC_OWN_END + 8,

@@ -5,8 +5,7 @@
 //   k_hub_init   : clears the selection words and the occurrences
 //   k_hub_sample : occurrences of each vertex in every stride-th 64-entry chunk of the columns
 //   k_hub_pick   : vertices and occurrences per occurrence bin (8 bins per octave); the bins
-//                  whose vertices become hubs, their first codes, and whether the hubs cover
-//                  enough of the sample for codes to pay
+//                  whose vertices become hubs, their first codes, and whether codes pay
 //   k_hub_assign : every vertex's code
 //   k_hub_short  : the blocks of rows below kLongRow entries, 16 lanes per row
 //   k_hub_long   : the others, a wave per row
@@ -18,17 +17,23 @@ namespace lstc {
 // Sampled entries (RMAT s23, ms a count: 11.1 with 2^20, 10.7 with 2^21, 10.8 with
 // 2^22), and at most one in 16: the hubs' counters are hot addresses.
 static constexpr uint64_t kSamples = 2u << 20, kMinStride = 16;
-// The hubs have to cover half of the sample.  Calls from codes against ids: RMAT s21
-// 2.21 / 3.24 ms, Chung-Lu of 1M vertices (gamma 2.1, mean degree 50) 1.87 / 2.10; a
-// uniform graph of 1M vertices and mean degree 40, whose hubs cover a twentieth,
-// 1.66 / 1.01.
+// Codes pay where much is streamed per arc and hubs are most of it.  With in-lists
+// an arc streams at most the smaller of the mean d+ of its two ends' rows, E (each a mean over
+// arcs); with the share c of the sample that the hubs cover, codes are taken
+// from E (2 c - 1) = 72 on.  Calls from codes against ids, ms: 90 at RMAT s17 0.28 / 0.35, 109 at s18
+// 0.40 / 0.43, 166 at s21 2.28 / 3.22, 173 at s23 10.4 / 17.1; 106 on a uniform graph of 100
+// thousand vertices and mean degree 400 1.50 / 1.76; below: 66 (20 thousand, 200)
+// 0.20 / 0.18, 60 (130 thousand, 300) 1.70 / 1.42, Chung-Lu graphs of 1M vertices and mean degree 50 62
+// (gamma 2.1) 1.84 / 1.70 and 23 (2.3) 1.97 / 1.47, of 3M 52 (2.1) 5.38 / 5.81 and 10 (2.3) 5.65 / 4.43.
+// Without in-lists an arc streams its target's row: codes from a mean of 128 on (RMAT s21 357:
+// 2.6 / 5.4, Chung-Lu of 3M, gamma 2.3, 138: 5.3 / 6.0; of 1M 111: 1.79 / 1.61; the uniform
+// graphs 133: 1.51 / 1.78 and 100: 1.73 / 1.47).  Either way half of the sample is covered.
+static constexpr double kMinWorth = 72, kMinPlainLen = 128;
 static constexpr uint32_t kCoverPct = 50;
-// Smaller graphs and shorter rows keep ids: the build is worth 0.1 ms (RMAT s17,
-// 1.9M arcs: 0.30 against 0.39 ms; a uniform graph of 3M vertices and 15 arcs a row,
-// found out by its sample, 2.36 against 2.24).  Without in-lists k_count has less to
-// lose to (Chung-Lu of 4.4M arcs 0.464 from codes, 0.441 from ids; of 6.8M arcs 0.620 /
-// 0.616; RMAT s19, 7.7M arcs, 0.65 / 0.92; s21 2.57 / 5.42).
-static constexpr uint64_t kMinArcs = 1ull << 20, kMinArcsPlain = 6ull << 20, kMinPerRow = 16;
+// Smaller graphs and shorter rows keep ids: the build is worth 0.1 ms (uniform graphs of
+// 1.2M arcs, E 82 to 158, 0.19 / 0.14 and 0.26 / 0.20).  Without in-lists k_count has less to lose to
+// (Chung-Lu of 4.4M arcs 0.464 / 0.441; RMAT s19, 7.7M arcs, 0.65 / 0.92).
+static constexpr uint64_t kMinArcs = 3ull << 19, kMinArcsPlain = 6ull << 20, kMinPerRow = 16;
 static constexpr uint32_t kAbsent = 0xFFFFFFFFu;  // past the end of a row (ids are below 2^32 - 2)
 
 __device__ __forceinline__ uint32_t occ_bin(uint32_t c) {
@@ -52,9 +57,15 @@ __global__ __launch_bounds__(256) void k_hub_init(HubSet hs, uint32_t n) {
     for (uint64_t v = (uint64_t)blockIdx.x * 256 + threadIdx.x; v < n; v += (uint64_t)gridDim.x * 256) hs.cnt[v] = 0;
 }
 
-// A wave takes four chunks at a time.
-__global__ __launch_bounds__(256) void k_hub_sample(GraphDev G, uint64_t m, uint32_t stride, uint32_t *__restrict__ cnt) {
+// A wave takes four chunks at a time; the rows of the first one's entries are measured
+// (HC_LEN: their lengths' sum, HC_LENS: how many).
+__global__ __launch_bounds__(256) void k_hub_sample(GraphDev G, uint64_t m, uint32_t stride, uint32_t *__restrict__ cnt,
+                                                    uint32_t *__restrict__ hctl) {
     constexpr uint32_t kPer = 4;
+    __shared__ unsigned long long s_len, s_lens;
+    if (threadIdx.x == 0) s_len = s_lens = 0;
+    __syncthreads();
+    unsigned long long len = 0, lens = 0;
     const uint32_t lane = threadIdx.x & 63;
     const uint64_t waves = (uint64_t)gridDim.x * 4, wave = (uint64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     for (uint64_t c0 = wave; c0 * 64 * stride < m; c0 += waves * kPer) {
@@ -68,26 +79,52 @@ __global__ __launch_bounds__(256) void k_hub_sample(GraphDev G, uint64_t m, uint
 #pragma unroll
         for (uint32_t q = 0; q < kPer; ++q)
             if (x[q] < G.n_rows) atomicAdd(cnt + x[q], 1u);
+        if (x[0] < G.n_rows) {
+            len += gload(G.off + x[0] + 1) - gload(G.off + x[0]);
+            ++lens;
+        }
+    }
+    if (lens) {
+        atomicAdd(&s_len, len);
+        atomicAdd(&s_lens, lens);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0 && s_lens) {
+        atomicAdd((unsigned long long *)(hctl + HC_LEN), s_len);
+        atomicAdd((unsigned long long *)(hctl + HC_LENS), s_lens);
     }
 }
 
 // Every workgroup adds its share to the bins; the last one to do so picks.  Bins
 // above HC_CUT are hubs; of bin HC_CUT the first HC_REST vertices that ask.
-__global__ __launch_bounds__(256) void k_hub_pick(const uint32_t *__restrict__ cnt, uint32_t n,
-                                                  uint32_t *__restrict__ hctl) {
+__global__ __launch_bounds__(256) void k_hub_pick(const uint32_t *__restrict__ cnt, const uint64_t *__restrict__ off,
+                                                  uint32_t n, uint64_t m, bool split, uint32_t *__restrict__ hctl) {
+    __shared__ unsigned long long s_sq;  // squares of the rows' lengths
     __shared__ uint32_t s_n[257], s_add[256];
     __shared__ unsigned long long s_sum[257];
     __shared__ uint32_t s_last;
     const uint32_t b = threadIdx.x;
     s_n[b] = 0;
     s_add[b] = 0;
+    if (b == 0) s_sq = 0;
     __syncthreads();
     constexpr uint32_t kPer = 8;
+    unsigned long long sq = 0;
     const uint64_t step = (uint64_t)gridDim.x * 256;
     for (uint64_t v = (uint64_t)blockIdx.x * 256 + b; v < n; v += step * kPer) {
         uint32_t c[kPer];
 #pragma unroll
         for (uint32_t q = 0; q < kPer; ++q) c[q] = v + q * step < n ? cnt[v + q * step] : 0u;
+        if (split) {
+            uint64_t d[kPer];
+#pragma unroll
+            for (uint32_t q = 0; q < kPer; ++q) {
+                const uint64_t w = v + q * step;
+                d[q] = w < n ? gload(off + w + 1) - gload(off + w) : 0;
+            }
+#pragma unroll
+            for (uint32_t q = 0; q < kPer; ++q) sq += d[q] * d[q];
+        }
 #pragma unroll
         for (uint32_t q = 0; q < kPer; ++q) {
             if (c[q] == 0) continue;
@@ -95,7 +132,9 @@ __global__ __launch_bounds__(256) void k_hub_pick(const uint32_t *__restrict__ c
             atomicAdd(&s_add[occ_bin(c[q])], c[q]);
         }
     }
+    if (sq) atomicAdd(&s_sq, sq);
     __syncthreads();
+    if (b == 0 && s_sq) atomicAdd((unsigned long long *)(hctl + HC_SQ), s_sq);
     if (s_n[b]) {
         atomicAdd(hctl + HC_HIST + b, s_n[b]);
         atomicAdd(hctl + HC_SUM + b, s_add[b]);
@@ -133,7 +172,14 @@ __global__ __launch_bounds__(256) void k_hub_pick(const uint32_t *__restrict__ c
     } else if (b != 0) {
         return;
     }
-    hctl[HC_ON] = all && covered * 100 >= all * kCoverPct ? 1u : 0u;
+    auto read64 = [&](uint32_t w) {
+        return (double)__hip_atomic_load((unsigned long long *)(hctl + w), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    if (all == 0 || covered * 100 < all * kCoverPct) return;  // (off)
+    const double to = read64(HC_LEN) / read64(HC_LENS), from = read64(HC_SQ) / (double)m;
+    const double share = (double)covered / (double)all;
+    const bool on = split ? fmin(from, to) * (2 * share - 1) >= kMinWorth : to >= kMinPlainLen;
+    hctl[HC_ON] = on ? 1u : 0u;
 }
 
 // A workgroup takes 4096 vertices at a time and one place per bin among all of them.
@@ -355,9 +401,10 @@ lstc_status hub_build(const GraphDev &g, uint64_t m, const HubSet &hs, hipStream
     const uint32_t flat = hmin(blocks, cus * 4);
     hipLaunchKernelGGL(k_hub_init, dim3(flat), dim3(256), 0, st, hs, n);
     LSTC_LAUNCHED("k_hub_init");
-    hipLaunchKernelGGL(k_hub_sample, dim3(cus * 8), dim3(256), 0, st, g, m, stride, hs.cnt);
+    hipLaunchKernelGGL(k_hub_sample, dim3(cus * 8), dim3(256), 0, st, g, m, stride, hs.cnt, hs.hctl);
     LSTC_LAUNCHED("k_hub_sample");
-    hipLaunchKernelGGL(k_hub_pick, dim3(hmin(blocks, cus)), dim3(256), 0, st, (const uint32_t *)hs.cnt, n, hs.hctl);
+    hipLaunchKernelGGL(k_hub_pick, dim3(hmin(blocks, cus)), dim3(256), 0, st, (const uint32_t *)hs.cnt, g.off, n, m,
+                       g.in_off != nullptr, hs.hctl);
     LSTC_LAUNCHED("k_hub_pick");
     hipLaunchKernelGGL(k_hub_assign, dim3(hmin(ceil_div_u32(n, 4096), cus * 8)), dim3(256), 0, st,
                        (const uint32_t *)hs.cnt, n, hs.hctl, hs.code);
