@@ -212,10 +212,10 @@ typedef struct lstc_tune {
  * d_count (1 uint64) is overwritten.  d_per_row (n_owned uint64, may be NULL)
  * receives the reference's per-row partials g_sum[u].
  *
- * The workspace of lstc_count_workspace also holds, for graphs of 2^20 arcs
+ * The workspace of lstc_count_workspace also holds, for graphs of 1.5 * 2^20 arcs
  * and 16 arcs per row on, their rows as 16-bit codes of frequent vertices, built
- * by the call, which the count then reads instead of the ids (lstc_count without
- * d_per_row from 6 * 2^20 arcs on; lstc_count_split with segment words,
+ * by the call, which the count then reads instead of the ids if the call finds that
+ * this pays (lstc_count without d_per_row from 6 * 2^20 arcs on; lstc_count_split with segment words,
  * lstc_count_split_stream).  A workspace without room for them is accepted as
  * long as it holds the engine's queue; the count then reads the ids.  Of the tune
  * only tiny_max reaches the count from codes.                                  */

@@ -20,15 +20,16 @@ static constexpr uint64_t kSamples = 2u << 20, kMinStride = 16;
 // Codes pay where much is streamed per arc and hubs are most of it.  With in-lists
 // an arc streams at most the smaller of the mean d+ of its two ends' rows, E (each a mean over
 // arcs); with the share c of the sample that the hubs cover, codes are taken
-// from E (2 c - 1) = 72 on.  Calls from codes against ids, ms: 90 at RMAT s17 0.28 / 0.35, 109 at s18
-// 0.40 / 0.43, 166 at s21 2.28 / 3.22, 173 at s23 10.4 / 17.1; 106 on a uniform graph of 100
-// thousand vertices and mean degree 400 1.50 / 1.76; below: 66 (20 thousand, 200)
-// 0.20 / 0.18, 60 (130 thousand, 300) 1.70 / 1.42, Chung-Lu graphs of 1M vertices and mean degree 50 62
-// (gamma 2.1) 1.84 / 1.70 and 23 (2.3) 1.97 / 1.47, of 3M 52 (2.1) 5.38 / 5.81 and 10 (2.3) 5.65 / 4.43.
+// from E (2 c - 1) = 61 on.  Calls from codes against ids, ms: 90 at RMAT s17 0.28 / 0.35, 109 at s18
+// 0.40 / 0.43, 166 at s21 2.2 / 3.2, 173 at s23 10.4 / 17.1; 106 on a uniform graph of 100
+// thousand vertices and mean degree 400 1.50 / 1.76, 66 on one of 20 thousand and 200 0.20 / 0.18
+// (0.22 if it is found out after the sample); Chung-Lu graphs, gamma 2.1, of 1M vertices and mean
+// degree 50, 62.5, 1.84 / 1.70 (2.02 after the sample).  Below: 60 (uniform, 130 thousand, 300)
+// 1.70 / 1.42, Chung-Lu of 3M 52 5.4 / 5.8; gamma 2.3, 1M, 23 1.97 / 1.47, 3M, 10 5.65 / 4.43.
 // Without in-lists an arc streams its target's row: codes from a mean of 128 on (RMAT s21 357:
 // 2.6 / 5.4, Chung-Lu of 3M, gamma 2.3, 138: 5.3 / 6.0; of 1M 111: 1.79 / 1.61; the uniform
 // graphs 133: 1.51 / 1.78 and 100: 1.73 / 1.47).  Either way half of the sample is covered.
-static constexpr double kMinWorth = 72, kMinPlainLen = 128;
+static constexpr double kMinWorth = 61, kMinPlainLen = 128;
 static constexpr uint32_t kCoverPct = 50;
 // Smaller graphs and shorter rows keep ids: the build is worth 0.1 ms (uniform graphs of
 // 1.2M arcs, E 82 to 158, 0.19 / 0.14 and 0.26 / 0.20).  Without in-lists k_count has less to lose to
@@ -51,21 +52,48 @@ __device__ __forceinline__ uint32_t code_of(const uint16_t *code, uint32_t n, ui
 // First unit of the block of row r, whose columns start at o.
 __device__ __forceinline__ uint32_t block_of(uint64_t r, uint64_t o) { return (uint32_t)((o >> 1) + 2 * r); }
 
-__global__ __launch_bounds__(256) void k_hub_init(HubSet hs, uint32_t n) {
+// Also the sum of the squares of the rows' lengths, one share per workgroup (at most
+// kInitBlocks of them, in the plan's counters, which are free until the plan).
+static constexpr uint32_t kInitBlocks = 1024;
+static_assert(kInitBlocks * 2 <= kHubSlots * kHubPlanWaves, "the shares' place");
+__global__ __launch_bounds__(256) void k_hub_init(HubSet hs, const uint64_t *__restrict__ off, uint32_t n) {
+    __shared__ unsigned long long s_sq;
+    if (threadIdx.x == 0) s_sq = 0;
+    __syncthreads();
     if (blockIdx.x == 0)
         for (uint32_t i = threadIdx.x; i < HC_WORDS; i += 256) hs.hctl[i] = 0;
-    for (uint64_t v = (uint64_t)blockIdx.x * 256 + threadIdx.x; v < n; v += (uint64_t)gridDim.x * 256) hs.cnt[v] = 0;
+    unsigned long long sq = 0;
+    for (uint64_t v = (uint64_t)blockIdx.x * 256 + threadIdx.x; v < n; v += (uint64_t)gridDim.x * 256) {
+        hs.cnt[v] = 0;
+        const uint64_t d = gload(off + v + 1) - gload(off + v);
+        sq += d * d;
+    }
+    if (sq) atomicAdd(&s_sq, sq);
+    __syncthreads();
+    if (threadIdx.x == 0) ((unsigned long long *)hs.plan_cnt)[blockIdx.x] = s_sq;
 }
 
-// A wave takes four chunks at a time; the rows of the first one's entries are measured
-// (HC_LEN: their lengths' sum, HC_LENS: how many).
-__global__ __launch_bounds__(256) void k_hub_sample(GraphDev G, uint64_t m, uint32_t stride, uint32_t *__restrict__ cnt,
-                                                    uint32_t *__restrict__ hctl) {
+// A wave takes four chunks at a time; every fourth wave measures the rows of the first
+// one's entries (HC_LEN: the sum of their lengths, HC_LENS: how many).  With in-lists it
+// leaves at once if the rows are too short for codes (see kMinWorth): the Chung-Lu graph of
+// 3M vertices and gamma 2.3 takes 4.48 ms then, 4.77 when the rule waits for the sample, 4.43 from ids.
+__global__ __launch_bounds__(256) void k_hub_sample(GraphDev G, uint64_t m, uint32_t stride, HubSet hs,
+                                                    uint32_t shares, bool split) {
     constexpr uint32_t kPer = 4;
-    __shared__ unsigned long long s_len, s_lens;
-    if (threadIdx.x == 0) s_len = s_lens = 0;
-    __syncthreads();
-    unsigned long long len = 0, lens = 0;
+    uint32_t *cnt = hs.cnt, *hctl = hs.hctl;
+    if (split) {
+        __shared__ unsigned long long s_sq;
+        if (threadIdx.x == 0) s_sq = 0;
+        __syncthreads();
+        unsigned long long sq = 0;
+        for (uint32_t i = threadIdx.x; i < shares; i += 256) sq += ((const unsigned long long *)hs.plan_cnt)[i];
+        if (sq) atomicAdd(&s_sq, sq);
+        __syncthreads();
+        const unsigned long long all = s_sq;
+        if (blockIdx.x == 0 && threadIdx.x == 0) *(unsigned long long *)(hctl + HC_SQ) = all;
+        if ((double)all < kMinWorth * (double)m) return;
+    }
+    uint32_t len = 0, lens = 0;
     const uint32_t lane = threadIdx.x & 63;
     const uint64_t waves = (uint64_t)gridDim.x * 4, wave = (uint64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     for (uint64_t c0 = wave; c0 * 64 * stride < m; c0 += waves * kPer) {
@@ -79,52 +107,39 @@ __global__ __launch_bounds__(256) void k_hub_sample(GraphDev G, uint64_t m, uint
 #pragma unroll
         for (uint32_t q = 0; q < kPer; ++q)
             if (x[q] < G.n_rows) atomicAdd(cnt + x[q], 1u);
-        if (x[0] < G.n_rows) {
-            len += gload(G.off + x[0] + 1) - gload(G.off + x[0]);
+        if (c0 % 4 == 0 && x[0] < G.n_rows) {
+            len += (uint32_t)min(gload(G.off + x[0] + 1) - gload(G.off + x[0]), (uint64_t)kMaxHubRow);
             ++lens;
         }
     }
-    if (lens) {
-        atomicAdd(&s_len, len);
-        atomicAdd(&s_lens, lens);
-    }
-    __syncthreads();
-    if (threadIdx.x == 0 && s_lens) {
-        atomicAdd((unsigned long long *)(hctl + HC_LEN), s_len);
-        atomicAdd((unsigned long long *)(hctl + HC_LENS), s_lens);
+    if (ballot(lens != 0) == 0) return;
+    // (a wave has at most a few dozen chunks of 64 lengths of at most 2^17: 32 bits hold the sum)
+    len = wave_sum32(len);
+    lens = wave_sum32(lens);
+    if (lane == 0) {
+        atomicAdd((unsigned long long *)(hctl + HC_LEN), (unsigned long long)len);
+        atomicAdd((unsigned long long *)(hctl + HC_LENS), (unsigned long long)lens);
     }
 }
 
 // Every workgroup adds its share to the bins; the last one to do so picks.  Bins
 // above HC_CUT are hubs; of bin HC_CUT the first HC_REST vertices that ask.
-__global__ __launch_bounds__(256) void k_hub_pick(const uint32_t *__restrict__ cnt, const uint64_t *__restrict__ off,
-                                                  uint32_t n, uint64_t m, bool split, uint32_t *__restrict__ hctl) {
-    __shared__ unsigned long long s_sq;  // squares of the rows' lengths
+__global__ __launch_bounds__(256) void k_hub_pick(const uint32_t *__restrict__ cnt, uint32_t n, uint64_t m,
+                                                  bool split, uint32_t *__restrict__ hctl) {
+    if (!sload(hctl + HC_LENS)) return;  // nothing was sampled
     __shared__ uint32_t s_n[257], s_add[256];
     __shared__ unsigned long long s_sum[257];
     __shared__ uint32_t s_last;
     const uint32_t b = threadIdx.x;
     s_n[b] = 0;
     s_add[b] = 0;
-    if (b == 0) s_sq = 0;
     __syncthreads();
     constexpr uint32_t kPer = 8;
-    unsigned long long sq = 0;
     const uint64_t step = (uint64_t)gridDim.x * 256;
     for (uint64_t v = (uint64_t)blockIdx.x * 256 + b; v < n; v += step * kPer) {
         uint32_t c[kPer];
 #pragma unroll
         for (uint32_t q = 0; q < kPer; ++q) c[q] = v + q * step < n ? cnt[v + q * step] : 0u;
-        if (split) {
-            uint64_t d[kPer];
-#pragma unroll
-            for (uint32_t q = 0; q < kPer; ++q) {
-                const uint64_t w = v + q * step;
-                d[q] = w < n ? gload(off + w + 1) - gload(off + w) : 0;
-            }
-#pragma unroll
-            for (uint32_t q = 0; q < kPer; ++q) sq += d[q] * d[q];
-        }
 #pragma unroll
         for (uint32_t q = 0; q < kPer; ++q) {
             if (c[q] == 0) continue;
@@ -132,9 +147,7 @@ __global__ __launch_bounds__(256) void k_hub_pick(const uint32_t *__restrict__ c
             atomicAdd(&s_add[occ_bin(c[q])], c[q]);
         }
     }
-    if (sq) atomicAdd(&s_sq, sq);
     __syncthreads();
-    if (b == 0 && s_sq) atomicAdd((unsigned long long *)(hctl + HC_SQ), s_sq);
     if (s_n[b]) {
         atomicAdd(hctl + HC_HIST + b, s_n[b]);
         atomicAdd(hctl + HC_SUM + b, s_add[b]);
@@ -398,12 +411,13 @@ lstc_status hub_build(const GraphDev &g, uint64_t m, const HubSet &hs, hipStream
     const uint32_t n = g.n_rows, cus = (uint32_t)device_cus();
     const uint32_t stride = (uint32_t)hmax<uint64_t>(kMinStride, m / kSamples);
     const uint32_t blocks = ceil_div_u32(n, 256);  // a wave per 64 rows
-    const uint32_t flat = hmin(blocks, cus * 4);
-    hipLaunchKernelGGL(k_hub_init, dim3(flat), dim3(256), 0, st, hs, n);
+    const uint32_t flat = hmin(hmin(blocks, cus * 4), kInitBlocks);
+    hipLaunchKernelGGL(k_hub_init, dim3(flat), dim3(256), 0, st, hs, g.off, n);
     LSTC_LAUNCHED("k_hub_init");
-    hipLaunchKernelGGL(k_hub_sample, dim3(cus * 8), dim3(256), 0, st, g, m, stride, hs.cnt, hs.hctl);
+    hipLaunchKernelGGL(k_hub_sample, dim3(cus * 8), dim3(256), 0, st, g, m, stride, hs, flat,
+                       g.in_off != nullptr);
     LSTC_LAUNCHED("k_hub_sample");
-    hipLaunchKernelGGL(k_hub_pick, dim3(hmin(blocks, cus)), dim3(256), 0, st, (const uint32_t *)hs.cnt, g.off, n, m,
+    hipLaunchKernelGGL(k_hub_pick, dim3(hmin(blocks, cus)), dim3(256), 0, st, (const uint32_t *)hs.cnt, n, m,
                        g.in_off != nullptr, hs.hctl);
     LSTC_LAUNCHED("k_hub_pick");
     hipLaunchKernelGGL(k_hub_assign, dim3(hmin(ceil_div_u32(n, 4096), cus * 8)), dim3(256), 0, st,
