@@ -20,16 +20,17 @@ static constexpr uint64_t kSamples = 2u << 20, kMinStride = 16;
 // Codes pay where much is streamed per arc and hubs are most of it.  With in-lists
 // an arc streams at most the smaller of the mean d+ of its two ends' rows, E (each a mean over
 // arcs); with the share c of the sample that the hubs cover, codes are taken
-// from E (2 c - 1) = 61 on.  Calls from codes against ids, ms: 90 at RMAT s17 0.28 / 0.35, 109 at s18
+// from E (2 c - 1) = 40 on, from 61 if the rows that arcs point at are the shorter ones (uniform graphs).  Calls from codes against ids, ms: 90 at RMAT s17 0.28 / 0.35, 109 at s18
 // 0.40 / 0.43, 166 at s21 2.2 / 3.2, 173 at s23 10.4 / 17.1; 106 on a uniform graph of 100
 // thousand vertices and mean degree 400 1.50 / 1.76, 66 on one of 20 thousand and 200 0.20 / 0.18
 // (0.22 if it is found out after the sample); Chung-Lu graphs, gamma 2.1, of 1M vertices and mean
-// degree 50, 62.5, 1.84 / 1.70 (2.02 after the sample).  Below: 60 (uniform, 130 thousand, 300)
-// 1.70 / 1.42, Chung-Lu of 3M 52 5.4 / 5.8; gamma 2.3, 1M, 23 1.97 / 1.47, 3M, 10 5.65 / 4.43.
+// degree 50, 62.5, 1.84 / 1.70 (2.02 after the sample), of 3M 52 5.4 / 5.8.  Below: 60 (uniform, 130
+// thousand, 300) 1.70 / 1.42; Chung-Lu, gamma 2.3, 1M, 23 1.97 / 1.47, 3M, 10 5.65 / 4.43.
+// Rows shorter than kMinRows (without in-lists kMinRowsPlain) in the mean over arcs are not sampled.
 // Without in-lists an arc streams its target's row: codes from a mean of 128 on (RMAT s21 357:
 // 2.6 / 5.4, Chung-Lu of 3M, gamma 2.3, 138: 5.3 / 6.0; of 1M 111: 1.79 / 1.61; the uniform
 // graphs 133: 1.51 / 1.78 and 100: 1.73 / 1.47).  Either way half of the sample is covered.
-static constexpr double kMinWorth = 61, kMinPlainLen = 128;
+static constexpr double kMinWorth = 40, kMinWorthFlat = 61, kMinRows = 48, kMinPlainLen = 128, kMinRowsPlain = 42;
 static constexpr uint32_t kCoverPct = 50;
 // Smaller graphs and shorter rows keep ids: the build is worth 0.1 ms (uniform graphs of
 // 1.2M arcs, E 82 to 158, 0.19 / 0.14 and 0.26 / 0.20).  Without in-lists k_count has less to lose to
@@ -74,14 +75,14 @@ __global__ __launch_bounds__(256) void k_hub_init(HubSet hs, const uint64_t *__r
 }
 
 // A wave takes four chunks at a time; every fourth wave measures the rows of the first
-// one's entries (HC_LEN: the sum of their lengths, HC_LENS: how many).  With in-lists it
-// leaves at once if the rows are too short for codes (see kMinWorth): the Chung-Lu graph of
+// one's entries (HC_LEN: the sum of their lengths, HC_LENS: how many).  It leaves
+// at once if the rows are too short for codes (see kMinRows): the Chung-Lu graph of
 // 3M vertices and gamma 2.3 takes 4.48 ms then, 4.77 when the rule waits for the sample, 4.43 from ids.
 __global__ __launch_bounds__(256) void k_hub_sample(GraphDev G, uint64_t m, uint32_t stride, HubSet hs,
                                                     uint32_t shares, bool split) {
     constexpr uint32_t kPer = 4;
     uint32_t *cnt = hs.cnt, *hctl = hs.hctl;
-    if (split) {
+    {
         __shared__ unsigned long long s_sq;
         if (threadIdx.x == 0) s_sq = 0;
         __syncthreads();
@@ -91,7 +92,7 @@ __global__ __launch_bounds__(256) void k_hub_sample(GraphDev G, uint64_t m, uint
         __syncthreads();
         const unsigned long long all = s_sq;
         if (blockIdx.x == 0 && threadIdx.x == 0) *(unsigned long long *)(hctl + HC_SQ) = all;
-        if ((double)all < kMinWorth * (double)m) return;
+        if ((double)all < (split ? kMinRows : kMinRowsPlain) * (double)m) return;
     }
     uint32_t len = 0, lens = 0;
     const uint32_t lane = threadIdx.x & 63;
@@ -191,7 +192,7 @@ __global__ __launch_bounds__(256) void k_hub_pick(const uint32_t *__restrict__ c
     if (all == 0 || covered * 100 < all * kCoverPct) return;  // (off)
     const double to = read64(HC_LEN) / read64(HC_LENS), from = read64(HC_SQ) / (double)m;
     const double share = (double)covered / (double)all;
-    const bool on = split ? fmin(from, to) * (2 * share - 1) >= kMinWorth : to >= kMinPlainLen;
+    const bool on = split ? fmin(from, to) * (2 * share - 1) >= (to < from ? kMinWorthFlat : kMinWorth) : to >= kMinPlainLen;
     hctl[HC_ON] = on ? 1u : 0u;
 }
 
