@@ -60,6 +60,25 @@ def test_workspace_queries_are_host_only():
     assert lib.lstc_count_workspace(1, 1, 0, None, None) == _lib.LSTC_ERR_INVALID
 
 
+def _desc(n, m, split=True):
+    lists = dict(in_off=0x10000, in_col=0x10000, col_seg=0x10000, in_seg=0x10000) if split else {}
+    return _lib.GraphDesc(off=0x10000, col=0x10000, m=m, n_rows=n, n_owned=n, **lists)
+
+
+@pytest.mark.parametrize("graphs", [2, 7])
+def test_batch_workspace_holds_no_code_arrays(graphs):
+    """A launch over several graphs reads ids: its workspace is the queue (two entries a row, one per 512 arcs)
+    and fixed-size control words, with no room for 16-bit codes (4 bytes an arc).  One graph has that room."""
+    lib = _lib.load()
+    n, m = 1 << 20, 32 << 20
+    nb, one = ctypes.c_size_t(), ctypes.c_size_t()
+    arr = (_lib.GraphDesc * graphs)(*[_desc(n, m) for _ in range(graphs)])
+    assert lib.lstc_count_batch_workspace(arr, graphs, None, ctypes.byref(nb)) == 0
+    assert nb.value < graphs * (16 * n + m // 64) + (1 << 20)
+    assert lib.lstc_count_batch_workspace((_lib.GraphDesc * 1)(_desc(n, m)), 1, None, ctypes.byref(one)) == 0
+    assert one.value > 4 * m
+
+
 # Shape validation happens on the host before any HIP call, so these run without
 # a device.  The pointers are placeholders that are never dereferenced.
 _FAKE = ctypes.c_void_p(0x10000)

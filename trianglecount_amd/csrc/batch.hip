@@ -52,6 +52,11 @@ static uint64_t arcs_total(const lstc_graph_desc *graphs, uint32_t G) {
     return t;
 }
 
+// The engine's workspace: only a launch over one graph can count from codes.
+static size_t engine_bytes(uint32_t G, uint64_t rows, uint64_t m) {
+    return G == 1 ? count_ws_bytes(rows, m) : count_ws_base(rows, m);
+}
+
 static size_t table_bytes(uint32_t G) {
     Carver c(nullptr, 0);
     c.take<GraphDev>(G ? G : 1);
@@ -85,7 +90,7 @@ extern "C" lstc_status lstc_count_batch_workspace(const lstc_graph_desc *graphs,
     (void)tune;
     if (!bytes) return fail(LSTC_ERR_INVALID, "lstc_count_batch_workspace: NULL bytes");
     if (G && !graphs) return fail(LSTC_ERR_INVALID, "lstc_count_batch_workspace: NULL graph array");
-    *bytes = table_bytes(G) + count_ws_bytes(planned_total(graphs, G), arcs_total(graphs, G));
+    *bytes = table_bytes(G) + engine_bytes(G, planned_total(graphs, G), arcs_total(graphs, G));
     return LSTC_OK;
 }
 
@@ -130,7 +135,7 @@ extern "C" lstc_status lstc_batch_plan_create(const lstc_graph_desc *graphs, uin
     p->G = G;
     if (tune) { p->tune = *tune; p->has_tune = true; }
     const size_t tb = table_bytes(G);
-    p->ws_bytes = count_ws_bytes(base[G], arcs_total(graphs, G));
+    p->ws_bytes = engine_bytes(G, base[G], arcs_total(graphs, G));
     p->dbytes = tb + p->ws_bytes;
     hipError_t e = hipMalloc(&p->dmem, p->dbytes);
     if (e != hipSuccess) { delete p; return fail(LSTC_ERR_OOM, "lstc_batch_plan_create: hipMalloc(%zu) failed", p->dbytes); }
