@@ -324,6 +324,7 @@ struct OrientInPass {
 __global__ __launch_bounds__(kCT) void k_orient_in_scatter(OrientInPass op, const uint64_t *__restrict__ tile_off) {
     __shared__ uint32_t s_w[2][kCT / 64];        // oriented arcs per wave of a round (two rounds in flight)
     __shared__ uint32_t s_in[kCR * (kCT / 64)];  // in-list arcs per (round, wave), then their exclusive prefix
+    static_assert(kCR * (kCT / 64) == kWave, "one wave scans s_in, an entry per lane");
     __shared__ uint32_t s_tile;
     __shared__ uint64_t s_excl;
     if (threadIdx.x == 0) s_tile = atomicAdd(op.ticket, 1u);
