@@ -411,6 +411,18 @@ lstc_status lstc_work_stats_workspace(uint32_t G, size_t *bytes);
 lstc_status lstc_work_stats(const lstc_graph_desc *graphs, uint32_t G, const lstc_tune *tune,
                             lstc_work *out, void *d_ws, size_t ws_bytes, lstc_stream s);
 
+/* What a count over one graph did that has run with this workspace and these
+ * sizes (diagnostic; lstc_count without d_per_row: split 0; lstc_count_split with
+ * segment words or lstc_count_split_stream: split 1): LSTC_PATH_DECIDED, the
+ * sizes let it look for codes that pay; LSTC_PATH_BUILT, it found them and built
+ * them; LSTC_PATH_CODES, it counted from them (else, as with *path == 0, from ids).
+ * Reads what the count left in d_ws; synchronises the stream.               */
+#define LSTC_PATH_DECIDED 1u
+#define LSTC_PATH_BUILT 2u
+#define LSTC_PATH_CODES 4u
+lstc_status lstc_count_path(uint32_t n_rows, uint32_t n_owned, uint64_t m, int split, void *d_ws, size_t ws_bytes,
+                            uint32_t *path, lstc_stream s);
+
 /* Count-kernel timing (diagnostic; the reference brackets its kernel with
  * cudaEvents, src/WithoutPartition/ShareKernelTCV62_update_v1.cu:263-290).
  * While enabled, every launch of the count kernel on a stream that is not

@@ -79,6 +79,15 @@ def test_batch_workspace_holds_no_code_arrays(graphs):
     assert one.value > 4 * m
 
 
+def test_count_path_needs_no_device_where_sizes_decide():
+    lib, path = _lib.load(), ctypes.c_uint32(9)
+    ws = ctypes.c_size_t(1 << 30)
+    assert lib.lstc_count_path(100, 100, 1000, 1, 0x10000, ws, ctypes.byref(path), None) == 0 and path.value == 0
+    for args in ((100, 100, 1000, 1, None, ws, ctypes.byref(path), None), (100, 101, 1000, 1, 0x10000, ws, ctypes.byref(path), None),
+                 (100, 100, 1000, 1, 0x10000, ws, None, None)):
+        assert lib.lstc_count_path(*args) == _lib.LSTC_ERR_INVALID
+
+
 # Shape validation happens on the host before any HIP call, so these run without
 # a device.  The pointers are placeholders that are never dereferenced.
 _FAKE = ctypes.c_void_p(0x10000)

@@ -1,0 +1,126 @@
+"""GPU tests of the count from 16-bit hub codes: every test says which way the call has to go
+(lstc_count_path), on graphs far from the lines of the rule that chooses, and compares the count
+with the oracle, a closed form, a golden count or the count from ids."""
+import json
+
+import numpy as np
+import pytest
+import torch
+
+import graphs as G
+from trianglecount_amd._lib import LSTC_PATH_BUILT, LSTC_PATH_CODES, LSTC_PATH_DECIDED
+
+pytestmark = pytest.mark.gpu
+
+CODES = LSTC_PATH_DECIDED | LSTC_PATH_BUILT | LSTC_PATH_CODES
+TAKEN_BACK = LSTC_PATH_DECIDED | LSTC_PATH_BUILT
+
+
+def _up(a):
+    return torch.from_numpy(np.ascontiguousarray(a).view(np.int32)).cuda()
+
+
+def _count(lstc, g, **kw):
+    """The count, and the way it took."""
+    ws = lstc.Workspace()
+    c = lstc.count(g, ws=ws, **kw)
+    return c, lstc.count_path(g, ws, kw.get("n_owned"), kw.get("split", True))
+
+
+def _shared_hubs(n, hubs, deg):
+    """`hubs` vertices joined to each other, and n others with `deg` of them each, in a window that moves along:
+    rows of `deg` entries, and in-lists of a large share of all vertices."""
+    v = np.arange(n, dtype=np.int64)
+    dst = (v[:, None] * 7 + np.arange(deg)) % hubs
+    i, j = np.triu_indices(hubs, 1)
+    src = np.concatenate([np.repeat(v + hubs, deg), i])
+    return n + hubs, src.astype(np.uint32), np.concatenate([dst.ravel(), j]).astype(np.uint32)
+
+
+def _lists(g):
+    """Lists that the split count streams per row: a row's own arcs and its in-list."""
+    d = np.diff(g.off.astype(np.int64))
+    src = np.repeat(np.arange(len(d)), d)
+    return d + np.bincount(g.col[d[src] <= d[g.col]], minlength=len(d))
+
+
+@pytest.mark.parametrize("name,parts,chunks", [("rmat", 8, 1), ("complete", 8, 1), ("uniform", 8, 1),
+                                               ("hubs_20k", 32, 1), ("hubs_60k", 32, 2)])
+def test_split_count_from_codes(lstc, oracle, name, parts, chunks):
+    """Rows without and with bitmaps, cut into 8 and 32 parts, and into several chunks per part."""
+    n, s, d = {"rmat": lambda: oracle.gen_rmat(16, 64, seed=2), "complete": lambda: G.complete(2301),
+               "uniform": lambda: oracle.gen_er(9001, 900.0, seed=4),
+               "hubs_20k": lambda: _shared_hubs(20_011, 400, 300),
+               "hubs_60k": lambda: _shared_hubs(60_013, 200, 150)}[name]()
+    og = oracle.clean_orient(n, s, d)[1]
+    most = int(_lists(og).max())
+    assert {8: 512 <= most < 2048 or name in ("complete", "rmat"), 32: most >= 2048}[parts]
+    assert chunks == 1 or most > 32 * 1024
+    want = oracle.count(og)
+    for stream in (True, False):
+        g = lstc.clean_orient(n, _up(s), _up(d), in_lists=True, stream_copy=stream)
+        assert [_count(lstc, g) for _ in range(2)] == [(want, CODES)] * 2
+
+
+@pytest.mark.parametrize("scale", [21, 22])
+def test_tails_from_codes(lstc, scale):
+    """More vertices than codes (s21: 6% of the columns are ids, s22 more), split and plain, against golden counts."""
+    with open(G.GOLDEN + "/rmat_counts.json") as f:
+        want = json.load(f)[str(scale)]["triangles"]
+    g = lstc.clean_orient(*lstc.generate_rmat(scale, 16, seed=1), in_lists=True, stream_copy=True)
+    assert _count(lstc, g) == (want, CODES)
+    assert _count(lstc, g, split=False) == (want, CODES)
+
+
+@pytest.mark.parametrize("owned", [1.0, 0.6])
+def test_plain_count_from_codes(lstc, owned):
+    g = lstc.clean_orient(*lstc.generate_rmat(20, 24, seed=3))
+    no = int(g.n * owned)
+    per_row = lstc.count(g, per_row=True, split=False)[1]
+    assert _count(lstc, g, n_owned=no) == (int(per_row[:no].sum()), CODES)
+
+
+def test_half_graph_part_from_codes(lstc):
+    """A part of two: halo rows own no arcs but stream and are streamed."""
+    g = lstc.clean_orient(*lstc.generate_rmat(21, 20, seed=9), keep_symmetric=True)
+    part = lstc.partition_random(g.n, 2, seed=4)
+    total = 0
+    for p in range(2):
+        h = lstc.stream_copy(lstc.halo_extract(g, part, p, split=True))
+        assert h.owned < h.n
+        c, path = _count(lstc, h)
+        assert path == CODES and c == int(lstc.count(h, per_row=True, split=False)[1].sum())
+        total += c
+    assert total == lstc.count(g, split=False)
+
+
+@pytest.mark.parametrize("n,mean", [(200_003, 100.0), (1_000_003, 12.0)])
+def test_uniform_graphs_stay_with_ids(lstc, n, mean):
+    """No vertices that stand out (and more of them than codes), or short rows."""
+    g = lstc.clean_orient(*lstc.generate_er(n, mean, seed=6), in_lists=True, stream_copy=True)
+    c, path = _count(lstc, g)
+    assert not path & LSTC_PATH_CODES
+    want = int(lstc.count(g, per_row=True, split=False)[1].sum())
+    assert c == want and lstc.count(g, split=False) == want
+
+
+@pytest.mark.parametrize("longest", [(1 << 17) - 1, 1 << 17, (1 << 17) + 60])
+def test_rows_that_codes_cannot_hold(lstc, oracle, longest):
+    """52 rows around the longest that a record can say (several in every wave of a workgroup of the build) behind
+    a graph for which codes are chosen and built: the rows, or their tails of tens of thousands of ids, take the
+    count back to ids."""
+    k = 52
+    og = oracle.clean_orient(*_shared_hubs(30_000, 600, 450))[1]
+    rows = np.diff(og.off.astype(np.int64))
+    heads, first = len(rows), len(rows) + 5 * k
+    path = np.arange(first, first + longest, dtype=np.uint32)  # v -> v + 1, all but the last
+    d = np.zeros(first + longest, np.int64)
+    d[:heads] = rows
+    d[heads:first:5] = longest
+    d[first:-1] = 1
+    off = np.concatenate([[0], np.cumsum(d)])
+    g = lstc.Graph(len(d), int(off[-1]), torch.from_numpy(off).cuda(), _up(np.concatenate([og.col, np.tile(path, k), path[1:]])))
+    want = k * (longest - 1) + oracle.count(og)  # a long row, v and v + 1
+    assert [_count(lstc, g) for _ in range(2)] == [(want, TAKEN_BACK)] * 2
+    lstc.in_lists(g)
+    assert [_count(lstc, g) for _ in range(2)] == [(want, TAKEN_BACK)] * 2

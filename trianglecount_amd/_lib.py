@@ -87,6 +87,7 @@ class ServerStats(C.Structure):
         return {k: getattr(self, k) for k, _ in self._fields_}
 
 
+LSTC_PATH_DECIDED, LSTC_PATH_BUILT, LSTC_PATH_CODES = 1, 2, 4
 LSTC_REQ_RMAT, LSTC_REQ_ER, LSTC_REQ_CSR = 0, 1, 2
 
 VP = C.c_void_p
@@ -146,6 +147,7 @@ SIGNATURES = {
     "lstc_tune_resolve": (ST, [C.POINTER(GraphDesc), U32, C.POINTER(Tune), C.POINTER(Tune)]),
     "lstc_work_stats_workspace": (ST, [U32, PSZ]),
     "lstc_work_stats": (ST, [C.POINTER(GraphDesc), U32, C.POINTER(Tune), C.POINTER(WorkStats), VP, SZ, VP]),
+    "lstc_count_path": (ST, [U32, U32, U64, I32, VP, SZ, PU32, VP]),
     "lstc_timing_enable": (ST, [I32]),
     "lstc_timing_read": (ST, [C.POINTER(C.c_double), PU64]),
     "lstc_autotune": (ST, [C.POINTER(GraphDesc), U32, U32, C.POINTER(Tune), C.POINTER(C.c_double), VP]),

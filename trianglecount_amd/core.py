@@ -355,6 +355,16 @@ def count(g: Graph, n_owned: int | None = None, per_row: bool = False, tune: Tun
     return total
 
 
+def count_path(g: Graph, ws: Workspace, n_owned: int | None = None, split: bool = True, stream=None) -> int:
+    """LSTC_PATH_* bits of the last ``count(g, n_owned, ws=ws, split=split)``: whether it looked for 16-bit codes
+    that pay, built them, and counted from them (0: from ids)."""
+    no = g.owned if n_owned is None else int(n_owned)
+    path = C.c_uint32()
+    check(load().lstc_count_path(g.n, no, g.m, int(split and g.split_ready(no)), C.c_void_p(ws.buf.data_ptr()),
+                                 ws.buf.numel(), C.byref(path), C.c_void_p(stream_handle(stream))), "lstc_count_path")
+    return path.value
+
+
 def triangle_support(g: Graph, n_owned: int | None = None, per_edge: bool = True, per_vertex: bool = True,
                      split: bool | None = None, ws: Workspace | None = None, stream=None):
     """Per-edge support (uint32 per arc of g.col) and per-vertex triangle counts (uint64 per row),

@@ -56,3 +56,11 @@ extern "C" lstc_status lstc_count_split_stream(const uint64_t *d_off, const uint
     return count_launch(&h, 1, nullptr, nullptr, (unsigned long long *)d_count, tune, d_ws, ws_bytes,
                         (hipStream_t)s);
 }
+
+extern "C" lstc_status lstc_count_path(uint32_t n_rows, uint32_t n_owned, uint64_t m, int split, void *d_ws,
+                                       size_t ws_bytes, uint32_t *path, lstc_stream s) {
+    if (!path) return fail(LSTC_ERR_INVALID, "lstc_count_path: NULL output");
+    if (!d_ws) return fail(LSTC_ERR_INVALID, "lstc_count_path: NULL workspace");
+    if (n_owned > n_rows) return fail(LSTC_ERR_INVALID, "lstc_count_path: n_owned %u > n_rows %u", n_owned, n_rows);
+    return count_path(n_rows, n_owned, m, split != 0, d_ws, ws_bytes, (hipStream_t)s, path);
+}

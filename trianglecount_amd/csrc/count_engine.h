@@ -114,6 +114,10 @@ lstc_status count_launch(const HostGraph *hosts, uint32_t G, const GraphDev *d_t
                          unsigned long long *d_counts, const lstc_tune *tune, void *ws, size_t ws_bytes,
                          hipStream_t st, bool timed = true);
 
+// lstc_count_path.
+lstc_status count_path(uint32_t n_rows, uint32_t n_owned, uint64_t m, bool split, void *ws, size_t ws_bytes,
+                       hipStream_t st, uint32_t *path);
+
 // Kernel timing (lstc_timing_enable): when enabled and the stream is not being
 // captured, timing_begin / timing_end record a hipEvent pair around a launch.
 struct TimingMark {

@@ -1083,11 +1083,29 @@ static constexpr int kHubU = 4;
 // queue entries: per row one kind A item and at most 1 + in-degree / kInChunk kind B items
 static uint64_t queue_cap(uint64_t total_rows, uint64_t total_m) { return 2 * total_rows + total_m / kInChunk + 1; }
 
+// The engine's own arrays, first in its workspace.
+struct PlanArrays {
+    uint32_t *ctl, *wcnt;
+    unsigned long long *queue;
+};
+static PlanArrays plan_arrays(Carver &c, uint64_t total_rows, uint64_t total_m) {
+    PlanArrays a;
+    a.ctl = c.take<uint32_t>(C_WORDS);
+    a.wcnt = c.take<uint32_t>(kPlanEntries);
+    a.queue = c.take<unsigned long long>(queue_cap(total_rows, total_m));
+    return a;
+}
+
+// The code arrays of a launch over one graph, behind them (hctl null: it counts from ids).
+static HubSet code_arrays(Carver &c, uint32_t rows, uint64_t m, bool split) {
+    if (!hub_fits(rows, m, split)) return HubSet{};
+    const HubSet h = hub_layout(c, rows, m);
+    return c.ok() ? h : HubSet{};
+}
+
 size_t count_ws_base(uint64_t total_rows, uint64_t total_m) {
     Carver c(nullptr, 0);
-    c.take<uint32_t>(C_WORDS);
-    c.take<uint32_t>(kPlanEntries);
-    c.take<unsigned long long>(queue_cap(total_rows, total_m));
+    (void)plan_arrays(c, total_rows, total_m);
     return c.need();
 }
 
@@ -1096,6 +1114,21 @@ size_t count_ws_bytes(uint64_t rows, uint64_t m) {
     c.take<char>(count_ws_base(rows, m));
     if (hub_fits(rows, m)) (void)hub_layout(c, rows, m);
     return c.need();
+}
+
+lstc_status count_path(uint32_t n_rows, uint32_t n_owned, uint64_t m, bool split, void *ws, size_t ws_bytes,
+                       hipStream_t st, uint32_t *path) {
+    *path = 0;
+    const uint64_t planned = split ? n_rows : n_owned;
+    Carver c(ws, ws_bytes);
+    (void)plan_arrays(c, planned, m);
+    const HubSet hs = planned ? code_arrays(c, n_rows, m, split) : HubSet{};
+    if (!hs.hctl) return LSTC_OK;
+    uint32_t words[HC_CHOSEN + 1];
+    LSTC_HIP(hipMemcpyAsync(words, hs.hctl, sizeof(words), hipMemcpyDeviceToHost, st));
+    LSTC_HIP(hipStreamSynchronize(st));
+    *path = LSTC_PATH_DECIDED | (words[HC_CHOSEN] ? LSTC_PATH_BUILT : 0u) | (words[HC_ON] ? LSTC_PATH_CODES : 0u);
+    return LSTC_OK;
 }
 
 lstc_status count_launch(const HostGraph *hosts, uint32_t G, const GraphDev *d_table, const uint64_t *d_row_base,
@@ -1115,9 +1148,9 @@ lstc_status count_launch(const HostGraph *hosts, uint32_t G, const GraphDev *d_t
     Carver c(ws, ws_bytes);
     if (queue_cap(total, total_m) >= 0xFFFFFFFFull)
         return fail(LSTC_ERR_INVALID, "count: more than 2^32-1 work items in one launch");
-    uint32_t *ctl = c.take<uint32_t>(C_WORDS);
-    uint32_t *wcnt = c.take<uint32_t>(kPlanEntries);
-    unsigned long long *queue = c.take<unsigned long long>(queue_cap(total, total_m));
+    const PlanArrays arrays = plan_arrays(c, total, total_m);
+    uint32_t *ctl = arrays.ctl, *wcnt = arrays.wcnt;
+    unsigned long long *queue = arrays.queue;
     if (!ws || !c.ok()) return fail(LSTC_ERR_WORKSPACE, "count: workspace %zu < %zu bytes", ws_bytes, c.need());
 
     GraphSet gs{};
@@ -1160,14 +1193,11 @@ lstc_status count_launch(const HostGraph *hosts, uint32_t G, const GraphDev *d_t
     uint32_t hub_grid = 0;
     using HubKern = void (*)(GraphDev, HubSet, unsigned long long *);
     const HubKern hub_kern = split ? (HubKern)k_count_hub<kHubU, true> : (HubKern)k_count_hub<kHubU, false>;
-    if (G == 1 && (split ? seg_ok(hosts[0]) : !hosts[0].per_row) && hub_fits(hosts[0].n_rows, total_m, split)) {
-        const HubSet h = hub_layout(c, hosts[0].n_rows, total_m);
-        if (c.ok()) {
-            hs = h;
-            const uint32_t hfit = resident_blocks((const void *)hub_kern, 64);
-            hub_grid = (uint32_t)cus * (hfit ? hfit : 1u);
-            LSTC_TRY(hub_build(gs.one, total_m, hs, st));
-        }
+    if (G == 1 && (split ? seg_ok(hosts[0]) : !hosts[0].per_row)) hs = code_arrays(c, hosts[0].n_rows, total_m, split);
+    if (hs.hctl) {
+        const uint32_t hfit = resident_blocks((const void *)hub_kern, 64);
+        hub_grid = (uint32_t)cus * (hfit ? hfit : 1u);
+        LSTC_TRY(hub_build(gs.one, total_m, hs, st));
     }
     const uint32_t *hub_on = hub_grid ? hs.hctl + HC_ON : nullptr;
     if (total <= kSmallPlan && !hub_grid) {

@@ -82,6 +82,7 @@ __device__ __forceinline__ RowRec split_rec(uint64_t r) {
 
 // words of the selection (uint32)
 enum { HC_ON = 0, HC_LONG_ROWS = 1, HC_DONE = 2, HC_CUT = 3, HC_REST = 4,
+       HC_CHOSEN = 5,  // HC_ON as it was chosen, before rows that codes cannot hold took it back
        HC_LEN = 8, HC_LENS = 10, HC_SQ = 12,  // 64-bit sums
        HC_HIST = 64, HC_SUM = HC_HIST + 256,
        HC_BASE = HC_SUM + 256, HC_USED = HC_BASE + 256,

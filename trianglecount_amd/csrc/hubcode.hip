@@ -193,7 +193,7 @@ __global__ __launch_bounds__(256) void k_hub_pick(const uint32_t *__restrict__ c
     const double to = read64(HC_LEN) / read64(HC_LENS), from = read64(HC_SQ) / (double)m;
     const double share = (double)covered / (double)all;
     const bool on = split ? fmin(from, to) * (2 * share - 1) >= (to < from ? kMinWorthFlat : kMinWorth) : to >= kMinPlainLen;
-    hctl[HC_ON] = on ? 1u : 0u;
+    hctl[HC_ON] = hctl[HC_CHOSEN] = on ? 1u : 0u;
 }
 
 // A workgroup takes 4096 vertices at a time and one place per bin among all of them.
