@@ -1,6 +1,7 @@
 """GPU tests of the count from 16-bit hub codes: every test says which way the call has to go
 (lstc_count_path), on graphs far from the lines of the rule that chooses, and compares the count
 with the oracle, a closed form, a golden count or the count from ids."""
+import ctypes as C
 import json
 
 import numpy as np
@@ -124,3 +125,36 @@ def test_rows_that_codes_cannot_hold(lstc, oracle, longest):
     assert [_count(lstc, g) for _ in range(2)] == [(want, TAKEN_BACK)] * 2
     lstc.in_lists(g)
     assert [_count(lstc, g) for _ in range(2)] == [(want, TAKEN_BACK)] * 2
+
+
+def _kernels(lstc, call):
+    """How many launches a stream-ordered call makes: the nodes of its capture."""
+    L, graph, n = lstc.load(), C.c_void_p(), C.c_size_t()
+    st = torch.cuda.Stream()
+    assert L.hipStreamBeginCapture(C.c_void_p(st.cuda_stream), 2) == 0  # relaxed
+    status = call(C.c_void_p(st.cuda_stream))
+    assert L.hipStreamEndCapture(C.c_void_p(st.cuda_stream), C.byref(graph)) == 0
+    lstc.check(status)
+    assert L.hipGraphGetNodes(graph, None, C.byref(n)) == 0 and L.hipGraphDestroy(graph) == 0
+    return n.value
+
+
+def test_static_count_reads_ids(lstc):
+    """A graph whose codes would fit the static scratch too: counted with the launches of a count whose workspace
+    holds the queue only, fewer than those of a count from codes."""
+    g = lstc.clean_orient(*lstc.generate_rmat(16, 64, seed=2), in_lists=True)
+    want, path = _count(lstc, g)
+    assert path == CODES
+    p = lambda t: C.c_void_p(t.data_ptr())  # noqa: E731
+    full = C.c_size_t()
+    lstc.check(lstc.load().lstc_count_workspace(g.n, g.n, g.m, None, C.byref(full)))
+    assert full.value < lstc.load().lstc_count_split_static_limit()
+    out, ws = torch.zeros(1, dtype=torch.int64, device="cuda"), torch.empty(full.value, dtype=torch.uint8, device="cuda")
+    graph = (p(g.off), p(g.col), p(g.in_off), p(g.in_col), p(g.col_seg), p(g.in_seg), g.n, g.n, g.m, p(out), None)
+    queue = 16 * g.n + g.m // 64 + (1 << 18)
+    split = [_kernels(lstc, lambda s: lstc.load().lstc_count_split(*graph, p(ws), size, s)) for size in (queue, full.value)]
+    static = _kernels(lstc, lambda s: lstc.load().lstc_count_split_static(*graph, s))
+    assert static == split[0] < split[1]
+    lstc.check(lstc.load().lstc_count_split_static(*graph, C.c_void_p(lstc.stream_handle())))
+    torch.cuda.synchronize()
+    assert int(out.item()) == want

@@ -64,6 +64,7 @@ extern "C" lstc_status lstc_count_split_static(const uint64_t *d_off, const uint
                     "(use lstc_count_split with a workspace)", need, kStaticScratch);
     void *ws = nullptr;
     LSTC_TRY(scratch_ptr(&ws));
-    return count_launch(&h, 1, nullptr, nullptr, (unsigned long long *)d_count, tune, ws, kStaticScratch,
-                        (hipStream_t)s, /*timed=*/false);
+    // with room for the queue only: the count reads ids, whatever else the array could hold
+    return count_launch(&h, 1, nullptr, nullptr, (unsigned long long *)d_count, tune, ws, need, (hipStream_t)s,
+                        /*timed=*/false);
 }
