@@ -158,3 +158,19 @@ def test_static_count_reads_ids(lstc):
     lstc.check(lstc.load().lstc_count_split_static(*graph, C.c_void_p(lstc.stream_handle())))
     torch.cuda.synchronize()
     assert int(out.item()) == want
+
+
+@pytest.mark.parametrize("split", [True, False])
+def test_arrays_longer_than_the_graph(lstc, split):
+    """Arrays sized before their graph was cleaned (the server's, with four times the arcs here): what lies behind the arcs
+    has no say in the choice, whether it names rows that would speak for codes or rows without entries."""
+    src = lstc.clean_orient(*lstc.generate_rmat(19, 24, seed=5), in_lists=split)
+    d = src.off[1:src.n + 1] - src.off[:src.n]
+    want, got = lstc.count(src), []
+    for behind in (int(d.argmax()), int(d.argmin())):
+        longer = lambda t, v: torch.cat([t, torch.full((4 * src.m - t.numel(),), v, dtype=t.dtype, device="cuda")])  # noqa: E731
+        lists = {k: longer(getattr(src, k)[:src.m], behind) for k in ("in_col", "col_seg", "in_seg")} if split else {}
+        g = lstc.Graph(src.n, 4 * src.m, src.off, longer(src.col[:src.m], behind), in_off=src.in_off,
+                       in_owned=src.in_owned, **lists)
+        got.append(_count(lstc, g))
+    assert int(d.min()) == 0 and got == [(want, CODES)] * 2

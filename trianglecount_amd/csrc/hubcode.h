@@ -116,7 +116,7 @@ static constexpr uint32_t kOwnGroup = 4, kLightGroup = 4, kSmallGroup = 16;
 bool hub_fits(uint64_t rows, uint64_t m, bool split = true);
 // Takes the arrays from the carver (also to size a workspace).
 HubSet hub_layout(Carver &c, uint64_t rows, uint64_t m);
-// Selects the hubs of the graph and builds its rows' blocks (kernels only).
+// Selects the hubs of the graph and builds its rows' blocks (kernels only).  m: its arcs, or more.
 lstc_status hub_build(const GraphDev &g, uint64_t m, const HubSet &hs, hipStream_t st);
 
 }  // namespace lstc

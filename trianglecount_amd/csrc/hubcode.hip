@@ -50,6 +50,10 @@ __device__ __forceinline__ uint32_t code_of(const uint16_t *code, uint32_t n, ui
     return x < n ? gload(code + x) : kNoCode;
 }
 
+// The arcs there are: the launch knows a bound (the server's arrays are sized before
+// their graph is cleaned), and what lies behind them in the columns is anything.
+__device__ __forceinline__ uint64_t arcs_of(const GraphDev &G) { return sload(G.off + G.n_rows); }
+
 // First unit of the block of row r, whose columns start at o.
 __device__ __forceinline__ uint32_t block_of(uint64_t r, uint64_t o) { return (uint32_t)((o >> 1) + 2 * r); }
 
@@ -78,10 +82,11 @@ __global__ __launch_bounds__(256) void k_hub_init(HubSet hs, const uint64_t *__r
 // one's entries (HC_LEN: the sum of their lengths, HC_LENS: how many).  It leaves
 // at once if the rows are too short for codes (see kMinRows): the Chung-Lu graph of
 // 3M vertices and gamma 2.3 takes 4.48 ms then, 4.77 when the rule waits for the sample, 4.43 from ids.
-__global__ __launch_bounds__(256) void k_hub_sample(GraphDev G, uint64_t m, uint32_t stride, HubSet hs,
-                                                    uint32_t shares, bool split) {
+__global__ __launch_bounds__(256) void k_hub_sample(GraphDev G, uint32_t stride, HubSet hs, uint32_t shares,
+                                                    bool split) {
     constexpr uint32_t kPer = 4;
     uint32_t *cnt = hs.cnt, *hctl = hs.hctl;
+    const uint64_t m = arcs_of(G);
     {
         __shared__ unsigned long long s_sq;
         if (threadIdx.x == 0) s_sq = 0;
@@ -125,9 +130,10 @@ __global__ __launch_bounds__(256) void k_hub_sample(GraphDev G, uint64_t m, uint
 
 // Every workgroup adds its share to the bins; the last one to do so picks.  Bins
 // above HC_CUT are hubs; of bin HC_CUT the first HC_REST vertices that ask.
-__global__ __launch_bounds__(256) void k_hub_pick(const uint32_t *__restrict__ cnt, uint32_t n, uint64_t m,
-                                                  bool split, uint32_t *__restrict__ hctl) {
+__global__ __launch_bounds__(256) void k_hub_pick(GraphDev G, const uint32_t *__restrict__ cnt, bool split,
+                                                  uint32_t *__restrict__ hctl) {
     if (!sload(hctl + HC_LENS)) return;  // nothing was sampled
+    const uint32_t n = G.n_rows;
     __shared__ uint32_t s_n[257], s_add[256];
     __shared__ unsigned long long s_sum[257];
     __shared__ uint32_t s_last;
@@ -190,7 +196,7 @@ __global__ __launch_bounds__(256) void k_hub_pick(const uint32_t *__restrict__ c
         return (double)__hip_atomic_load((unsigned long long *)(hctl + w), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     };
     if (all == 0 || covered * 100 < all * kCoverPct) return;  // (off)
-    const double to = read64(HC_LEN) / read64(HC_LENS), from = read64(HC_SQ) / (double)m;
+    const double to = read64(HC_LEN) / read64(HC_LENS), from = read64(HC_SQ) / (double)arcs_of(G);
     const double share = (double)covered / (double)all;
     const bool on = split ? fmin(from, to) * (2 * share - 1) >= (to < from ? kMinWorthFlat : kMinWorth) : to >= kMinPlainLen;
     hctl[HC_ON] = hctl[HC_CHOSEN] = on ? 1u : 0u;
@@ -415,10 +421,10 @@ lstc_status hub_build(const GraphDev &g, uint64_t m, const HubSet &hs, hipStream
     const uint32_t flat = hmin(hmin(blocks, cus * 4), kInitBlocks);
     hipLaunchKernelGGL(k_hub_init, dim3(flat), dim3(256), 0, st, hs, g.off, n);
     LSTC_LAUNCHED("k_hub_init");
-    hipLaunchKernelGGL(k_hub_sample, dim3(cus * 8), dim3(256), 0, st, g, m, stride, hs, flat,
+    hipLaunchKernelGGL(k_hub_sample, dim3(cus * 8), dim3(256), 0, st, g, stride, hs, flat,
                        g.in_off != nullptr);
     LSTC_LAUNCHED("k_hub_sample");
-    hipLaunchKernelGGL(k_hub_pick, dim3(hmin(blocks, cus)), dim3(256), 0, st, (const uint32_t *)hs.cnt, n, m,
+    hipLaunchKernelGGL(k_hub_pick, dim3(hmin(blocks, cus)), dim3(256), 0, st, g, (const uint32_t *)hs.cnt,
                        g.in_off != nullptr, hs.hctl);
     LSTC_LAUNCHED("k_hub_pick");
     hipLaunchKernelGGL(k_hub_assign, dim3(hmin(ceil_div_u32(n, 4096), cus * 8)), dim3(256), 0, st,
