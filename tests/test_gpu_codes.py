@@ -127,6 +127,17 @@ def test_rows_that_codes_cannot_hold(lstc, oracle, longest):
     assert [_count(lstc, g) for _ in range(2)] == [(want, TAKEN_BACK)] * 2
 
 
+def test_choice_looks_at_all_columns(lstc, oracle):
+    """70 thousand rows that point at vertices without entries, and behind them a graph that is worth codes."""
+    og = oracle.clean_orient(*_shared_hubs(30_000, 600, 450))[1]
+    rows, deg, ends = 70_000, 100, 20_000
+    d = np.concatenate([np.full(rows, deg), np.zeros(ends, np.int64), np.diff(og.off.astype(np.int64))])
+    col = np.concatenate([(rows + (np.arange(rows)[:, None] * 31 + np.arange(deg)) % (ends - deg)).ravel().astype(np.uint32),
+                          og.col + np.uint32(rows + ends)])
+    g = lstc.Graph(len(d), len(col), torch.from_numpy(np.concatenate([[0], np.cumsum(d)])).cuda(), _up(col))
+    assert _count(lstc, g) == (oracle.count(og), CODES)
+
+
 def _kernels(lstc, call):
     """How many launches a stream-ordered call makes: the nodes of its capture."""
     L, graph, n = lstc.load(), C.c_void_p(), C.c_size_t()
