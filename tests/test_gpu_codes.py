@@ -95,6 +95,23 @@ def test_half_graph_part_from_codes(lstc):
     assert total == lstc.count(g, split=False)
 
 
+@pytest.mark.parametrize("owned", [0, 1, 1000])
+def test_few_owned_rows_of_a_large_graph(lstc, owned):
+    """The codes of a whole graph are not built, nor looked for, to count a few of its rows."""
+    g = lstc.clean_orient(*lstc.generate_rmat(20, 24, seed=3))
+    per_row = lstc.count(g, per_row=True, split=False)[1]
+    assert _count(lstc, g, n_owned=owned) == (int(per_row[:owned].sum()), 0)
+
+
+def test_small_part_stays_with_ids(lstc):
+    """A part of 16 with its halo holds most of the graph's arcs; its owned rows have a sixteenth of them."""
+    g = lstc.clean_orient(*lstc.generate_rmat(20, 24, seed=3), keep_symmetric=True)
+    h = lstc.stream_copy(lstc.halo_extract(g, lstc.partition_random(g.n, 16, seed=4), 3, split=True))
+    assert h.m > g.m // 2
+    want = int(lstc.count(h, per_row=True, split=False)[1].sum())
+    assert _count(lstc, h) == (want, 0) and _count(lstc, h, split=False) == (want, 0)
+
+
 @pytest.mark.parametrize("n,mean", [(200_003, 100.0), (1_000_003, 12.0)])
 def test_uniform_graphs_stay_with_ids(lstc, n, mean):
     """No vertices that stand out (and more of them than codes), or short rows."""

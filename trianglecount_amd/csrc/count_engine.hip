@@ -1097,8 +1097,8 @@ static PlanArrays plan_arrays(Carver &c, uint64_t total_rows, uint64_t total_m) 
 }
 
 // The code arrays of a launch over one graph, behind them (hctl null: it counts from ids).
-static HubSet code_arrays(Carver &c, uint32_t rows, uint64_t m, bool split) {
-    if (!hub_fits(rows, m, split)) return HubSet{};
+static HubSet code_arrays(Carver &c, uint32_t rows, uint32_t owned, uint64_t m, bool split) {
+    if (!hub_fits(rows, m, split) || !hub_worth(rows, owned, m, split)) return HubSet{};
     const HubSet h = hub_layout(c, rows, m);
     return c.ok() ? h : HubSet{};
 }
@@ -1122,7 +1122,7 @@ lstc_status count_path(uint32_t n_rows, uint32_t n_owned, uint64_t m, bool split
     const uint64_t planned = split ? n_rows : n_owned;
     Carver c(ws, ws_bytes);
     (void)plan_arrays(c, planned, m);
-    const HubSet hs = planned ? code_arrays(c, n_rows, m, split) : HubSet{};
+    const HubSet hs = planned ? code_arrays(c, n_rows, n_owned, m, split) : HubSet{};
     if (!hs.hctl) return LSTC_OK;
     uint32_t words[HC_CHOSEN + 1];
     LSTC_HIP(hipMemcpyAsync(words, hs.hctl, sizeof(words), hipMemcpyDeviceToHost, st));
@@ -1193,7 +1193,8 @@ lstc_status count_launch(const HostGraph *hosts, uint32_t G, const GraphDev *d_t
     uint32_t hub_grid = 0;
     using HubKern = void (*)(GraphDev, HubSet, unsigned long long *);
     const HubKern hub_kern = split ? (HubKern)k_count_hub<kHubU, true> : (HubKern)k_count_hub<kHubU, false>;
-    if (G == 1 && (split ? seg_ok(hosts[0]) : !hosts[0].per_row)) hs = code_arrays(c, hosts[0].n_rows, total_m, split);
+    if (G == 1 && (split ? seg_ok(hosts[0]) : !hosts[0].per_row))
+        hs = code_arrays(c, hosts[0].n_rows, hosts[0].n_owned, total_m, split);
     if (hs.hctl) {
         const uint32_t hfit = resident_blocks((const void *)hub_kern, 64);
         hub_grid = (uint32_t)cus * (hfit ? hfit : 1u);

@@ -114,6 +114,8 @@ static constexpr uint32_t kOwnGroup = 4, kLightGroup = 4, kSmallGroup = 16;
 // Whether a graph of this size may use codes: enough arcs, and enough per row, that
 // building them pays (see count_launch), and positions that fit 32-bit byte offsets.
 bool hub_fits(uint64_t rows, uint64_t m, bool split = true);
+// Whether enough of it is owned that a count may look for codes.
+bool hub_worth(uint64_t rows, uint64_t owned, uint64_t m, bool split);
 // Takes the arrays from the carver (also to size a workspace).
 HubSet hub_layout(Carver &c, uint64_t rows, uint64_t m);
 // Selects the hubs of the graph and builds its rows' blocks (kernels only).  m: its arcs, or more.

@@ -32,6 +32,15 @@ static constexpr uint64_t kSamples = 2u << 20, kMinStride = 16;
 // graphs 133: 1.51 / 1.78 and 100: 1.73 / 1.47).  Either way half of the sample is covered.
 static constexpr double kMinWorth = 40, kMinWorthFlat = 61, kMinRows = 48, kMinPlainLen = 128, kMinRowsPlain = 42;
 static constexpr uint32_t kCoverPct = 50;
+// The build takes all rows, the count only streams for the owned ones' arcs: the means above count times the share of
+// the arcs that owned rows have (ms from ids / from codes: a part of RMAT s21 in two, E 84, 1.77 / 1.47, in eight 22 0.65 / 0.78; of
+// s23 in eight 22 2.72 / 2.80, in 32 6 1.23 / 1.69).  Without in-lists from 40 on (s21 in eight 47 0.88 / 0.75, s23 in eight
+// 73 4.79 / 3.03, in 32 20 1.54 / 1.64), and row lengths of 12 before the sample.
+static constexpr double kMinPlainLenOwned = 40, kMinRowsOwnedPlain = 12;
+// Below this many arcs of owned rows (by the rows' share; decided on the host) a count of a part is over before a
+// build pays, or before the launches are that find it out: s21 in eight, 6.3M, 0.65 / 0.78 with in-lists, in 32, 2.6M,
+// 0.31 / 0.51, 0.36 / 0.56 without them; the first row of s23 alone 0.01 / 1.42.
+static constexpr double kMinOwned = 12 << 20, kMinOwnedPlain = 3 << 20;
 // Smaller graphs and shorter rows keep ids: the build is worth 0.1 ms (uniform graphs of
 // 1.2M arcs, E 82 to 158, 0.19 / 0.14 and 0.26 / 0.20).  Without in-lists k_count has less to lose to
 // (Chung-Lu of 4.4M arcs 0.464 / 0.441; RMAT s19, 7.7M arcs, 0.65 / 0.92).
@@ -53,6 +62,10 @@ __device__ __forceinline__ uint32_t code_of(const uint16_t *code, uint32_t n, ui
 // The arcs there are: the launch knows a bound (the server's arrays are sized before
 // their graph is cleaned), and what lies behind them in the columns is anything.
 __device__ __forceinline__ uint64_t arcs_of(const GraphDev &G) { return sload(G.off + G.n_rows); }
+// The share of them that the owned rows have.
+__device__ __forceinline__ double owned_share(const GraphDev &G) {
+    return (double)sload(G.off + G.n_owned) / (double)arcs_of(G);
+}
 
 // First unit of the block of row r, whose columns start at o.
 __device__ __forceinline__ uint32_t block_of(uint64_t r, uint64_t o) { return (uint32_t)((o >> 1) + 2 * r); }
@@ -98,7 +111,8 @@ __global__ __launch_bounds__(256) void k_hub_sample(GraphDev G, uint32_t stride,
         __syncthreads();
         const unsigned long long all = s_sq;
         if (blockIdx.x == 0 && threadIdx.x == 0) *(unsigned long long *)(hctl + HC_SQ) = all;
-        if ((double)all < (split ? kMinRows : kMinRowsPlain) * (double)m) return;
+        const double from = (double)all / (double)m, share = owned_share(G);
+        if (split ? from * share < kMinRows : from < kMinRowsPlain || from * share < kMinRowsOwnedPlain) return;
     }
     uint32_t len = 0, lens = 0;
     const uint32_t lane = threadIdx.x & 63;
@@ -203,8 +217,9 @@ __global__ __launch_bounds__(256) void k_hub_pick(GraphDev G, const uint32_t *__
     };
     if (all == 0 || covered * 100 < all * kCoverPct) return;  // (off)
     const double to = read64(HC_LEN) / read64(HC_LENS), from = read64(HC_SQ) / (double)arcs_of(G);
-    const double share = (double)covered / (double)all;
-    const bool on = split ? fmin(from, to) * (2 * share - 1) >= (to < from ? kMinWorthFlat : kMinWorth) : to >= kMinPlainLen;
+    const double cover = (double)covered / (double)all, share = owned_share(G);
+    const bool on = split ? fmin(from, to) * share * (2 * cover - 1) >= (to < from ? kMinWorthFlat : kMinWorth)
+                          : to >= kMinPlainLen && to * share >= kMinPlainLenOwned;
     hctl[HC_ON] = hctl[HC_CHOSEN] = on ? 1u : 0u;
 }
 
@@ -403,6 +418,10 @@ static uint64_t hub_units(uint64_t rows, uint64_t m) { return m / 2 + 2 * rows +
 
 bool hub_fits(uint64_t rows, uint64_t m, bool split) {
     return m >= (split ? kMinArcs : kMinArcsPlain) && m >= kMinPerRow * rows && rows < (1ull << 32) && hub_units(rows, m) < (1ull << 29);
+}
+
+bool hub_worth(uint64_t rows, uint64_t owned, uint64_t m, bool split) {
+    return owned == rows || (double)m * (double)owned >= (split ? kMinOwned : kMinOwnedPlain) * (double)rows;
 }
 
 HubSet hub_layout(Carver &c, uint64_t rows, uint64_t m) {
