@@ -17,34 +17,60 @@ namespace lstc {
 // Sampled entries (RMAT s23, ms a count: 11.1 with 2^20, 10.7 with 2^21, 10.8 with
 // 2^22), and at most one in 16: the hubs' counters are hot addresses.
 static constexpr uint64_t kSamples = 2u << 20, kMinStride = 16;
-// Codes pay where much is streamed per arc and hubs are most of it.  With in-lists
-// an arc streams at most the smaller of the mean d+ of its two ends' rows, E (each a mean over
-// arcs); with the share c of the sample that the hubs cover, codes are taken
-// from E (2 c - 1) = 40 on, from 61 if the rows that arcs point at are the shorter ones (uniform graphs).  Calls from codes against ids, ms: 90 at RMAT s17 0.28 / 0.35, 109 at s18
-// 0.40 / 0.43, 166 at s21 2.2 / 3.2, 173 at s23 10.4 / 17.1; 106 on a uniform graph of 100
-// thousand vertices and mean degree 400 1.50 / 1.76, 66 on one of 20 thousand and 200 0.20 / 0.18
-// (0.22 if it is found out after the sample); Chung-Lu graphs, gamma 2.1, of 1M vertices and mean
-// degree 50, 62.5, 1.84 / 1.70 (2.02 after the sample), of 3M 52 5.4 / 5.8.  Below: 60 (uniform, 130
-// thousand, 300) 1.70 / 1.42; Chung-Lu, gamma 2.3, 1M, 23 1.97 / 1.47, 3M, 10 5.65 / 4.43.
-// Rows shorter than kMinRows (without in-lists kMinRowsPlain) in the mean over arcs are not sampled.
-// Without in-lists an arc streams its target's row: codes from a mean of 128 on (RMAT s21 357:
-// 2.6 / 5.4, Chung-Lu of 3M, gamma 2.3, 138: 5.3 / 6.0; of 1M 111: 1.79 / 1.61; the uniform
-// graphs 133: 1.51 / 1.78 and 100: 1.73 / 1.47).  Either way half of the sample is covered.
-static constexpr double kMinWorth = 40, kMinWorthFlat = 61, kMinRows = 48, kMinPlainLen = 128, kMinRowsPlain = 42;
-static constexpr uint32_t kCoverPct = 50;
-// The build takes all rows, the count only streams for the owned ones' arcs: the means above count times the share of
-// the arcs that owned rows have (ms from ids / from codes: a part of RMAT s21 in two, E 84, 1.77 / 1.47, in eight 22 0.65 / 0.78; of
-// s23 in eight 22 2.72 / 2.80, in 32 6 1.23 / 1.69).  Without in-lists from 40 on (s21 in eight 47 0.88 / 0.75, s23 in eight
-// 73 4.79 / 3.03, in 32 20 1.54 / 1.64), and row lengths of 12 before the sample.
-static constexpr double kMinPlainLenOwned = 40, kMinRowsOwnedPlain = 12;
-// Below this many arcs of owned rows (by the rows' share; decided on the host) a count of a part is over before a
-// build pays, or before the launches are that find it out: s21 in eight, 6.3M, 0.65 / 0.78 with in-lists, in 32, 2.6M,
-// 0.31 / 0.51, 0.36 / 0.56 without them; the first row of s23 alone 0.01 / 1.42.
+// When codes pay.  What they save is in proportion to what is streamed: per arc of the owned
+// rows, with in-lists, at most the smaller of the mean d+ of its two ends' rows (`from` and `to`,
+// each a mean over arcs), without in-lists its target's row.  What they cost, the build, is in
+// proportion to all arcs; so the lines below are on these means times the owned rows' share of the arcs.
+//
+// 1. Before the sample (worth_sampling), from the row lengths alone.  Found out here, a graph
+// costs 0.02 to 0.04 ms, after the sample 0.1 to 0.3 ms.
+// 2. After it (k_hub_pick), with `to`, the share c of the columns that hubs cover, and the
+// tails' share of what would be streamed.
+// Figures: ms a call from ids / from codes.
+//
+// With in-lists, from on: RMAT s17 90 0.338 / 0.273, s18 109 0.428 / 0.403, s21 189 3.14 / 2.15, s23 270
+// 16.9 / 10.3; Chung-Lu graphs (gamma 2.1, mean degree 50) of 300 thousand vertices 65 0.594 / 0.638,
+// 1M 84 1.70 / 1.85, 1.5M 92 2.63 / 2.72, 2M 96 3.57 / 3.59, 3M 103 5.59 / 5.39; gamma 2.3, mean 150, 300
+// thousand vertices 104 1.57 / 1.45, gamma 2.5 84 1.47 / 1.54.  The line rises with the vertices, of which the hubs
+// are a smaller part.  Without in-lists: gamma 2.3, mean 50, 1M vertices 43 1.61 / 1.79, 2M 45 3.67 / 3.43, 3M 47
+// 6.01 / 5.29; 2.1, 300 thousand 65 0.568 / 0.605, 500 thousand 73 1.03 / 0.94; gamma 2.5, mean 150, 300 thousand
+// 84 1.58 / 1.39, 1M 87 6.80 / 5.19.
+static constexpr double kMinFrom = 86, kMinFromMore = 14, kMinFromRows = 1 << 21;  // 86 to 100
+static constexpr double kMinFromPlain = 70, kMinFromPlainBig = 45;
+static constexpr uint64_t kBigPlain = 1ull << 25;  // arcs from which the second holds
+// Owned rows: a part of RMAT s21 in two, from times share 95, 1.77 / 1.47, in eight 25 0.68 / 0.78; of s23 in eight 35
+// 2.80 / 2.80, in 32 10 1.46 / 1.69.  Without in-lists `from` says less, and a smaller share pays: s23, the first 3% of the
+// rows (a seventh of the count) 5.27 / 2.99, 0.3% 1.51 / 1.90.
+static constexpr double kMinFromOwnedPlain = 12;
+// Below this many arcs of owned rows (by the rows' share; decided on the host) a count of a part
+// is over before a build pays, or before the launches are that find it out: s21 in eight 6.3M 0.68 / 0.78, in 32 2.6M
+// 0.36 / 0.51; one row of s23 0.04 / 1.42.
 static constexpr double kMinOwned = 12 << 20, kMinOwnedPlain = 3 << 20;
-// Smaller graphs and shorter rows keep ids: the build is worth 0.1 ms (uniform graphs of
-// 1.2M arcs, E 82 to 158, 0.19 / 0.14 and 0.26 / 0.20).  Without in-lists k_count has less to lose to
-// (Chung-Lu of 4.4M arcs 0.464 / 0.441; RMAT s19, 7.7M arcs, 0.65 / 0.92).
+// Uniform graphs: where neither degree nor order of the vertices means anything, d+ runs evenly from 0 to
+// twice its mean, and the mean over arcs is 4/3 of that (1.25 to 1.32 measured with mean degrees of 40 to
+// 1800; power laws of gamma 2.5 1.14 to 1.22, 2.3 1.4 and more, RMAT 3 and more).  A count of them from ids is fast (every list is
+// short), and without hubs the codes cover what their number covers: from 105 thousand vertices on the tails cost
+// more than the codes save (115 thousand, mean degree 400, 1.93 / 2.14; 130 thousand, 600, 4.4 / 7.7; 160 thousand, 400,
+// plain 3.0 / 5.5).  Below, by the sum of the squares of the row lengths: 2e8 20 thousand vertices, mean degree 200, 0.170 / 0.212,
+// 5e8 10 thousand, 400, 0.230 / 0.281 and 40 thousand, 200, 0.306 / 0.293, 6e8 8 thousand, 500, 0.268 / 0.319, 7.6e8 60 thousand,
+// 200, 0.439 / 0.379, 1e9 4 thousand, 1000, 0.456 / 0.367; plain 1e9 80 thousand, 200, 0.450 / 0.467, 1.3e9 100 thousand, 200,
+// 0.603 / 0.619, 3e9 60 thousand, 400, 1.00 / 0.78.
+static constexpr double kUniformLow = 1.23, kUniformHigh = 1.4, kMinUniform = 7e8, kMinUniformPlain = 2e9;
+static constexpr uint32_t kMaxUniformRows = 105000;
+// After the sample, with in-lists: min(from, to) (2 c - 1) (3M vertices, gamma 2.1, 52 5.59 / 5.39; 2.5, mean 150, 1M 23
+// 4.73 / 5.72; with the target's row the shorter one, uniform graphs of 100 thousand, mean 200, 56 0.672 / 0.639).
+// Without: `to` (gamma 2.3, 1M vertices 111 1.61 / 1.79, 2M 128 3.67 / 3.43; RMAT of 6M arcs 131 0.541 / 0.589, which kMinFromPlain
+// keeps out), times the share for parts (s21 357: 17% of the count, 63 0.94 / 0.77, 10%, 36 0.53 / 0.72).  Either way half of the sample is covered.
+static constexpr double kMinWorth = 40, kMinWorthFlat = 50, kMinPlainLen = 120, kMinPlainLenOwned = 40;
+static constexpr uint32_t kCoverPct = 50;
+// Tails are walked at a quarter of the codes' speed.  Graphs whose arcs point at the longer rows hardly
+// stream any (without in-lists below 1% of the entries for gamma 2.1 and RMAT, 6% for gamma 2.5 and 1M vertices, 6.80 /
+// 5.19) and are not looked at for them (25 us); uniform graphs of 100 thousand vertices 3.3%, of 115 thousand 6.6%, of 130 thousand 10%.
+static constexpr double kMaxTailShare = 0.08;
+// Smaller graphs and shorter rows keep ids: the build is worth 0.1 ms (RMAT s14 of 0.7M arcs 0.147 / 0.229).  Without
+// in-lists k_count has less to lose to (Chung-Lu of 3.3M arcs 0.261 / 0.377; RMAT s19, 7.7M arcs, 0.88 / 0.63).
 static constexpr uint64_t kMinArcs = 3ull << 19, kMinArcsPlain = 6ull << 20, kMinPerRow = 16;
+static constexpr uint64_t kArcSeed = 0x68756263;  // of the arcs that stand for all when the tails are measured
 static constexpr uint32_t kAbsent = 0xFFFFFFFFu;  // past the end of a row (ids are below 2^32 - 2)
 
 __device__ __forceinline__ uint32_t occ_bin(uint32_t c) {
@@ -65,6 +91,15 @@ __device__ __forceinline__ uint64_t arcs_of(const GraphDev &G) { return sload(G.
 // The share of them that the owned rows have.
 __device__ __forceinline__ double owned_share(const GraphDev &G) {
     return (double)sload(G.off + G.n_owned) / (double)arcs_of(G);
+}
+
+// Whether the graph may be worth codes, from the sum of the squares of its row lengths.
+__device__ __forceinline__ bool worth_sampling(const GraphDev &G, double squares, bool split) {
+    const double arcs = (double)arcs_of(G), from = squares / arcs, share = owned_share(G), mean = arcs / G.n_rows;
+    if (from >= kUniformLow * mean && from <= kUniformHigh * mean)
+        return G.n_rows <= kMaxUniformRows && squares * share >= (split ? kMinUniform : kMinUniformPlain);
+    if (split) return from * share >= kMinFrom + kMinFromMore * fmin(1., G.n_rows / kMinFromRows);
+    return from >= (arcs >= (double)kBigPlain ? kMinFromPlainBig : kMinFromPlain) && from * share >= kMinFromOwnedPlain;
 }
 
 // First unit of the block of row r, whose columns start at o.
@@ -94,7 +129,7 @@ __global__ __launch_bounds__(256) void k_hub_init(HubSet hs, const uint64_t *__r
 // A wave takes four chunks at a time; every fourth wave measures the rows of one of
 // them (in turn the first to the fourth, which lie a quarter of the columns apart in a graph of
 // up to 2^25 arcs): HC_LEN, the sum of their lengths, HC_LENS: how many.  It leaves
-// at once if the rows are too short for codes (see kMinRows): the Chung-Lu graph of
+// at once if the rows are too short for codes: the Chung-Lu graph of
 // 3M vertices and gamma 2.3 takes 4.48 ms then, 4.77 when the rule waits for the sample, 4.43 from ids.
 __global__ __launch_bounds__(256) void k_hub_sample(GraphDev G, uint32_t stride, HubSet hs, uint32_t shares,
                                                     bool split) {
@@ -111,8 +146,7 @@ __global__ __launch_bounds__(256) void k_hub_sample(GraphDev G, uint32_t stride,
         __syncthreads();
         const unsigned long long all = s_sq;
         if (blockIdx.x == 0 && threadIdx.x == 0) *(unsigned long long *)(hctl + HC_SQ) = all;
-        const double from = (double)all / (double)m, share = owned_share(G);
-        if (split ? from * share < kMinRows : from < kMinRowsPlain || from * share < kMinRowsOwnedPlain) return;
+        if (!worth_sampling(G, (double)all, split)) return;
     }
     uint32_t len = 0, lens = 0;
     const uint32_t lane = threadIdx.x & 63;
@@ -146,6 +180,47 @@ __global__ __launch_bounds__(256) void k_hub_sample(GraphDev G, uint32_t stride,
         atomicAdd((unsigned long long *)(hctl + HC_LEN), (unsigned long long)len);
         atomicAdd((unsigned long long *)(hctl + HC_LENS), (unsigned long long)lens);
     }
+}
+
+// The tails' share of the entries that arcs stream, by a workgroup of 256: kArcs arcs per
+// thread, kEntries entries of each one's target's row.  Vertices of bins below `cut` and cut_tail of
+// that bin's are no hubs.
+__device__ __forceinline__ double tail_share(const GraphDev &G, const uint32_t *__restrict__ cnt, uint32_t cut,
+                                             double cut_tail) {
+    constexpr uint32_t kArcs = 4, kEntries = 8;
+    __shared__ uint64_t s_entries[4], s_tails[4];
+    const uint32_t tid = threadIdx.x, n = G.n_rows, some = (uint32_t)(16 * cut_tail);  // in sixteenths
+    uint32_t x[kArcs], y[kArcs][kEntries];
+    uint64_t o[kArcs], d[kArcs], entries = 0, tails = 0;
+#pragma unroll
+    for (uint32_t q = 0; q < kArcs; ++q) x[q] = gload(G.col + rng64(kArcSeed, q * 256 + tid) % arcs_of(G));
+#pragma unroll
+    for (uint32_t q = 0; q < kArcs; ++q) {
+        o[q] = gload(G.off + (x[q] < n ? x[q] : 0u));
+        d[q] = gload(G.off + (x[q] < n ? x[q] + 1 : 0u)) - o[q];  // (an id without a row: no entries)
+    }
+#pragma unroll
+    for (uint32_t q = 0; q < kArcs; ++q)
+#pragma unroll
+        for (uint32_t k = 0; k < kEntries; ++k)
+            y[q][k] = d[q] ? gload(G.col + o[q] + (2 * k + 1) * d[q] / (2 * kEntries)) : kAbsent;
+#pragma unroll
+    for (uint32_t q = 0; q < kArcs; ++q) {
+        uint32_t t = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < kEntries; ++k) {
+            const uint32_t c = y[q][k] < n ? cnt[y[q][k]] : 0u, bin = occ_bin(c);
+            t += c == 0 || bin < cut ? 16u : bin == cut ? some : 0u;
+        }
+        entries += d[q] * kEntries * 16;
+        tails += d[q] * t;
+    }
+    entries = wave_sum64(entries);
+    tails = wave_sum64(tails);
+    if ((tid & 63) == 0) s_entries[tid >> 6] = entries, s_tails[tid >> 6] = tails;
+    __syncthreads();
+    return (double)(s_tails[0] + s_tails[1] + s_tails[2] + s_tails[3]) /
+           (double)(s_entries[0] + s_entries[1] + s_entries[2] + s_entries[3] + 1);
 }
 
 // Every workgroup adds its share to the bins; the last one to do so picks.  Bins
@@ -202,24 +277,30 @@ __global__ __launch_bounds__(256) void k_hub_pick(GraphDev G, const uint32_t *__
     __syncthreads();
     hctl[HC_BASE + b] = s_n[b + 1];
     const unsigned long long all = s_sum[0];
-    unsigned long long covered = all;
-    if (s_n[0] > kHubs) {
-        if (!(sn > kHubs && s_n[b + 1] <= kHubs)) return;  // the cut bin's thread goes on
-        const uint32_t rest = kHubs - s_n[b + 1];
-        covered = s_sum[b + 1] + own_sum * rest / own_n;
-        hctl[HC_CUT] = b;
-        hctl[HC_REST] = rest;
-    } else if (b != 0) {
-        return;
+    __shared__ uint32_t s_cut, s_rest;
+    __shared__ unsigned long long s_cov;
+    if (b == 0) s_cut = s_rest = 0, s_cov = all;
+    __syncthreads();
+    if (s_n[0] > kHubs && sn > kHubs && s_n[b + 1] <= kHubs) {
+        s_cut = b;
+        s_rest = kHubs - s_n[b + 1];
+        s_cov = s_sum[b + 1] + own_sum * s_rest / own_n;
     }
+    __syncthreads();
+    const uint32_t cut = s_cut, rest = s_rest, cut_n = s_n[cut] - s_n[cut + 1];
+    const unsigned long long covered = s_cov;
+    if (all == 0 || covered * 100 < all * kCoverPct) return;  // (off)
     auto read64 = [&](uint32_t w) {
         return (double)__hip_atomic_load((unsigned long long *)(hctl + w), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     };
-    if (all == 0 || covered * 100 < all * kCoverPct) return;  // (off)
     const double to = read64(HC_LEN) / read64(HC_LENS), from = read64(HC_SQ) / (double)arcs_of(G);
     const double cover = (double)covered / (double)all, share = owned_share(G);
-    const bool on = split ? fmin(from, to) * share * (2 * cover - 1) >= (to < from ? kMinWorthFlat : kMinWorth)
-                          : to >= kMinPlainLen && to * share >= kMinPlainLenOwned;
+    bool on = split ? fmin(from, to) * share * (2 * cover - 1) >= (to < from ? kMinWorthFlat : kMinWorth)
+                    : to >= kMinPlainLen && to * share >= kMinPlainLenOwned;
+    if (on && to < from && n > kHubs) on = tail_share(G, cnt, cut, cut_n ? (double)(cut_n - rest) / cut_n : 1.) <= kMaxTailShare;
+    if (b != 0) return;
+    hctl[HC_CUT] = cut;
+    hctl[HC_REST] = rest;
     hctl[HC_ON] = hctl[HC_CHOSEN] = on ? 1u : 0u;
 }
 
