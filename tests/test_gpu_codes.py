@@ -112,14 +112,20 @@ def test_small_part_stays_with_ids(lstc):
     assert _count(lstc, h) == (want, 0) and _count(lstc, h, split=False) == (want, 0)
 
 
-@pytest.mark.parametrize("n,mean", [(200_003, 100.0), (1_000_003, 12.0)])
-def test_uniform_graphs_stay_with_ids(lstc, n, mean):
-    """No vertices that stand out (and more of them than codes), or short rows."""
-    g = lstc.clean_orient(*lstc.generate_er(n, mean, seed=6), in_lists=True, stream_copy=True)
-    c, path = _count(lstc, g)
-    assert not path & LSTC_PATH_CODES
+@pytest.mark.parametrize("n,mean,joined", [(200_003, 100.0, 0), (1_000_003, 12.0, 0), (130_003, 600.0, 0),
+                                           (160_001, 400.0, 60)])
+def test_uniform_graphs_stay_with_ids(lstc, n, mean, joined):
+    """Short rows; no vertices that stand out, and more of them than codes; the same with a few vertices joined to
+    all others, so that only the tails tell.  No codes are built."""
+    _, src, dst = lstc.generate_er(n, mean, seed=6)
+    if joined:
+        v = torch.arange(n, dtype=torch.int32, device="cuda").repeat(joined)
+        src, dst = torch.cat([src, v]), torch.cat([dst, torch.arange(joined, dtype=torch.int32, device="cuda").repeat_interleave(n)])
+    g = lstc.clean_orient(n, src, dst, in_lists=True, stream_copy=True)
     want = int(lstc.count(g, per_row=True, split=False)[1].sum())
-    assert c == want and lstc.count(g, split=False) == want
+    for split in (True, False):
+        c, path = _count(lstc, g, split=split)
+        assert c == want and not path & LSTC_PATH_BUILT
 
 
 @pytest.mark.parametrize("longest", [(1 << 17) - 1, 1 << 17, (1 << 17) + 60])

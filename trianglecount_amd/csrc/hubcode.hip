@@ -35,7 +35,11 @@ static constexpr uint64_t kSamples = 2u << 20, kMinStride = 16;
 // are a smaller part.  Without in-lists: gamma 2.3, mean 50, 1M vertices 43 1.61 / 1.79, 2M 45 3.67 / 3.43, 3M 47
 // 6.01 / 5.29; 2.1, 300 thousand 65 0.568 / 0.605, 500 thousand 73 1.03 / 0.94; gamma 2.5, mean 150, 300 thousand
 // 84 1.58 / 1.39, 1M 87 6.80 / 5.19.
+// Below 5.5M arcs ids wait for the items of the largest hubs, which codes cut into parts: gamma 2.1, 80 thousand
+// vertices 47 0.40 / 0.32, 110 thousand 51 0.32 / 0.34, 150 thousand 55 0.41 / 0.39, 230 thousand 61 0.52 / 0.52, 260 thousand 63 0.53 / 0.56.
 static constexpr double kMinFrom = 86, kMinFromMore = 14, kMinFromRows = 1 << 21;  // 86 to 100
+static constexpr double kMinFromSmall = 44;
+static constexpr uint64_t kSmall = 11ull << 19;  // arcs below which this holds
 static constexpr double kMinFromPlain = 70, kMinFromPlainBig = 45;
 static constexpr uint64_t kBigPlain = 1ull << 25;  // arcs from which the second holds
 // Owned rows: a part of RMAT s21 in two, from times share 95, 1.77 / 1.47, in eight 25 0.68 / 0.78; of s23 in eight 35
@@ -52,10 +56,12 @@ static constexpr double kMinOwned = 12 << 20, kMinOwnedPlain = 3 << 20;
 // short), and without hubs the codes cover what their number covers: from 105 thousand vertices on the tails cost
 // more than the codes save (115 thousand, mean degree 400, 1.93 / 2.14; 130 thousand, 600, 4.4 / 7.7; 160 thousand, 400,
 // plain 3.0 / 5.5).  Below, by the sum of the squares of the row lengths: 2e8 20 thousand vertices, mean degree 200, 0.170 / 0.212,
-// 5e8 10 thousand, 400, 0.230 / 0.281 and 40 thousand, 200, 0.306 / 0.293, 6e8 8 thousand, 500, 0.268 / 0.319, 7.6e8 60 thousand,
+// 5e8 10 thousand, 400 (2M arcs) 0.230 / 0.281 and 40 thousand, 200 (4M) 0.306 / 0.293, 6e8 8 thousand, 500, 0.268 / 0.319, 7.6e8 60 thousand,
 // 200, 0.439 / 0.379, 1e9 4 thousand, 1000, 0.456 / 0.367; plain 1e9 80 thousand, 200, 0.450 / 0.467, 1.3e9 100 thousand, 200,
 // 0.603 / 0.619, 3e9 60 thousand, 400, 1.00 / 0.78.
 static constexpr double kUniformLow = 1.23, kUniformHigh = 1.4, kMinUniform = 7e8, kMinUniformPlain = 2e9;
+static constexpr double kMinUniformMore = 4.5e8;    // with in-lists, from
+static constexpr uint64_t kUniformMore = 7ull << 19;  // so many arcs on
 static constexpr uint32_t kMaxUniformRows = 105000;
 // After the sample, with in-lists: min(from, to) (2 c - 1) (3M vertices, gamma 2.1, 52 5.59 / 5.39; 2.5, mean 150, 1M 23
 // 4.73 / 5.72; with the target's row the shorter one, uniform graphs of 100 thousand, mean 200, 56 0.672 / 0.639).
@@ -97,8 +103,10 @@ __device__ __forceinline__ double owned_share(const GraphDev &G) {
 __device__ __forceinline__ bool worth_sampling(const GraphDev &G, double squares, bool split) {
     const double arcs = (double)arcs_of(G), from = squares / arcs, share = owned_share(G), mean = arcs / G.n_rows;
     if (from >= kUniformLow * mean && from <= kUniformHigh * mean)
-        return G.n_rows <= kMaxUniformRows && squares * share >= (split ? kMinUniform : kMinUniformPlain);
-    if (split) return from * share >= kMinFrom + kMinFromMore * fmin(1., G.n_rows / kMinFromRows);
+        return G.n_rows <= kMaxUniformRows &&
+               squares * share >= (!split ? kMinUniformPlain : arcs < (double)kUniformMore ? kMinUniform : kMinUniformMore);
+    if (split)
+        return from * share >= (arcs < (double)kSmall ? kMinFromSmall : kMinFrom + kMinFromMore * fmin(1., G.n_rows / kMinFromRows));
     return from >= (arcs >= (double)kBigPlain ? kMinFromPlainBig : kMinFromPlain) && from * share >= kMinFromOwnedPlain;
 }
 
@@ -187,7 +195,7 @@ __global__ __launch_bounds__(256) void k_hub_sample(GraphDev G, uint32_t stride,
 // that bin's are no hubs.
 __device__ __forceinline__ double tail_share(const GraphDev &G, const uint32_t *__restrict__ cnt, uint32_t cut,
                                              double cut_tail) {
-    constexpr uint32_t kArcs = 4, kEntries = 8;
+    constexpr uint32_t kArcs = 2, kEntries = 4;
     __shared__ uint64_t s_entries[4], s_tails[4];
     const uint32_t tid = threadIdx.x, n = G.n_rows, some = (uint32_t)(16 * cut_tail);  // in sixteenths
     uint32_t x[kArcs], y[kArcs][kEntries];
