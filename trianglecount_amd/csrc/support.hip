@@ -291,8 +291,10 @@ __device__ __forceinline__ uint64_t sup_position(const uint32_t *__restrict__ co
 // [Ka, Ka + Kb): kind B, the in-list source u = src[c - Ka], N+(u) streamed.
 // N+(r) is hashed in tiles of TILE keys (a wave tile, or kSupGroupTile); the
 // candidates go in passes of at most kSupPass, each followed by a flush of the
-// slot counters.
-template <int U, bool NARROW, int NT, uint32_t TILE>
+// slot counters.  LISTS: there may be kind B candidates; a walk without them has
+// its own copy of the code (sharing the split rule's, the plain walk kept 56 bytes a lane
+// in scratch for 44: uniform graph of 600 thousand vertices, mean degree 40, 0.87 ms for 0.78).
+template <bool LISTS, int U, bool NARROW, int NT, uint32_t TILE>
 __device__ __forceinline__ void sup_item(const SupTab &Q, const SupWin &W, const uint64_t *__restrict__ off,
                                          const uint32_t *__restrict__ col, const uint32_t *__restrict__ src,
                                          uint32_t n_rows, uint32_t r, uint64_t rb, uint32_t K, uint32_t Ka,
@@ -330,7 +332,7 @@ __device__ __forceinline__ void sup_item(const SupTab &Q, const SupWin &W, const
                         len = (uint32_t)(gload(off + w + 1) - s0);
                         if (below && len >= below) len = 0;  // that arc streams N+(r), at w
                     }
-                } else if (c < p1) {
+                } else if (LISTS && c < p1) {
                     const uint32_t u = gload(src + (c - Ka));
                     if (u < n_rows) {
                         const uint64_t s0 = gload(off + u);
@@ -344,7 +346,7 @@ __device__ __forceinline__ void sup_item(const SupTab &Q, const SupWin &W, const
                 const uint32_t h = sup_window<U, NARROW>(Q, W, col, support, s, len, qmask, qshift, lane, nseg);
                 if (lane < nseg && h != 0) {
                     const uint32_t cc = c0 + W.cand[lane];
-                    if (cc < Ka) {  // arc r -> w
+                    if (!LISTS || cc < Ka) {  // arc r -> w
                         const uint64_t a = rb + cc;
                         if (support) atomicAdd(support + a, h);
                         if (per_vertex) atomicAdd(per_vertex + gload(col + a), (unsigned long long)h);
@@ -414,7 +416,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 8 : 4) void k_support(cons
             const uint32_t r = L.rows[i];
             const uint64_t rb = off[r];
             const uint32_t K = (uint32_t)(off[r + 1] - rb);
-            sup_item<kSupUnroll, NARROW, WAVES * 64, kSupGroupTile>(sup_group_tab(L), W, off, col, nullptr, n_rows, r,
+            sup_item<false, kSupUnroll, NARROW, WAVES * 64, kSupGroupTile>(sup_group_tab(L), W, off, col, nullptr, n_rows, r,
                                                                     rb, K, K, 0, 0, support, per_vertex, &L.next, tid);
         }
         __syncthreads();
@@ -425,7 +427,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 8 : 4) void k_support(cons
         const uint64_t rb = off[u];
         const uint32_t K = (uint32_t)(off[u + 1] - rb);
         if (K < 2 || K > WT) continue;
-        sup_item<kSupUnroll, NARROW, 64, WT>(Q, W, off, col, nullptr, n_rows, (uint32_t)u, rb, K, K, 0, 0, support,
+        sup_item<false, kSupUnroll, NARROW, 64, WT>(Q, W, off, col, nullptr, n_rows, (uint32_t)u, rb, K, K, 0, 0, support,
                                              per_vertex, nullptr, tid & 63);
     }
 }
@@ -498,7 +500,7 @@ __device__ __forceinline__ void sup_split_item(const SupTab &Q, const SupWin &W,
     const uint64_t b0 = (uint64_t)chunk * kSupChunk;
     const uint32_t Kb = b0 < kb ? (uint32_t)min(kb - b0, (uint64_t)kSupChunk) : 0u;
     if (Ka + Kb == 0) return;
-    sup_item<kSupUnroll, NARROW, NT, TILE>(Q, W, off, col, in_col + ib + b0, n_rows, r, rb, K, Ka, Kb, K, support,
+    sup_item<true, kSupUnroll, NARROW, NT, TILE>(Q, W, off, col, in_col + ib + b0, n_rows, r, rb, K, Ka, Kb, K, support,
                                            per_vertex, next, tid);
 }
 
