@@ -97,3 +97,15 @@ def test_support_split_item_edges(lstc, n):
     g = lstc.clean_orient(n, up(s), up(d), in_lists=True)
     sup, pv = lstc.triangle_support(g, split=True)
     assert (sup == n - 2).all() and (pv == (n - 1) * (n - 2) // 2).all()
+
+
+@pytest.mark.parametrize("k", [64, 65, 66])
+def test_support_split_many_items(lstc, k):
+    """1200 complete graphs side by side, with longest rows on both sides of the length up to which waves take several
+    items at once, and enough items that they do."""
+    _, s, d = G.complete(k)
+    shift = np.arange(1200, dtype=np.uint32)[:, None] * np.uint32(k)
+    up = lambda a: torch.from_numpy((a[None] + shift).astype(np.uint32).ravel().view(np.int32)).cuda()  # noqa: E731
+    g = lstc.clean_orient(1200 * k, up(s), up(d), in_lists=True)
+    sup, pv = lstc.triangle_support(g, split=True)
+    assert (sup == k - 2).all() and (pv == (k - 1) * (k - 2) // 2).all()

@@ -447,19 +447,24 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 8 : 4) void k_support(cons
 static constexpr uint32_t kSupChunk = 512;
 // Items are dealt in kSupHeads classes (item t to class t % kSupHeads), each with
 // its own head per kind on a line of its own; a workgroup starts with class blockIdx %
-// kSupHeads and goes on with the others' leftovers.  Waves take up to kSupMaxGroup
-// items at once while many are left, one at the end.  One head for all and one item a
-// ticket put a million tickets on one address: RMAT s21 23.4 ms (groups of 4 on one
-// head 19.5, of 16 22.5 and of 64 25.9: the long items at their ends), now 18.7, and
-// 17.6 with eight waves per workgroup instead of four, which the one head had kept from
-// paying; RMAT s23 123 -> 92 ms, a uniform graph of 300 thousand vertices 3.4 -> 0.43,
-// a 1000 x 1000 grid 9.3 -> 0.81.
-static constexpr uint32_t kSupHeads = 8, kSupHeadStride = 32, kSupMaxGroup = 8;
+// kSupHeads and goes on with the others' leftovers.  One head for all put a million
+// tickets on one address: RMAT s21 25.4 ms, now 20.2, RMAT s23 119 -> 92.
+// Where no row is longer than kSupShort, waves take up to kSupMaxGroup items at
+// once while many are left, one at the end: a uniform graph of 600 thousand vertices, mean
+// degree 40, 1.47 -> 0.81 ms.  Not where there are longer rows, whose items then queue behind each other in one
+// wave (groups of 8 / single items, ms: RMAT s17 1.83 / 1.57, s18 3.15 / 2.55, s19 5.4 / 4.6, s21 20.8 / 20.2; Chung-Lu of 300 thousand
+// vertices 6.7 / 5.1, of gamma 2.5 and mean degree 150 12.0 / 10.0), unless there are so many rows that the tickets count
+// again (kSupMany: Chung-Lu of 1M vertices 12.9 / 12.6, 2.5M 25.0 / 26.8, 3M 28.2 / 30.6, RMAT s22 43.7 / 43.0, s23 92 / 92).  Eight waves per workgroup; four were
+// no faster (s21 18.7 / 17.6 with groups).
+static constexpr uint32_t kSupHeads = 8, kSupHeadStride = 32, kSupMaxGroup = 8, kSupShort = 64, kSupMany = 3u << 19;
+static constexpr uint32_t kSupHasLong = 2 * kSupHeads * kSupHeadStride;  // this word: a row is longer than kSupShort
+static constexpr uint32_t kSupTicketWords = kSupHasLong + 1;
 
 // Items per row, group rows and wave rows counted apart.
 __global__ void k_sup_items(const uint64_t *__restrict__ off, const uint64_t *__restrict__ in_off, uint32_t n_rows,
                             uint32_t n_owned, uint32_t wave_tile, uint32_t *__restrict__ items_g,
-                            uint32_t *__restrict__ items_w) {
+                            uint32_t *__restrict__ items_w, uint32_t *__restrict__ ticket) {
+    bool has_long = false;
     for (uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; r < n_rows; r += (uint64_t)gridDim.x * blockDim.x) {
         const uint64_t K = off[r + 1] - off[r], kb = in_off[r + 1] - in_off[r];
         const uint32_t nb = (uint32_t)((kb + kSupChunk - 1) / kSupChunk);
@@ -467,7 +472,9 @@ __global__ void k_sup_items(const uint64_t *__restrict__ off, const uint64_t *__
         const uint32_t it = K == 0 ? 0u : (nb > a ? nb : a);
         items_g[r] = K > wave_tile ? it : 0u;
         items_w[r] = K > wave_tile ? 0u : it;
+        has_long |= K > kSupShort;
     }
+    if (__syncthreads_or(has_long) && threadIdx.x == 0) ticket[kSupHasLong] = 1;
 }
 
 // item_row[t]: group items at [0, n_g), wave items at n_g + [0, n_w).
@@ -533,13 +540,14 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 8 : 4) void k_support_spli
         }
     }
     const SupTab Q = sup_wave_tab(L, wv);
+    const uint32_t most = ticket[kSupHasLong] && n_rows < kSupMany ? 1u : kSupMaxGroup;
     const uint32_t share = gridDim.x * WAVES / kSupHeads * 4;  // a quarter of what is left per wave of the class
     for (uint32_t c = 0; c < kSupHeads; ++c) {  // wave items (every wave leaves once the items are taken)
         const uint32_t x = (blockIdx.x + c) % kSupHeads;
         const uint32_t n_x = n_w > x ? (n_w - x - 1) / kSupHeads + 1 : 0u;  // the class's items x, x + 8, ...
         uint32_t *head = ticket + (kSupHeads + x) * kSupHeadStride;
         for (uint32_t seen = c ? read_lane(sup_head(head), 0) : 0u; seen < n_x;) {
-            const uint32_t g = max(1u, min(kSupMaxGroup, (n_x - seen) / share));
+            const uint32_t g = max(1u, min(most, (n_x - seen) / share));
             uint32_t h = 0;
             if (lane == 0) h = atomicAdd(head, g);
             h = read_lane(h, 0);
@@ -570,7 +578,7 @@ static SupLayout sup_layout(void *ws, size_t ws_bytes, uint32_t n_rows, uint64_t
     L.off_g = c.take<uint64_t>((size_t)n_rows + 1);
     L.off_w = c.take<uint64_t>((size_t)n_rows + 1);
     L.item_row = c.take<uint32_t>(2 * (size_t)n_rows + m / kSupChunk + 1);
-    L.ticket = c.take<uint32_t>(2 * kSupHeads * kSupHeadStride);
+    L.ticket = c.take<uint32_t>(kSupTicketWords);
     L.scan_bytes = scan_ws_bytes((uint64_t)n_rows + 1);
     L.scan_ws = c.take<char>(L.scan_bytes);
     L.bytes = c.need();
@@ -640,15 +648,15 @@ extern "C" lstc_status lstc_triangle_support_split(const uint64_t *d_off, const 
     if (d_per_vertex && n_rows) LSTC_TRY(fill_u64(d_per_vertex, 0, n_rows, st));
     if (n_rows == 0 || m == 0) return LSTC_OK;
     const uint32_t grid_n = (uint32_t)hmin<uint64_t>(((uint64_t)n_rows + 255) / 256, (uint64_t)device_cus() * 16);
+    LSTC_TRY(fill_u32(L.ticket, 0, kSupTicketWords, st));
     hipLaunchKernelGGL(k_sup_items, dim3(grid_n), dim3(256), 0, st, d_off, d_in_off, n_rows, n_owned,
-                       sup_wave_tile<kSupSplitWaves>(), L.items_g, L.items_w);
+                       sup_wave_tile<kSupSplitWaves>(), L.items_g, L.items_w, L.ticket);
     LSTC_LAUNCHED("k_sup_items");
     LSTC_TRY(scan_exclusive_u32_to_u64(L.items_g, L.off_g, n_rows, L.off_g + n_rows, L.scan_ws, L.scan_bytes, st));
     LSTC_TRY(scan_exclusive_u32_to_u64(L.items_w, L.off_w, n_rows, L.off_w + n_rows, L.scan_ws, L.scan_bytes, st));
     hipLaunchKernelGGL(k_sup_item_rows, dim3(grid_n), dim3(256), 0, st, L.items_g, L.items_w, L.off_g, L.off_w,
                        n_rows, L.item_row);
     LSTC_LAUNCHED("k_sup_item_rows");
-    LSTC_TRY(fill_u32(L.ticket, 0, 2 * kSupHeads * kSupHeadStride, st));
     const uint32_t grid = (uint32_t)device_cus() * 4;  // persistent: four workgroups per CU (LDS)
     if (m < (1ull << 30))  // column positions as 32-bit byte offsets
         hipLaunchKernelGGL((k_support_split<true, kSupSplitWaves>), dim3(grid), dim3(kSupSplitWaves * 64), 0, st, d_off,
