@@ -429,7 +429,7 @@ __global__ __launch_bounds__(256) void k_hub_short(GraphDev G, HubSet hs) {
 // loads) come in by lane at once.
 __global__ __launch_bounds__(256) void k_hub_long(GraphDev G, HubSet hs) {
     constexpr uint32_t kRegs = 8, kStep = 64 * kRegs, kBatch = 8;
-    __shared__ __align__(8) uint32_t s_word[4][kTopWords];
+    __shared__ uint32_t s_word[4][kTopWords];
     if (!sload(hs.hctl + HC_ON)) return;
     const uint32_t lane = threadIdx.x & 63, wv = uniform(threadIdx.x >> 6);
     uint32_t *word = s_word[wv];
@@ -497,7 +497,7 @@ __global__ __launch_bounds__(256) void k_hub_long(GraphDev G, HubSet hs) {
         }
         if (lane < ((0u - nh) & 3u)) codes[ph + lane] = (uint16_t)kNoCode;
         if (lane == 0 && (nt & 1u)) tails[pt] = kTailPad;
-        if (bm) hs.units[first - kTopUnits + lane] = *(const uint64_t *)(word + 2 * lane);
+        if (bm) hs.units[first - kTopUnits + lane] = (uint64_t)word[2 * lane + 1] << 32 | word[2 * lane];
         if (lane == 0) hs.rec[r] = make_rec(first, units, (nt + 1) / 2, bm ? 1u : 0u);
       }
     }

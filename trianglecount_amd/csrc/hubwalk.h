@@ -103,7 +103,10 @@ __device__ __forceinline__ void hub_insert(const HubItem &it, HubAhead &a, const
                                            uint32_t lane) {
 #pragma unroll
     for (uint32_t i = 0; i < kHubWords / 256; ++i) ((uint4 *)s.bits)[64 * i + lane] = uint4{0, 0, 0, 0};
-    if (it.row.bitmap) *(uint64_t *)(s.bits + 2 * lane) = a.top;  // (the row's codes are all behind the top hubs then)
+    if (it.row.bitmap) {  // (the row's codes are all behind the top hubs then)
+        s.bits[2 * lane] = (uint32_t)a.top;
+        s.bits[2 * lane + 1] = (uint32_t)(a.top >> 32);
+    }
     set_codes(s.bits, a.codes);
     for (uint32_t u = 64 + lane; u < it.row.units; u += 64) set_codes(s.bits, gload(units + it.row.start + u));
     if (it.row.tail == 0) return;
