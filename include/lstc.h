@@ -217,8 +217,8 @@ typedef struct lstc_tune {
  * by the call, which the count then reads instead of the ids if the call finds that
  * this pays (lstc_count without d_per_row from 6 * 2^20 arcs on; lstc_count_split with segment words,
  * lstc_count_split_stream).  A workspace without room for them is accepted as
- * long as it holds the engine's queue; the count then reads the ids.  Of the tune
- * only tiny_max reaches the count from codes.                                  */
+ * long as it holds the engine's queue; the count then reads the ids.  The tune is
+ * that of a count from ids; one from codes takes nothing from it.              */
 lstc_status lstc_count_workspace(uint32_t n_rows, uint32_t n_owned, uint64_t m,
                                  const lstc_tune *tune, size_t *bytes);
 lstc_status lstc_count(const uint64_t *d_off, const uint32_t *d_col, uint32_t n_rows,
@@ -437,8 +437,9 @@ lstc_status lstc_timing_read(double *kernel_ms, uint64_t *launches);
  * (src/WithoutPartition/ShareKernelTCV62_update_v1.cu:8-9, src/profiling/occup_*.txt).
  * lstc_autotune times candidate lstc_tune values on the caller's batch
  * (coordinate descent, hipEvents, `reps` launches each) and returns the fastest;
- * every candidate must reproduce the default counts exactly.  It allocates its
- * own scratch and synchronises the stream.  The cache is a TSV of
+ * every candidate must reproduce the default counts exactly.  Counts from ids are
+ * timed, also of a graph that lstc_count would count from codes: the knobs are
+ * theirs.  It allocates its own scratch and synchronises the stream.  The cache is a TSV of
  * (device, shape class, knobs, ms); the last matching line wins.              */
 lstc_status lstc_shape_class(const lstc_graph_desc *graphs, uint32_t G, uint32_t *shape_class);
 /* The tuning a launch over these graphs runs with: defaults filled in, ranges

@@ -32,3 +32,19 @@ def test_autotune_keeps_counts_and_caches(lstc, oracle, tmp_path):
     assert hit2 and ms2 is None and t2.as_dict() == d
     # another shape class misses the cache
     assert lstc.shape_class(gs[:1]) != lstc.shape_class(gs)
+
+
+def test_autotune_times_counts_from_ids(lstc):
+    """The knobs are those of the count from ids; one of this graph from codes takes half its time."""
+    import torch
+    g = lstc.clean_orient(*lstc.generate_rmat(21, 16, seed=1))
+    ws, out = lstc.Workspace(), torch.zeros(1, dtype=torch.int64, device="cuda")
+    lstc.count(g, ws=ws, out=out)
+    assert lstc.count_path(g, ws) == 7
+    e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+    e[0].record()
+    for _ in range(5):
+        lstc.count(g, ws=ws, out=out, sync=False)
+    e[1].record()
+    torch.cuda.synchronize()
+    assert lstc.autotune([g], reps=2)[1] > 1.4 * e[0].elapsed_time(e[1]) / 5

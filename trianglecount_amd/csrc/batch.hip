@@ -53,8 +53,8 @@ static uint64_t arcs_total(const lstc_graph_desc *graphs, uint32_t G) {
 }
 
 // The engine's workspace: only a launch over one graph can count from codes.
-static size_t engine_bytes(uint32_t G, uint64_t rows, uint64_t m) {
-    return G == 1 ? count_ws_bytes(rows, m) : count_ws_base(rows, m);
+static size_t engine_bytes(uint32_t G, uint64_t rows, uint64_t m, bool codes = true) {
+    return G == 1 && codes ? count_ws_bytes(rows, m) : count_ws_base(rows, m);
 }
 
 static size_t table_bytes(uint32_t G) {
@@ -124,6 +124,11 @@ extern "C" lstc_status lstc_count_batch(const lstc_graph_desc *graphs, uint32_t 
 
 extern "C" lstc_status lstc_batch_plan_create(const lstc_graph_desc *graphs, uint32_t G, const lstc_tune *tune,
                                               lstc_batch_plan **out) {
+    return plan_create(graphs, G, tune, true, out);
+}
+
+lstc_status lstc::plan_create(const lstc_graph_desc *graphs, uint32_t G, const lstc_tune *tune, bool codes,
+                              lstc_batch_plan **out) {
     if (!out) return fail(LSTC_ERR_INVALID, "lstc_batch_plan_create: NULL out");
     *out = nullptr;
     if (G == 0) return fail(LSTC_ERR_INVALID, "lstc_batch_plan_create: empty batch");
@@ -135,7 +140,7 @@ extern "C" lstc_status lstc_batch_plan_create(const lstc_graph_desc *graphs, uin
     p->G = G;
     if (tune) { p->tune = *tune; p->has_tune = true; }
     const size_t tb = table_bytes(G);
-    p->ws_bytes = engine_bytes(G, base[G], arcs_total(graphs, G));
+    p->ws_bytes = engine_bytes(G, base[G], arcs_total(graphs, G), codes);
     p->dbytes = tb + p->ws_bytes;
     hipError_t e = hipMalloc(&p->dmem, p->dbytes);
     if (e != hipSuccess) { delete p; return fail(LSTC_ERR_OOM, "lstc_batch_plan_create: hipMalloc(%zu) failed", p->dbytes); }

@@ -114,6 +114,10 @@ lstc_status count_launch(const HostGraph *hosts, uint32_t G, const GraphDev *d_t
                          unsigned long long *d_counts, const lstc_tune *tune, void *ws, size_t ws_bytes,
                          hipStream_t st, bool timed = true);
 
+// lstc_batch_plan_create; without `codes` a plan of one graph has no room for them and reads ids (batch.hip).
+lstc_status plan_create(const lstc_graph_desc *graphs, uint32_t G, const lstc_tune *tune, bool codes,
+                        lstc_batch_plan **out);
+
 // lstc_count_path.
 lstc_status count_path(uint32_t n_rows, uint32_t n_owned, uint64_t m, bool split, void *ws, size_t ws_bytes,
                        hipStream_t st, uint32_t *path);

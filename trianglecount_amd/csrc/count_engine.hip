@@ -302,7 +302,7 @@ __device__ __forceinline__ RowPlan plan_row(const GraphSet &gs, const Bounds &bd
 template <int PASS>
 __global__ __launch_bounds__(256) void k_plan_rows(GraphSet gs, Bounds bd, uint32_t *__restrict__ wcnt,
                                                    unsigned long long *__restrict__ queue, HubSet hs) {
-    if (hs.hctl && sload(hs.hctl + HC_ON)) return hub_plan_rows<PASS>(gs.one, hs, bd.tiny_max);
+    if (hs.hctl && sload(hs.hctl + HC_ON)) return hub_plan_rows<PASS>(gs.one, hs);
     const uint32_t lane = lane_id();
     const uint32_t wave = blockIdx.x * 4 + (threadIdx.x >> 6);
     const uint64_t total = gs.total_rows;

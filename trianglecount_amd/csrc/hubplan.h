@@ -10,9 +10,11 @@ namespace lstc {
 // (heavy rows often lie together: 325 -> 64 us at RMAT s23 for the writing pass
 // against contiguous ranges): pass 0 counts its items per queue region,
 // hub_plan_scan turns that into positions, pass 1 writes the items.  Lane s keeps
-// the counter of region s.
+// the counter of region s.  Tiny rows are those of up to kTinyMax entries whatever the
+// tune says (limits of 8, 4 and none, ms a call: RMAT s21 2.15, 2.25, 2.36, s23 10.26, 10.54, 11.05, where ids
+// are fastest with 4).
 template <int PASS>
-__device__ __forceinline__ void hub_plan_rows(const GraphDev &G, const HubSet &hs, uint32_t tiny_max) {
+__device__ __forceinline__ void hub_plan_rows(const GraphDev &G, const HubSet &hs) {
     if (blockIdx.x * 4 >= hs.plan_waves) return;
     const uint32_t lane = threadIdx.x & 63, wave = blockIdx.x * 4 + (threadIdx.x >> 6);
     const uint64_t end = G.n_rows;
@@ -27,7 +29,7 @@ __device__ __forceinline__ void hub_plan_rows(const GraphDev &G, const HubSet &h
             const uint32_t k = (uint32_t)(gload(G.off + r + 1) - gload(G.off + r));
             const uint32_t kb = G.in_off ? (uint32_t)(gload(G.in_off + r + 1) - gload(G.in_off + r)) : 0u;
             in_only = r >= G.n_owned;
-            tiny = G.in_off && k >= 2 && k <= tiny_max;
+            tiny = G.in_off && k >= 2 && k <= kTinyMax;
             n = k < 2 ? 0u : (in_only ? 0u : k) + kb;
         }
         for (uint64_t heavy = ballot(n >= kHeavy); heavy; heavy &= heavy - 1) {

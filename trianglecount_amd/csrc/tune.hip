@@ -7,7 +7,10 @@
 // descent from the defaults, one knob at a time over its candidate values, each
 // candidate timed with hipEvents over `reps` launches after a warm-up.  Every
 // candidate must reproduce the default's counts exactly, otherwise the search
-// stops with LSTC_ERR_INVALID (a knob may change speed, never results).
+// stops with LSTC_ERR_INVALID (a knob may change speed, never results).  One
+// graph is counted from ids here, whatever a count of it would read: the knobs are
+// those of that kernel, and the winner also goes to graphs of its class that read ids
+// (timed from codes, the knobs change nothing and noise picks one).
 // Winners are cached in a TSV keyed by (device, shape class).
 #include <math.h>
 #include <stdio.h>
@@ -94,7 +97,7 @@ extern "C" lstc_status lstc_autotune(const lstc_graph_desc *graphs, uint32_t G, 
 
     auto measure = [&](const lstc_tune &t, double *ms, std::vector<unsigned long long> &counts) -> lstc_status {
         if (plan) { lstc_batch_plan_destroy(plan); plan = nullptr; }
-        LSTC_TRY(lstc_batch_plan_create(graphs, G, &t, &plan));
+        LSTC_TRY(plan_create(graphs, G, &t, /*codes=*/false, &plan));
         LSTC_TRY(lstc_batch_plan_run(plan, (uint64_t *)d_counts, st));  // warm-up
         LSTC_HIP(hipEventRecord(e0, st));
         for (uint32_t r = 0; r < reps; ++r) LSTC_TRY(lstc_batch_plan_run(plan, (uint64_t *)d_counts, st));
