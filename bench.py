@@ -17,8 +17,10 @@ Prints one JSON line.
 from __future__ import annotations
 
 import argparse
+import hashlib
 import json
 import os
+import re
 import sys
 import time
 
@@ -47,19 +49,34 @@ def merge_model_bytes(st):
     return 8 * (st["n"] + 1) + 4 * st["m"] + 16 * st["m"] + 4 * (st["sum_out_sq"] + st["sum_in_out"])
 
 
-def committed_traffic(scale):
+# what the count kernels are built from
+KERNEL_SOURCES = ("count_engine.h", "count_engine.hip", "hubcode.h", "hubcode.hip", "hubplan.h", "hubwalk.h", "segwalk.h",
+                  "wave.h")
+
+
+def kernel_state():
+    """A digest of the count kernels' sources, comments and spacing left out."""
+    h = hashlib.sha256()
+    for name in KERNEL_SOURCES:
+        with open(os.path.join(ROOT, "trianglecount_amd", "csrc", name)) as f:
+            h.update("".join(re.sub(r"//[^\n]*", "", f.read()).split()).encode())
+    return h.hexdigest()[:16]
+
+
+def committed_traffic(scale, kernel, root=None):
     """HBM-side bytes per count-kernel launch from the committed rocprofv3 PMC summary of this
     workload (profiles/k_count_rmat_s<scale>_pmc.txt: FETCH_SIZE and WRITE_SIZE per dispatch,
-    each scaled by what the counter reads for a known-size copy kernel in the same run), or None."""
-    p = os.path.join(ROOT, "profiles", f"k_count_rmat_s{scale}_pmc.txt")
+    each scaled by what the counter reads for a known-size copy kernel in the same run), or None:
+    also if the summary is another kernel's, or was taken from other sources than these."""
+    p = os.path.join(root or ROOT, "profiles", f"k_count_rmat_s{scale}_pmc.txt")
     try:
         with open(p) as f:
-            for line in f:
-                if line.startswith("traffic_bytes_per_launch:"):
-                    return int(line.split(":", 1)[1]), os.path.relpath(p, ROOT)
+            said = dict(ln.rstrip("\n").split(": ", 1) for ln in f if re.match(r"[a-z_]+: \S+$", ln))
     except OSError:
-        pass
-    return None, None
+        return None, None
+    if said.get("kernel") != kernel or said.get("kernel_state") != kernel_state() or "traffic_bytes_per_launch" not in said:
+        return None, None
+    return int(said["traffic_bytes_per_launch"]), os.path.relpath(p, root or ROOT)
 
 
 def timed_counts(T, g, steps, warmup, stream, ws, split=True):
@@ -496,6 +513,7 @@ def main():
         sys.exit(2)
     import torch
     import trianglecount_amd as T
+    from trianglecount_amd._lib import LSTC_PATH_CODES
     from trianglecount_amd import workloads as W
     T.load()
     torch.cuda.set_device(0)
@@ -541,6 +559,7 @@ def main():
     log(f"rmat s{args.scale}: n={g.n} m={g.m} max d+={st['max_out']} gen {t_gen:.2f}s prep {t_prep*1e3:.1f} ms")
 
     tri, ms, kern_ms, wall = timed_counts(T, g, args.steps, args.warmup, stream, ws)
+    from_codes = bool(T.count_path(g, ws) & LSTC_PATH_CODES)
     work = T.work_stats([g], ws=ws)[0]
     tri_plain, ms_plain = tri, None
     inl_ms = None
@@ -565,13 +584,14 @@ def main():
         raise SystemExit(f"count {tri} differs from the oracle's {gold['triangles']}")
     gteps = g.m / (ms / 1e3) / 1e9
     mm = merge_model_bytes(st)
-    traffic, traffic_src = committed_traffic(args.scale)
-    # bytes the count kernel moves: measured (profiles/) where this workload has a profile; otherwise
-    # the id-list model, an upper bound for a count that reads 16-bit codes
-    moved = traffic or work["bytes"]
-    achieved = moved / (kern_ms / 1e3) / 1e9
-    log(f"count {tri} in {ms:.3f} ms/step (kernel {kern_ms:.3f} ms) -> {gteps:.3f} GTEPS; "
-        f"{moved/1e9:.1f} GB -> {achieved:.0f} GB/s")
+    kernel = "k_count_hub" if from_codes else "k_count"
+    traffic, traffic_src = committed_traffic(args.scale, kernel)
+    # bytes the count kernel moves: measured (profiles/) where this workload has a profile of these sources; otherwise
+    # those of the id-list model, for a count that reads ids
+    moved = traffic or (None if from_codes else work["bytes"])
+    achieved = moved and moved / (kern_ms / 1e3) / 1e9
+    log(f"count {tri} in {ms:.3f} ms/step (kernel {kern_ms:.3f} ms) -> {gteps:.3f} GTEPS"
+        + (f"; {moved/1e9:.1f} GB -> {achieved:.0f} GB/s" if moved else ""))
 
     extra = {}
     legs = set() if args.no_extra else {x for x in args.legs.split(",") if x}
@@ -638,14 +658,15 @@ def main():
                                   "(lstc_clean_orient_stream), one synchronisation",
                    "symmetric_prep_ms": t_sym and round(t_sym * 1e3, 2),
                    "end_to_end_gteps": round(g.m / (t_prep + ms / 1e3) / 1e9, 4),
-                   "count_mode": "split, rows as 16-bit hub codes built in every step (lstc_count_split_stream)",
+                   "count_mode": ("split, rows as 16-bit hub codes built in every step" if from_codes else
+                                  "split, ids from the row-aligned copy") + " (lstc_count_split_stream)",
                    "in_lists_from_bare_csr_ms": inl_ms and round(inl_ms, 3),
                    "plain_csr_count_ms": ms_plain and round(ms_plain, 4),
                    "plain_csr_gteps": ms_plain and round(g.m / (ms_plain / 1e3) / 1e9, 4)},
-        "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
-                     "kernel": "k_count_hub", "kernel_ms": round(kern_ms, 4),
-                     "achieved_from": "measured traffic" if traffic else "id-list model",
+        "roofline": {"bound": "hbm", "achieved": achieved and round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                     "frac": achieved and round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
+                     "kernel": kernel, "kernel_ms": round(kern_ms, 4),
+                     "achieved_from": "measured traffic" if traffic else "id-list model" if moved else None,
                      "id_list_model_bytes": work["bytes"], "work": work,
                      "traffic_source": traffic_src,
                      "merge_model_bytes": mm, "merge_model_gbs": round(mm / (kern_ms / 1e3) / 1e9, 1)},

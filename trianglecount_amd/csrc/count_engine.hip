@@ -983,8 +983,8 @@ __global__ __launch_bounds__(WAVES * 64, UNROLL == 4 ? 8 : 6) void k_count(Graph
 }
 
 // ------------------------------------------------------------------ hub count kernel
-// The split count over hub codes (hubcode.h): every item is one wave's, one wave per
-// workgroup (9.1 KB of LDS: 16 waves per CU).
+// The count over hub codes (hubcode.h), with in-lists (SPLIT) or without: every item is
+// one wave's, one wave per workgroup (9.1 KB of LDS: 16 waves per CU).
 //
 // What bounds it (RMAT s23, 8.8 ms; k_count took 16.9): the fabric behind the L2,
 // which delivers 7.2-7.8 TB/s here wherever the lines come from, so bytes and L2

@@ -97,7 +97,7 @@ struct HubSet {
     uint32_t *cnt;        // per row: occurrences in the sample
     uint16_t *code;       // per row: its vertex's code
     uint64_t *rec;        // per row
-    uint32_t *long_rows;  // rows of at least kTopMin entries
+    uint32_t *long_rows;  // rows of at least kLongRow entries
     uint64_t *units;
     uint32_t *plan_cnt;   // [kHubSlots][plan_waves]
     uint32_t plan_waves;

@@ -17,64 +17,75 @@ namespace lstc {
 // Sampled entries (RMAT s23, ms a count: 11.1 with 2^20, 10.7 with 2^21, 10.8 with
 // 2^22), and at most one in 16: the hubs' counters are hot addresses.
 static constexpr uint64_t kSamples = 2u << 20, kMinStride = 16;
-// When codes pay.  What they save is in proportion to what is streamed: per arc of the owned
-// rows, with in-lists, at most the smaller of the mean d+ of its two ends' rows (`from` and `to`,
-// each a mean over arcs), without in-lists its target's row.  What they cost, the build, is in
-// proportion to all arcs; so the lines below are on these means times the owned rows' share of the arcs.
+// When codes pay.  What they save is in proportion to what is streamed: per arc of the
+// owned rows, with in-lists at most the smaller of the mean d+ of its two ends' rows
+// (`from` and `to`, each a mean over arcs), without in-lists its target's row.  What they
+// cost, the build, is in proportion to all arcs; so these means count times the owned
+// rows' share of the arcs.  Three decisions:
+//   hub_worth       on the host, by the sizes;
+//   worth_sampling  before the sample, by the row lengths (a graph that it refuses has
+//                   cost 0.02 to 0.04 ms; refused after the sample, 0.1 to 0.3 ms);
+//   k_hub_pick      after it, with `to`, the share c of the columns that hubs cover, and
+//                   the share of tails in what would be streamed.
+// The figures are ms a call from ids / from codes (CL: Chung-Lu graphs of the gamma, mean
+// degree and number of vertices; ER: uniform graphs of the vertices and mean degree).
 //
-// 1. Before the sample (worth_sampling), from the row lengths alone.  Found out here, a graph
-// costs 0.02 to 0.04 ms, after the sample 0.1 to 0.3 ms.
-// 2. After it (k_hub_pick), with `to`, the share c of the columns that hubs cover, and the
-// tails' share of what would be streamed.
-// Figures: ms a call from ids / from codes.
-//
-// With in-lists, from on: RMAT s17 90 0.338 / 0.273, s18 109 0.428 / 0.403, s21 189 3.14 / 2.15, s23 270
-// 16.9 / 10.3; Chung-Lu graphs (gamma 2.1, mean degree 50) of 300 thousand vertices 65 0.594 / 0.638,
-// 1M 84 1.70 / 1.85, 1.5M 92 2.63 / 2.72, 2M 96 3.57 / 3.59, 3M 103 5.59 / 5.39; gamma 2.3, mean 150, 300
-// thousand vertices 104 1.57 / 1.45, gamma 2.5 84 1.47 / 1.54.  The line rises with the vertices, of which the hubs
-// are a smaller part.  Without in-lists: gamma 2.3, mean 50, 1M vertices 43 1.61 / 1.79, 2M 45 3.67 / 3.43, 3M 47
-// 6.01 / 5.29; 2.1, 300 thousand 65 0.568 / 0.605, 500 thousand 73 1.03 / 0.94; gamma 2.5, mean 150, 300 thousand
-// 84 1.58 / 1.39, 1M 87 6.80 / 5.19.
-// Below 5.5M arcs ids wait for the items of the largest hubs, which codes cut into parts: gamma 2.1, 80 thousand
-// vertices 47 0.40 / 0.32, 110 thousand 51 0.32 / 0.34, 150 thousand 55 0.41 / 0.39, 230 thousand 61 0.52 / 0.52, 260 thousand 63 0.53 / 0.56.
+// worth_sampling with in-lists, `from`:
+//   RMAT s18 109 0.428 / 0.403, s21 189 3.14 / 2.15, s23 270 16.9 / 10.3
+//   CL 2.1, 50: 300K 65 0.594 / 0.638, 1M 84 1.70 / 1.85, 2M 96 3.57 / 3.59, 3M 103 5.59 / 5.39
+//   CL 2.3, 150, 300K 104 1.57 / 1.45; CL 2.5, 150, 300K 84 1.47 / 1.54
+// The line rises with the vertices, of which the hubs are a smaller part.  Below kSmall
+// arcs ids wait for the items of the largest hubs, which codes cut into parts:
+//   RMAT s17 90 0.338 / 0.273; CL 2.1, 50: 80K 47 0.40 / 0.32, 110K 51 0.32 / 0.34,
+//   150K 55 0.41 / 0.39, 230K 61 0.52 / 0.52, 260K (5.9M arcs) 63 0.53 / 0.56
 static constexpr double kMinFrom = 86, kMinFromMore = 14, kMinFromRows = 1 << 21;  // 86 to 100
 static constexpr double kMinFromSmall = 44;
-static constexpr uint64_t kSmall = 11ull << 19;  // arcs below which this holds
+static constexpr uint64_t kSmall = 11ull << 19;
+// Without in-lists; from kBigPlain arcs on ids no longer stream from the caches:
+//   CL 2.1, 50: 300K 65 0.568 / 0.605, 500K 73 1.03 / 0.94; CL 2.5, 150, 300K 84 1.58 / 1.39
+//   CL 2.3, 50: 1M (25M arcs) 43 1.61 / 1.79, 2M 45 3.67 / 3.43, 3M 47 6.01 / 5.29
 static constexpr double kMinFromPlain = 70, kMinFromPlainBig = 45;
-static constexpr uint64_t kBigPlain = 1ull << 25;  // arcs from which the second holds
-// Owned rows: a part of RMAT s21 in two, from times share 95, 1.77 / 1.47, in eight 25 0.68 / 0.78; of s23 in eight 35
-// 2.80 / 2.80, in 32 10 1.46 / 1.69.  Without in-lists `from` says less, and a smaller share pays: s23, the first 3% of the
-// rows (a seventh of the count) 5.27 / 2.99, 0.3% 1.51 / 1.90.
+static constexpr uint64_t kBigPlain = 1ull << 25;
+// Parts, `from` times the share with in-lists: RMAT s21 in two 95 1.77 / 1.47, in eight 25
+// 0.65 / 0.78, s23 in eight 35 2.72 / 2.80, in 32 10 1.23 / 1.69.  Without them:
+// s23 in eight 35 4.79 / 3.03, in 32 10 1.54 / 1.64.
 static constexpr double kMinFromOwnedPlain = 12;
-// Below this many arcs of owned rows (by the rows' share; decided on the host) a count of a part
-// is over before a build pays, or before the launches are that find it out: s21 in eight 6.3M 0.68 / 0.78, in 32 2.6M
-// 0.36 / 0.51; one row of s23 0.04 / 1.42.
+// Below this many arcs of owned rows (by the rows' share) a part's count is over before
+// a build pays, or before the launches that would find it out: s21 in eight, 6.3M,
+// 0.65 / 0.78 with in-lists; in 32, 2.6M, 0.31 / 0.51, and 0.36 / 0.56 without; the first
+// row of s23 alone 0.01 / 1.42.
 static constexpr double kMinOwned = 12 << 20, kMinOwnedPlain = 3 << 20;
-// Uniform graphs: where neither degree nor order of the vertices means anything, d+ runs evenly from 0 to
-// twice its mean, and the mean over arcs is 4/3 of that (1.25 to 1.32 measured with mean degrees of 40 to
-// 1800; power laws of gamma 2.5 1.14 to 1.22, 2.3 1.4 and more, RMAT 3 and more).  A count of them from ids is fast (every list is
-// short), and without hubs the codes cover what their number covers: from 105 thousand vertices on the tails cost
-// more than the codes save (115 thousand, mean degree 400, 1.93 / 2.14; 130 thousand, 600, 4.4 / 7.7; 160 thousand, 400,
-// plain 3.0 / 5.5).  Below, by the sum of the squares of the row lengths: 2e8 20 thousand vertices, mean degree 200, 0.170 / 0.212,
-// 5e8 10 thousand, 400 (2M arcs) 0.230 / 0.281 and 40 thousand, 200 (4M) 0.306 / 0.293, 6e8 8 thousand, 500, 0.268 / 0.319, 7.6e8 60 thousand,
-// 200, 0.439 / 0.379, 1e9 4 thousand, 1000, 0.456 / 0.367; plain 1e9 80 thousand, 200, 0.450 / 0.467, 1.3e9 100 thousand, 200,
-// 0.603 / 0.619, 3e9 60 thousand, 400, 1.00 / 0.78.
-static constexpr double kUniformLow = 1.23, kUniformHigh = 1.4, kMinUniform = 7e8, kMinUniformPlain = 2e9;
-static constexpr double kMinUniformMore = 4.5e8;    // with in-lists, from
-static constexpr uint64_t kUniformMore = 7ull << 19;  // so many arcs on
+// Uniform graphs.  Where neither degree nor id means anything, d+ runs evenly from 0 to
+// twice its mean, and its mean over arcs is 4/3 of that (ER with mean degrees of 40 to 1800
+// 1.25 to 1.32; power laws of gamma 2.5 1.14 to 1.22, 2.3 from 1.4 on, RMAT from 2.8 on).
+// Ids are fast there, and without hubs the codes cover what their number covers:
+//   ER 100K, 400 1.70 / 1.53; 115K, 400 1.93 / 2.14; 130K, 600 4.4 / 7.7; 160K, 400, without in-lists 3.0 / 5.5
+// With fewer vertices, by the sum of the squares of the row lengths:
+//   with in-lists: 20K, 200 2e8 0.170 / 0.212; 10K, 400 (2M arcs) 5e8 0.230 / 0.281;
+//     40K, 200 (4M arcs) 5e8 0.306 / 0.293; 8K, 500 6e8 0.268 / 0.319; 60K, 200 8e8 0.439 / 0.379;
+//     4K, 1000 1e9 0.456 / 0.367
+//   without: 80K, 200 1e9 0.450 / 0.467; 100K, 200 1.3e9 0.603 / 0.619; 60K, 400 3e9 1.00 / 0.78
+static constexpr double kUniformLow = 1.23, kUniformHigh = 1.4;
 static constexpr uint32_t kMaxUniformRows = 105000;
-// After the sample, with in-lists: min(from, to) (2 c - 1) (3M vertices, gamma 2.1, 52 5.59 / 5.39; 2.5, mean 150, 1M 23
-// 4.73 / 5.72; with the target's row the shorter one, uniform graphs of 100 thousand, mean 200, 56 0.672 / 0.639).
-// Without: `to` (gamma 2.3, 1M vertices 111 1.61 / 1.79, 2M 128 3.67 / 3.43; RMAT of 6M arcs 131 0.541 / 0.589, which kMinFromPlain
-// keeps out), times the share for parts (s21 357: 17% of the count, 63 0.94 / 0.77, 10%, 36 0.53 / 0.72).  Either way half of the sample is covered.
-static constexpr double kMinWorth = 40, kMinWorthFlat = 50, kMinPlainLen = 120, kMinPlainLenOwned = 40;
+static constexpr double kMinUniform = 7e8, kMinUniformMore = 4.5e8, kMinUniformPlain = 2e9;
+static constexpr uint64_t kUniformMore = 7ull << 19;  // arcs from which kMinUniformMore holds
+// k_hub_pick with in-lists, min(from, to) (2 c - 1) times the share: CL 2.1, 50, 3M 52 5.59 /
+// 5.39; CL 2.5, 150, 1M 23 4.73 / 5.72; kMinWorthFlat where arcs point at the shorter rows: ER
+// 100K, 200 56 0.672 / 0.639.
+static constexpr double kMinWorth = 40, kMinWorthFlat = 50;
+// Without, `to`: CL 2.3, 50: 1M 111 1.61 / 1.79, 2M 128 3.67 / 3.43; times the share: s21 in
+// eight 47 0.88 / 0.75, s23 in eight 73 4.79 / 3.03, in 32 20 1.54 / 1.64.
+static constexpr double kMinPlainLen = 120, kMinPlainLenOwned = 40;
+// Either way hubs cover half of the sample at least.
 static constexpr uint32_t kCoverPct = 50;
-// Tails are walked at a quarter of the codes' speed.  Graphs whose arcs point at the longer rows hardly
-// stream any (without in-lists below 1% of the entries for gamma 2.1 and RMAT, 6% for gamma 2.5 and 1M vertices, 6.80 /
-// 5.19) and are not looked at for them (25 us); uniform graphs of 100 thousand vertices 3.3%, of 115 thousand 6.6%, of 130 thousand 10%.
+// Tails are walked at a quarter of the codes' speed.  They are measured (in 10 us) where arcs
+// point at the shorter rows: ER 100K 3.3% of the entries, 115K 6.6%, 130K 10%.  Graphs
+// whose arcs point at the longer rows hardly stream any (CL 2.1 and RMAT below 1%; CL
+// 2.5, 150, 1M 6%, without in-lists 6.80 / 5.19).
 static constexpr double kMaxTailShare = 0.08;
-// Smaller graphs and shorter rows keep ids: the build is worth 0.1 ms (RMAT s14 of 0.7M arcs 0.147 / 0.229).  Without
-// in-lists k_count has less to lose to (Chung-Lu of 3.3M arcs 0.261 / 0.377; RMAT s19, 7.7M arcs, 0.88 / 0.63).
+// Smaller graphs and shorter rows keep ids: the build is worth 0.1 ms (RMAT s14, 0.7M arcs,
+// 0.147 / 0.229).  Without in-lists ids have less to lose to (CL 2.1, 50, 150K, 3.3M arcs,
+// 0.261 / 0.377; RMAT s19, 7.7M arcs, 0.88 / 0.63).
 static constexpr uint64_t kMinArcs = 3ull << 19, kMinArcsPlain = 6ull << 20, kMinPerRow = 16;
 static constexpr uint64_t kArcSeed = 0x68756263;  // of the arcs that stand for all when the tails are measured
 static constexpr uint32_t kAbsent = 0xFFFFFFFFu;  // past the end of a row (ids are below 2^32 - 2)
@@ -102,11 +113,14 @@ __device__ __forceinline__ double owned_share(const GraphDev &G) {
 // Whether the graph may be worth codes, from the sum of the squares of its row lengths.
 __device__ __forceinline__ bool worth_sampling(const GraphDev &G, double squares, bool split) {
     const double arcs = (double)arcs_of(G), from = squares / arcs, share = owned_share(G), mean = arcs / G.n_rows;
-    if (from >= kUniformLow * mean && from <= kUniformHigh * mean)
-        return G.n_rows <= kMaxUniformRows &&
-               squares * share >= (!split ? kMinUniformPlain : arcs < (double)kUniformMore ? kMinUniform : kMinUniformMore);
-    if (split)
-        return from * share >= (arcs < (double)kSmall ? kMinFromSmall : kMinFrom + kMinFromMore * fmin(1., G.n_rows / kMinFromRows));
+    if (from >= kUniformLow * mean && from <= kUniformHigh * mean) {
+        const double line = !split ? kMinUniformPlain : arcs < (double)kUniformMore ? kMinUniform : kMinUniformMore;
+        return G.n_rows <= kMaxUniformRows && squares * share >= line;
+    }
+    if (split) {
+        const double large = kMinFrom + kMinFromMore * fmin(1., G.n_rows / kMinFromRows);
+        return from * share >= (arcs < (double)kSmall ? kMinFromSmall : large);
+    }
     return from >= (arcs >= (double)kBigPlain ? kMinFromPlainBig : kMinFromPlain) && from * share >= kMinFromOwnedPlain;
 }
 
@@ -137,8 +151,7 @@ __global__ __launch_bounds__(256) void k_hub_init(HubSet hs, const uint64_t *__r
 // A wave takes four chunks at a time; every fourth wave measures the rows of one of
 // them (in turn the first to the fourth, which lie a quarter of the columns apart in a graph of
 // up to 2^25 arcs): HC_LEN, the sum of their lengths, HC_LENS: how many.  It leaves
-// at once if the rows are too short for codes: the Chung-Lu graph of
-// 3M vertices and gamma 2.3 takes 4.48 ms then, 4.77 when the rule waits for the sample, 4.43 from ids.
+// at once if the row lengths speak against codes.
 __global__ __launch_bounds__(256) void k_hub_sample(GraphDev G, uint32_t stride, HubSet hs, uint32_t shares,
                                                     bool split) {
     constexpr uint32_t kPer = 4;
@@ -305,7 +318,8 @@ __global__ __launch_bounds__(256) void k_hub_pick(GraphDev G, const uint32_t *__
     const double cover = (double)covered / (double)all, share = owned_share(G);
     bool on = split ? fmin(from, to) * share * (2 * cover - 1) >= (to < from ? kMinWorthFlat : kMinWorth)
                     : to >= kMinPlainLen && to * share >= kMinPlainLenOwned;
-    if (on && to < from && n > kHubs) on = tail_share(G, cnt, cut, cut_n ? (double)(cut_n - rest) / cut_n : 1.) <= kMaxTailShare;
+    if (on && to < from && n > kHubs)
+        on = tail_share(G, cnt, cut, cut_n ? (double)(cut_n - rest) / cut_n : 1.) <= kMaxTailShare;
     if (b != 0) return;
     hctl[HC_CUT] = cut;
     hctl[HC_REST] = rest;
@@ -424,9 +438,9 @@ __global__ __launch_bounds__(256) void k_hub_short(GraphDev G, HubSet hs) {
     if (valid && !lng) hs.rec[r] = mine;
 }
 
-// A wave per long row, 512 entries in registers at a time (read twice if there
-// are more).  A tail of more than kMaxTail ids takes the launch back to k_count.  A wave takes kBatch rows together: their headers (four dependent
-// loads) come in by lane at once.
+// A wave per long row, 512 entries in registers at a time (read twice if there are more).  A tail of more than
+// kMaxTail ids takes the launch back to k_count.  A wave takes kBatch rows together: their headers (four
+// dependent loads) come in by lane at once.
 __global__ __launch_bounds__(256) void k_hub_long(GraphDev G, HubSet hs) {
     constexpr uint32_t kRegs = 8, kStep = 64 * kRegs, kBatch = 8;
     __shared__ uint32_t s_word[4][kTopWords];
@@ -437,76 +451,77 @@ __global__ __launch_bounds__(256) void k_hub_long(GraphDev G, HubSet hs) {
     uint16_t *codes = (uint16_t *)hs.units;
     uint32_t *tails = (uint32_t *)hs.units;
     for (uint32_t i0 = (blockIdx.x * 4 + wv) * kBatch; i0 < n_long; i0 += gridDim.x * 4 * kBatch) {
-      const uint32_t nb = min(kBatch, n_long - i0);
-      uint32_t l_row = 0, l_d = 0, l_start = 0;
-      uint64_t l_off = 0;
-      if (lane < nb) {
-          l_row = gload(hs.long_rows + i0 + lane);
-          l_off = gload(G.off + l_row);
-          l_d = (uint32_t)(gload(G.off + l_row + 1) - l_off);
-          l_start = block_of(l_row, l_off);
-      }
-      for (uint32_t ib = 0; ib < nb; ++ib) {
-        const uint32_t r = read_lane(l_row, ib), d = read_lane(l_d, ib), start = read_lane(l_start, ib);
-        const uint32_t *colr = G.col + read_lane64(l_off, ib);
-        uint32_t x[kRegs], c[kRegs];
-        auto fetch = [&](uint32_t p0) {
-#pragma unroll
-            for (uint32_t q = 0; q < kRegs; ++q) {
-                const uint32_t p = p0 + 64 * q + lane;
-                x[q] = kAbsent;
-                if (p < d) x[q] = gload(colr + p);
-            }
-#pragma unroll
-            for (uint32_t q = 0; q < kRegs; ++q) {
-                c[q] = kNoCode;
-                if (x[q] != kAbsent) c[q] = code_of(hs.code, G.n_rows, x[q]);
-            }
-        };
-        uint32_t top = 0, hub = 0;
-        for (uint32_t p0 = 0; p0 < d; p0 += kStep) {
-            fetch(p0);
-#pragma unroll
-            for (uint32_t q = 0; q < kRegs; ++q) {
-                top += (uint32_t)__popcll(ballot(c[q] < kTop));
-                hub += (uint32_t)__popcll(ballot(c[q] != kNoCode));
-            }
+        const uint32_t nb = min(kBatch, n_long - i0);
+        uint32_t l_row = 0, l_d = 0, l_start = 0;
+        uint64_t l_off = 0;
+        if (lane < nb) {
+            l_row = gload(hs.long_rows + i0 + lane);
+            l_off = gload(G.off + l_row);
+            l_d = (uint32_t)(gload(G.off + l_row + 1) - l_off);
+            l_start = block_of(l_row, l_off);
         }
-        const bool bm = top >= kTopMin;
-        const uint32_t floor = bm ? kTop : 0u;  // codes below go to the bitmap
-        const uint32_t nh = bm ? hub - top : hub, units = (nh + 3) / 4, nt = d - hub;
-        if (nt > kMaxTail && lane == 0) hs.hctl[HC_ON] = 0;  // (this launch's waves read it before their rows)
-        // from a 128-byte boundary: with a bitmap there is always room for that, else if there is
-        const uint32_t aligned = (start + 15u) & ~15u;
-        const bool fits = aligned - start + units + (nt + 1) / 2 <= (d + 1) / 2 + 1;
-        const uint32_t first = bm ? aligned + kTopUnits : fits ? aligned : start;
-        word[lane] = word[64 + lane] = 0;
-        uint32_t ph = first * 4, pt = (first + units) * 2;
-        for (uint32_t p0 = 0; p0 < d; p0 += kStep) {
-            if (d > kStep) fetch(p0);
+        for (uint32_t ib = 0; ib < nb; ++ib) {
+            const uint32_t r = read_lane(l_row, ib), d = read_lane(l_d, ib), start = read_lane(l_start, ib);
+            const uint32_t *colr = G.col + read_lane64(l_off, ib);
+            uint32_t x[kRegs], c[kRegs];
+            auto fetch = [&](uint32_t p0) {
 #pragma unroll
-            for (uint32_t q = 0; q < kRegs; ++q) {
-                const bool in = x[q] != kAbsent, h = c[q] != kNoCode && c[q] >= floor, t = in && c[q] == kNoCode;
-                const uint64_t hm = ballot(h), tm = ballot(t);
-                if (h) codes[ph + mask_rank(hm)] = (uint16_t)c[q];
-                else if (t) tails[pt + mask_rank(tm)] = x[q];
-                else if (in) atomicOr(&word[c[q] >> 5], 1u << (c[q] & 31u));
-                ph += (uint32_t)__popcll(hm);
-                pt += (uint32_t)__popcll(tm);
+                for (uint32_t q = 0; q < kRegs; ++q) {
+                    const uint32_t p = p0 + 64 * q + lane;
+                    x[q] = kAbsent;
+                    if (p < d) x[q] = gload(colr + p);
+                }
+#pragma unroll
+                for (uint32_t q = 0; q < kRegs; ++q) {
+                    c[q] = kNoCode;
+                    if (x[q] != kAbsent) c[q] = code_of(hs.code, G.n_rows, x[q]);
+                }
+            };
+            uint32_t top = 0, hub = 0;
+            for (uint32_t p0 = 0; p0 < d; p0 += kStep) {
+                fetch(p0);
+#pragma unroll
+                for (uint32_t q = 0; q < kRegs; ++q) {
+                    top += (uint32_t)__popcll(ballot(c[q] < kTop));
+                    hub += (uint32_t)__popcll(ballot(c[q] != kNoCode));
+                }
             }
+            const bool bm = top >= kTopMin;
+            const uint32_t floor = bm ? kTop : 0u;  // codes below go to the bitmap
+            const uint32_t nh = bm ? hub - top : hub, units = (nh + 3) / 4, nt = d - hub;
+            if (nt > kMaxTail && lane == 0) hs.hctl[HC_ON] = 0;  // (this launch's waves read it before their rows)
+            // from a 128-byte boundary: with a bitmap there is always room for that, else if there is
+            const uint32_t aligned = (start + 15u) & ~15u;
+            const bool fits = aligned - start + units + (nt + 1) / 2 <= (d + 1) / 2 + 1;
+            const uint32_t first = bm ? aligned + kTopUnits : fits ? aligned : start;
+            word[lane] = word[64 + lane] = 0;
+            uint32_t ph = first * 4, pt = (first + units) * 2;
+            for (uint32_t p0 = 0; p0 < d; p0 += kStep) {
+                if (d > kStep) fetch(p0);
+#pragma unroll
+                for (uint32_t q = 0; q < kRegs; ++q) {
+                    const bool in = x[q] != kAbsent, h = c[q] != kNoCode && c[q] >= floor, t = in && c[q] == kNoCode;
+                    const uint64_t hm = ballot(h), tm = ballot(t);
+                    if (h) codes[ph + mask_rank(hm)] = (uint16_t)c[q];
+                    else if (t) tails[pt + mask_rank(tm)] = x[q];
+                    else if (in) atomicOr(&word[c[q] >> 5], 1u << (c[q] & 31u));
+                    ph += (uint32_t)__popcll(hm);
+                    pt += (uint32_t)__popcll(tm);
+                }
+            }
+            if (lane < ((0u - nh) & 3u)) codes[ph + lane] = (uint16_t)kNoCode;
+            if (lane == 0 && (nt & 1u)) tails[pt] = kTailPad;
+            if (bm) hs.units[first - kTopUnits + lane] = (uint64_t)word[2 * lane + 1] << 32 | word[2 * lane];
+            if (lane == 0) hs.rec[r] = make_rec(first, units, (nt + 1) / 2, bm ? 1u : 0u);
         }
-        if (lane < ((0u - nh) & 3u)) codes[ph + lane] = (uint16_t)kNoCode;
-        if (lane == 0 && (nt & 1u)) tails[pt] = kTailPad;
-        if (bm) hs.units[first - kTopUnits + lane] = (uint64_t)word[2 * lane + 1] << 32 | word[2 * lane];
-        if (lane == 0) hs.rec[r] = make_rec(first, units, (nt + 1) / 2, bm ? 1u : 0u);
-      }
     }
 }
 
 static uint64_t hub_units(uint64_t rows, uint64_t m) { return m / 2 + 2 * rows + 64; }
 
 bool hub_fits(uint64_t rows, uint64_t m, bool split) {
-    return m >= (split ? kMinArcs : kMinArcsPlain) && m >= kMinPerRow * rows && rows < (1ull << 32) && hub_units(rows, m) < (1ull << 29);
+    return m >= (split ? kMinArcs : kMinArcsPlain) && m >= kMinPerRow * rows && rows < (1ull << 32) &&
+           hub_units(rows, m) < (1ull << 29);
 }
 
 bool hub_worth(uint64_t rows, uint64_t owned, uint64_t m, bool split) {

@@ -445,17 +445,16 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 8 : 4) void k_support(cons
 // (1024: RMAT s23 85 against 92 ms, but RMAT s19 6.0 against 5.7 and Chung-Lu of 300
 // thousand vertices 8.0 against 6.7, which wait for their longest items.)
 static constexpr uint32_t kSupChunk = 512;
-// Items are dealt in kSupHeads classes (item t to class t % kSupHeads), each with
-// its own head per kind on a line of its own; a workgroup starts with class blockIdx %
-// kSupHeads and goes on with the others' leftovers.  One head for all put a million
-// tickets on one address: RMAT s21 25.4 ms, now 20.2, RMAT s23 119 -> 92.
-// Where no row is longer than kSupShort, waves take up to kSupMaxGroup items at
-// once while many are left, one at the end: a uniform graph of 600 thousand vertices, mean
-// degree 40, 1.47 -> 0.81 ms.  Not where there are longer rows, whose items then queue behind each other in one
-// wave (groups of 8 / single items, ms: RMAT s17 1.83 / 1.57, s18 3.15 / 2.55, s19 5.4 / 4.6, s21 20.8 / 20.2; Chung-Lu of 300 thousand
-// vertices 6.7 / 5.1, of gamma 2.5 and mean degree 150 12.0 / 10.0), unless there are so many rows that the tickets count
-// again (kSupMany: Chung-Lu of 1M vertices 12.9 / 12.6, 2.5M 25.0 / 26.8, 3M 28.2 / 30.6, RMAT s22 43.7 / 43.0, s23 92 / 92).  Eight waves per workgroup; four were
-// no faster (s21 18.7 / 17.6 with groups).
+// Items are dealt in kSupHeads classes (item t to class t % kSupHeads), each with its own head per kind on a
+// line of its own; a workgroup starts with class blockIdx % kSupHeads and goes on with the others' leftovers.
+// One head for all put a million tickets on one address: RMAT s21 25.4 ms, now 20.2, RMAT s23 119 -> 92. Where
+// no row is longer than kSupShort, waves take up to kSupMaxGroup items at once while many are left, one at the
+// end: a uniform graph of 600 thousand vertices, mean degree 40, 1.47 -> 0.81 ms.  Not where there are longer
+// rows, whose items then queue behind each other in one wave (groups of 8 / single items, ms: RMAT s17 1.83 /
+// 1.57, s18 3.15 / 2.55, s19 5.4 / 4.6, s21 20.8 / 20.2; Chung-Lu of 300 thousand vertices 6.7 / 5.1, of gamma
+// 2.5 and mean degree 150 12.0 / 10.0), unless there are so many rows that the tickets count again (kSupMany:
+// Chung-Lu of 1M vertices 12.9 / 12.6, 2.5M 25.0 / 26.8, 3M 28.2 / 30.6, RMAT s22 43.7 / 43.0, s23 92 / 92).
+// Eight waves per workgroup; four were no faster (s21 18.7 / 17.6 with groups).
 static constexpr uint32_t kSupHeads = 8, kSupHeadStride = 32, kSupMaxGroup = 8, kSupShort = 64, kSupMany = 3u << 19;
 static constexpr uint32_t kSupHasLong = 2 * kSupHeads * kSupHeadStride;  // this word: a row is longer than kSupShort
 static constexpr uint32_t kSupTicketWords = kSupHasLong + 1;
