@@ -106,3 +106,22 @@ def test_per_row_in_batch(lstc, oracle):
         t_ref, rows_ref = oracle.count_k1(oracle.CSR(g.n, off, col))
         t, rows = lstc.count(g, per_row=True)
         assert t == t_ref and np.array_equal(rows, rows_ref)
+
+
+@pytest.mark.parametrize("scales", [(17, 17, 16, 17), (16,), (16, 16), (15, 14), (17, 12, 12)])
+def test_ticket_classes(lstc, oracle, scales):
+    """Both sides of the launch sizes (arcs per graph with in-lists, arcs without) that set the number of ticket heads."""
+    graphs = [oracle.gen_rmat(s, 16, seed=1) for s in scales]
+    want = [oracle.count(oracle.clean_orient(*g)[1]) for g in graphs]
+    up = lambda a: torch.from_numpy(np.ascontiguousarray(a).view(np.int32)).cuda()  # noqa: E731
+    for in_lists in (True, False):
+        gs = [lstc.clean_orient(n, up(s), up(d), in_lists=in_lists) for n, s, d in graphs]
+        plan = lstc.BatchPlan(gs)
+        try:
+            for _ in range(3):
+                plan.counts.fill_(3)
+                plan.launch_graph()
+                assert plan.results() == want
+        finally:
+            plan.close()
+        assert [lstc.count(g, split=in_lists) for g in gs] == want

@@ -74,11 +74,17 @@ static constexpr uint32_t kBigGroup = 2;              // big items per ticket
 // ticket b (no atomic) and goes on with its class, then with the others' leftovers.
 // A launch of a few hundred tickets then costs few atomics where every one of the
 // resident workgroups used to ask the one head (1009-vertex uniform graph: k_count
-// 39.5 -> 20 us), and launches of short items do not queue on one address (mixed
-// batch of 66 graphs: 3.02 ms with one class, 2.84 with eight; 64 served requests
-// 9.93 -> 9.31 ms).  Without in-lists the items are long and one class balances
-// them better (RMAT s21: 5.38 ms against 5.50).
-static constexpr uint32_t kHeads = 8;
+// 39.5 -> 20 us), and launches of short items do not queue on one address.  Long items are
+// balanced better by fewer classes (ms with 1, 4 and 8):
+//   mixed batch of 66 graphs 3.02, -, 2.84; 64 RMAT s14 1.30, 1.02, 0.98; RMAT s16 0.21, 0.17, 0.17
+//   8 Chung-Lu graphs of 100 thousand vertices 2.09, 2.11, 2.60; 8 RMAT s17 1.84, 1.88, 2.12;
+//   4 RMAT s18 1.55, 1.54, 1.64; 16 RMAT s17 3.21, 2.89, 3.12; 2 RMAT s21 6.65, 6.19, 6.27
+// so launches of graphs of kLongArcs arcs in the mean have kFewHeads.  Without in-lists the items
+// are longer still (RMAT s21 5.38 with one class, 5.50 with 8; 8 RMAT s17 1.70, 1.96), and
+// only launches below kShortArcs arcs have more than one class (20 thousand uniform vertices, 0.2M
+// arcs, 0.076, 0.047; RMAT s15, 0.4M, 0.089, 0.073; s16, 0.9M, 0.155, 0.158).
+static constexpr uint32_t kHeads = 8, kFewHeads = 4;
+static constexpr uint64_t kLongArcs = 3ull << 19, kShortArcs = 1ull << 19;
 static constexpr uint32_t kHeadStride = 32;  // words between heads
 
 // ctl (uint32) layout
@@ -208,7 +214,9 @@ __device__ __forceinline__ uint64_t umin64(uint64_t a, uint64_t b) { return a < 
 // 32-64 small tickets per workgroup (measured on RMAT s21 and s23: fewer,
 // larger tickets leave a ragged tail, more of them queue on the ticket heads).
 // A launch with less than 16 small items per workgroup takes one per wave, so
-// that its items spread over the chip (a 1009-vertex uniform graph has 2000).
+// that its items spread over the chip (a 1009-vertex uniform graph has 2000), unless the
+// tickets would then queue on one head (22500-vertex grid without in-lists, 0.071 ms then,
+// 0.060 with 16 per ticket; 0.056 now).
 __device__ __forceinline__ void plan_tickets(uint32_t *ctl, uint32_t n_big, uint32_t n_small, uint32_t n_tiny,
                                              uint32_t small_group, uint32_t grid, uint32_t waves, uint32_t classes,
                                              uint32_t tid) {
@@ -220,7 +228,7 @@ __device__ __forceinline__ void plan_tickets(uint32_t *ctl, uint32_t n_big, uint
         const uint32_t per_wg = n_small / (grid ? grid : 1u);
         sg = 16;
         while (sg < 64 && 2 * sg <= per_wg / 32) sg *= 2;
-        if (per_wg < 16) sg = waves;
+        if (per_wg < 16 && (classes > 1 || n_small <= grid * waves)) sg = waves;
     }
     ctl[C_SGROUP] = sg;
     const uint32_t small_t = (n_small + sg - 1) / sg;
@@ -1184,7 +1192,7 @@ lstc_status count_launch(const HostGraph *hosts, uint32_t G, const GraphDev *d_t
     if (fit && grid > (uint32_t)cus * fit) grid = (uint32_t)cus * fit;
     bool split = false;
     for (uint32_t g = 0; g < G; ++g) split = split || split_ok(hosts[g]);
-    const uint32_t classes = split ? kHeads : 1u;
+    const uint32_t classes = split ? (total_m < kLongArcs * G ? kHeads : kFewHeads) : total_m < kShortArcs ? kHeads : 1u;
     // Codes: one graph with in-lists and segment words, or counted without in-lists
     // and without per-row output, and a workspace that holds their arrays (count_ws_base is
     // still enough for k_count).  Whether its hubs cover its columns well enough is
