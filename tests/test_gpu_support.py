@@ -99,13 +99,12 @@ def test_support_split_item_edges(lstc, n):
     assert (sup == n - 2).all() and (pv == (n - 1) * (n - 2) // 2).all()
 
 
-@pytest.mark.parametrize("k", [64, 65, 66])
-def test_support_split_many_items(lstc, k):
-    """1200 complete graphs side by side, with longest rows on both sides of the length up to which waves take several
-    items at once, and enough items that they do."""
+@pytest.mark.parametrize("k,copies", [(64, 1200), (64, 2600), (12, 40_000), (9, 90_000)])
+def test_support_split_many_items(lstc, k, copies):
+    """Complete graphs side by side: items that waves take one by one, and in groups of 2, 6 and 8."""
     _, s, d = G.complete(k)
-    shift = np.arange(1200, dtype=np.uint32)[:, None] * np.uint32(k)
+    shift = np.arange(copies, dtype=np.uint32)[:, None] * np.uint32(k)
     up = lambda a: torch.from_numpy((a[None] + shift).astype(np.uint32).ravel().view(np.int32)).cuda()  # noqa: E731
-    g = lstc.clean_orient(1200 * k, up(s), up(d), in_lists=True)
+    g = lstc.clean_orient(copies * k, up(s), up(d), in_lists=True)
     sup, pv = lstc.triangle_support(g, split=True)
     assert (sup == k - 2).all() and (pv == (k - 1) * (k - 2) // 2).all()

@@ -445,25 +445,26 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 8 : 4) void k_support(cons
 // (1024: RMAT s23 85 against 92 ms, but RMAT s19 6.0 against 5.7 and Chung-Lu of 300
 // thousand vertices 8.0 against 6.7, which wait for their longest items.)
 static constexpr uint32_t kSupChunk = 512;
-// Items are dealt in kSupHeads classes (item t to class t % kSupHeads), each with its own head per kind on a
-// line of its own; a workgroup starts with class blockIdx % kSupHeads and goes on with the others' leftovers.
-// One head for all put a million tickets on one address: RMAT s21 25.4 ms, now 20.2, RMAT s23 119 -> 92. Where
-// no row is longer than kSupShort, waves take up to kSupMaxGroup items at once while many are left, one at the
-// end: a uniform graph of 600 thousand vertices, mean degree 40, 1.47 -> 0.81 ms.  Not where there are longer
-// rows, whose items then queue behind each other in one wave (groups of 8 / single items, ms: RMAT s17 1.83 /
-// 1.57, s18 3.15 / 2.55, s19 5.4 / 4.6, s21 20.8 / 20.2; Chung-Lu of 300 thousand vertices 6.7 / 5.1, of gamma
-// 2.5 and mean degree 150 12.0 / 10.0), unless there are so many rows that the tickets count again (kSupMany:
-// Chung-Lu of 1M vertices 12.9 / 12.6, 2.5M 25.0 / 26.8, 3M 28.2 / 30.6, RMAT s22 43.7 / 43.0, s23 92 / 92).
-// Eight waves per workgroup; four were no faster (s21 18.7 / 17.6 with groups).
-static constexpr uint32_t kSupHeads = 8, kSupHeadStride = 32, kSupMaxGroup = 8, kSupShort = 64, kSupMany = 3u << 19;
-static constexpr uint32_t kSupHasLong = 2 * kSupHeads * kSupHeadStride;  // this word: a row is longer than kSupShort
-static constexpr uint32_t kSupTicketWords = kSupHasLong + 1;
+// Items are dealt in kSupHeads classes (item t to class t % kSupHeads), each with
+// its own head per kind on a line of its own; a workgroup starts with class blockIdx %
+// kSupHeads and goes on with the others' leftovers.  One head for all put a million
+// tickets on one address: RMAT s21 25.4 ms, now 20.0, s23 119 -> 92.
+// A class of many items per wave deals them in groups of up to kSupMaxGroup and only the
+// last kSupSingle per wave one by one (see SupDeal); single items throughout: a uniform graph of 600
+// thousand vertices, mean degree 40, 1.43 ms for 0.81.  The items of a group lie far apart:
+// long items are often neighbours (RMAT, or vertices sorted by degree), and queue behind
+// each other in one wave when a group takes them side by side (side by side / single /
+// apart, ms: RMAT s17 1.76 / 1.46 / 1.46, s18 3.02 / 2.55 / 2.52, s19 5.45 / 4.6 / 4.87;
+// Chung-Lu of 300 thousand vertices 6.8 / 5.1 / 5.1, of gamma 2.5 and mean degree 150 12.5 / 10.0 / 9.7;
+// with the vertices renumbered at random RMAT s19 4.20 / 4.41 / 4.05, s20 8.0 / 8.3 / 8.1, Chung-Lu of 300
+// thousand vertices 2.63 / 2.48 / 2.90, 700 thousand 5.7 / 6.3 / 5.6).  Eight waves per workgroup;
+// four: s21 18.7 for 17.6 with groups side by side.
+static constexpr uint32_t kSupHeads = 8, kSupHeadStride = 32, kSupMaxGroup = 8, kSupSingle = 8;
 
 // Items per row, group rows and wave rows counted apart.
 __global__ void k_sup_items(const uint64_t *__restrict__ off, const uint64_t *__restrict__ in_off, uint32_t n_rows,
                             uint32_t n_owned, uint32_t wave_tile, uint32_t *__restrict__ items_g,
-                            uint32_t *__restrict__ items_w, uint32_t *__restrict__ ticket) {
-    bool has_long = false;
+                            uint32_t *__restrict__ items_w) {
     for (uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; r < n_rows; r += (uint64_t)gridDim.x * blockDim.x) {
         const uint64_t K = off[r + 1] - off[r], kb = in_off[r + 1] - in_off[r];
         const uint32_t nb = (uint32_t)((kb + kSupChunk - 1) / kSupChunk);
@@ -471,9 +472,7 @@ __global__ void k_sup_items(const uint64_t *__restrict__ off, const uint64_t *__
         const uint32_t it = K == 0 ? 0u : (nb > a ? nb : a);
         items_g[r] = K > wave_tile ? it : 0u;
         items_w[r] = K > wave_tile ? 0u : it;
-        has_long |= K > kSupShort;
     }
-    if (__syncthreads_or(has_long) && threadIdx.x == 0) ticket[kSupHasLong] = 1;
 }
 
 // item_row[t]: group items at [0, n_g), wave items at n_g + [0, n_w).
@@ -486,6 +485,21 @@ __global__ void k_sup_item_rows(const uint32_t *__restrict__ items_g, const uint
         for (uint32_t c = 0; c < items_w[r]; ++c) item_row[n_g + off_w[r] + c] = (uint32_t)r;
     }
 }
+
+// How a class deals its n items to its waves: in groups while there are many, then one
+// by one.  Ticket h of the groups has the items h, h + groups, h + 2 groups, ...
+struct SupDeal {
+    uint32_t group, groups, tickets;
+    __device__ __forceinline__ SupDeal(uint32_t n, uint32_t waves) {
+        group = max(1u, min(kSupMaxGroup, n / (8 * waves)));
+        groups = group > 1 ? (n - kSupSingle * waves) / group : 0u;
+        tickets = groups + (n - groups * group);
+    }
+    __device__ __forceinline__ uint32_t items(uint32_t h) const { return h < groups ? group : 1u; }
+    __device__ __forceinline__ uint32_t item(uint32_t h, uint32_t j) const {
+        return h < groups ? h + j * groups : groups * (group - 1) + h;
+    }
+};
 
 // A ticket head as it is now (it only grows, so an old value costs one atomic at most).
 __device__ __forceinline__ uint32_t sup_head(uint32_t *head) {
@@ -539,25 +553,21 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 8 : 4) void k_support_spli
         }
     }
     const SupTab Q = sup_wave_tab(L, wv);
-    const uint32_t most = ticket[kSupHasLong] && n_rows < kSupMany ? 1u : kSupMaxGroup;
-    const uint32_t share = gridDim.x * WAVES / kSupHeads * 4;  // a quarter of what is left per wave of the class
     for (uint32_t c = 0; c < kSupHeads; ++c) {  // wave items (every wave leaves once the items are taken)
         const uint32_t x = (blockIdx.x + c) % kSupHeads;
         const uint32_t n_x = n_w > x ? (n_w - x - 1) / kSupHeads + 1 : 0u;  // the class's items x, x + 8, ...
+        const SupDeal deal(n_x, gridDim.x * WAVES / kSupHeads);
         uint32_t *head = ticket + (kSupHeads + x) * kSupHeadStride;
-        for (uint32_t seen = c ? read_lane(sup_head(head), 0) : 0u; seen < n_x;) {
-            const uint32_t g = max(1u, min(most, (n_x - seen) / share));
-            uint32_t h = 0;
-            if (lane == 0) h = atomicAdd(head, g);
+        for (uint32_t h = c ? read_lane(sup_head(head), 0) : 0u; h < deal.tickets;) {
+            if (lane == 0) h = atomicAdd(head, 1u);
             h = read_lane(h, 0);
-            if (h >= n_x) break;
-            for (uint32_t i = h, e = min(h + g, n_x); i < e; ++i) {
-                const uint32_t t = i * kSupHeads + x, r = item_row[n_g + t];
+            if (h >= deal.tickets) break;
+            for (uint32_t j = 0; j < deal.items(h); ++j) {
+                const uint32_t t = deal.item(h, j) * kSupHeads + x, r = item_row[n_g + t];
                 sup_split_item<NARROW, 64, sup_wave_tile<WAVES>()>(Q, W, off, col, in_off, in_col, n_rows, n_owned, r,
                                                                    t - (uint32_t)off_w[r], support, per_vertex, nullptr,
                                                                    lane);
             }
-            seen = h + g;
         }
     }
 }
@@ -577,7 +587,7 @@ static SupLayout sup_layout(void *ws, size_t ws_bytes, uint32_t n_rows, uint64_t
     L.off_g = c.take<uint64_t>((size_t)n_rows + 1);
     L.off_w = c.take<uint64_t>((size_t)n_rows + 1);
     L.item_row = c.take<uint32_t>(2 * (size_t)n_rows + m / kSupChunk + 1);
-    L.ticket = c.take<uint32_t>(kSupTicketWords);
+    L.ticket = c.take<uint32_t>(2 * kSupHeads * kSupHeadStride);
     L.scan_bytes = scan_ws_bytes((uint64_t)n_rows + 1);
     L.scan_ws = c.take<char>(L.scan_bytes);
     L.bytes = c.need();
@@ -647,9 +657,9 @@ extern "C" lstc_status lstc_triangle_support_split(const uint64_t *d_off, const 
     if (d_per_vertex && n_rows) LSTC_TRY(fill_u64(d_per_vertex, 0, n_rows, st));
     if (n_rows == 0 || m == 0) return LSTC_OK;
     const uint32_t grid_n = (uint32_t)hmin<uint64_t>(((uint64_t)n_rows + 255) / 256, (uint64_t)device_cus() * 16);
-    LSTC_TRY(fill_u32(L.ticket, 0, kSupTicketWords, st));
+    LSTC_TRY(fill_u32(L.ticket, 0, 2 * kSupHeads * kSupHeadStride, st));
     hipLaunchKernelGGL(k_sup_items, dim3(grid_n), dim3(256), 0, st, d_off, d_in_off, n_rows, n_owned,
-                       sup_wave_tile<kSupSplitWaves>(), L.items_g, L.items_w, L.ticket);
+                       sup_wave_tile<kSupSplitWaves>(), L.items_g, L.items_w);
     LSTC_LAUNCHED("k_sup_items");
     LSTC_TRY(scan_exclusive_u32_to_u64(L.items_g, L.off_g, n_rows, L.off_g + n_rows, L.scan_ws, L.scan_bytes, st));
     LSTC_TRY(scan_exclusive_u32_to_u64(L.items_w, L.off_w, n_rows, L.off_w + n_rows, L.scan_ws, L.scan_bytes, st));
