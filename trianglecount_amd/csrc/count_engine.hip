@@ -994,8 +994,9 @@ __global__ __launch_bounds__(WAVES * 64, UNROLL == 4 ? 8 : 6) void k_count(Graph
 // The count over hub codes (hubcode.h), with in-lists (SPLIT) or without: every item is
 // one wave's, one wave per workgroup (9.1 KB of LDS: 16 waves per CU).
 //
-// What bounds it (RMAT s23, 8.8 ms; k_count took 16.9): the fabric behind the L2,
-// which delivers 7.2-7.8 TB/s here wherever the lines come from, so bytes and L2
+// What bounds it (RMAT s23, 8.8 ms; k_count took 16.9): the loads behind the L2, 6.7 TB/s of
+// them (k_count 7.2); the texture data unit is busy 99% of the time, 58% of it stalled on the
+// cache; so bytes and L2
 // hits are what counts.  k_count fetched 121 GB a launch.  16-bit codes and bitmaps
 // of the top hubs: 75 GB.  Parts of heavy rows per XCD and step (hubcode.h), so that
 // lists are met again while they are in L2: 62 GB; the same share of a row's own arcs
