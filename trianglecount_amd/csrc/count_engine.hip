@@ -85,6 +85,7 @@ static constexpr uint32_t kBigGroup = 2;              // big items per ticket
 // arcs, 0.076, 0.047; RMAT s15, 0.4M, 0.089, 0.073; s16, 0.9M, 0.155, 0.158).
 static constexpr uint32_t kHeads = 8, kFewHeads = 4;
 static constexpr uint64_t kLongArcs = 3ull << 19, kShortArcs = 1ull << 19;
+static constexpr uint64_t kFineArcs = 400;  // arcs per ticket of single items on one head (plan_tickets)
 static constexpr uint32_t kHeadStride = 32;  // words between heads
 
 // ctl (uint32) layout
@@ -214,12 +215,13 @@ __device__ __forceinline__ uint64_t umin64(uint64_t a, uint64_t b) { return a < 
 // 32-64 small tickets per workgroup (measured on RMAT s21 and s23: fewer,
 // larger tickets leave a ragged tail, more of them queue on the ticket heads).
 // A launch with less than 16 small items per workgroup takes one per wave, so
-// that its items spread over the chip (a 1009-vertex uniform graph has 2000), unless the
-// tickets would then queue on one head (22500-vertex grid without in-lists, 0.071 ms then,
-// 0.060 with 16 per ticket; 0.056 now).
+// that its items spread over the chip (a 1009-vertex uniform graph has 2000), if that makes
+// at most `fine` tickets: with one head, more of them queue on it unless the items are
+// long (uniform graphs without in-lists, 16 / 1 item per wave: 30 thousand vertices of mean degree 40
+// 0.054 / 0.108 ms, 15 thousand of 100 0.071 / 0.078, 20 thousand of 200 0.175 / 0.153).
 __device__ __forceinline__ void plan_tickets(uint32_t *ctl, uint32_t n_big, uint32_t n_small, uint32_t n_tiny,
                                              uint32_t small_group, uint32_t grid, uint32_t waves, uint32_t classes,
-                                             uint32_t tid) {
+                                             uint32_t fine, uint32_t tid) {
     if (tid < classes) ctl[C_HEADS + tid * kHeadStride] = (grid + classes - 1 - tid) / classes;
     if (tid != 0) return;
     ctl[C_CLASSES] = classes;
@@ -228,7 +230,7 @@ __device__ __forceinline__ void plan_tickets(uint32_t *ctl, uint32_t n_big, uint
         const uint32_t per_wg = n_small / (grid ? grid : 1u);
         sg = 16;
         while (sg < 64 && 2 * sg <= per_wg / 32) sg *= 2;
-        if (per_wg < 16 && (classes > 1 || n_small <= grid * waves)) sg = waves;
+        if (per_wg < 16 && n_small <= (uint64_t)fine * waves) sg = waves;
     }
     ctl[C_SGROUP] = sg;
     const uint32_t small_t = (n_small + sg - 1) / sg;
@@ -354,7 +356,7 @@ __global__ __launch_bounds__(256) void k_plan_rows(GraphSet gs, Bounds bd, uint3
 __global__ __launch_bounds__(1024) void k_plan_scan(uint32_t *__restrict__ wcnt, uint32_t *__restrict__ ctl,
                                                     unsigned long long *__restrict__ counts, uint32_t G,
                                                     uint32_t small_group, uint32_t grid, uint32_t waves, uint32_t classes,
-                                                    HubSet hs, uint32_t hub_grid) {
+                                                    uint32_t fine, HubSet hs, uint32_t hub_grid) {
     if (hs.hctl && sload(hs.hctl + HC_ON)) return hub_plan_scan(hs, counts, hub_grid);
     constexpr uint32_t kPer = (kPlanEntries + 4095) / 4096 * 4;  // 16-byte loads and stores
     static_assert(kPlanEntries % 4 == 0, "plan entries come in whole 16-byte words");
@@ -396,7 +398,7 @@ __global__ __launch_bounds__(1024) void k_plan_scan(uint32_t *__restrict__ wcnt,
     __syncthreads();
     for (uint32_t i = tid; i < G; i += 1024) counts[i] = 0;
     // slots 0..2 hold bins 5,4,3 (big), slots 3..5 bins 2,1,0 (small), slot 6 the tiny rows
-    plan_tickets(ctl, s_slot[3], s_slot[6] - s_slot[3], s_slot[7] - s_slot[6], small_group, grid, waves, classes, tid);
+    plan_tickets(ctl, s_slot[3], s_slot[6] - s_slot[3], s_slot[7] - s_slot[6], small_group, grid, waves, classes, fine, tid);
 }
 
 // The whole plan of a launch of at most kSmallPlan rows in one workgroup: the
@@ -408,7 +410,7 @@ static constexpr uint32_t kSmallPlan = 1024 * kSmallPlanPer;
 __global__ __launch_bounds__(1024) void k_plan_small(GraphSet gs, Bounds bd, uint32_t *__restrict__ ctl,
                                                      unsigned long long *__restrict__ queue,
                                                      unsigned long long *__restrict__ counts, uint32_t small_group,
-                                                     uint32_t grid, uint32_t waves, uint32_t classes) {
+                                                     uint32_t grid, uint32_t waves, uint32_t classes, uint32_t fine) {
     __shared__ uint32_t s_wave[kSlots][16];
     const uint32_t tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     RowPlan p[kSmallPlanPer];
@@ -452,7 +454,7 @@ __global__ __launch_bounds__(1024) void k_plan_small(GraphSet gs, Bounds bd, uin
         if (s == 5) n_small = base - n_big;
     }
     for (uint32_t i = tid; i < gs.G; i += 1024) counts[i] = 0;
-    plan_tickets(ctl, n_big, n_small, base - n_big - n_small, small_group, grid, waves, classes, tid);
+    plan_tickets(ctl, n_big, n_small, base - n_big - n_small, small_group, grid, waves, classes, fine, tid);
 }
 
 // ------------------------------------------------------------------ table build
@@ -1194,6 +1196,7 @@ lstc_status count_launch(const HostGraph *hosts, uint32_t G, const GraphDev *d_t
     bool split = false;
     for (uint32_t g = 0; g < G; ++g) split = split || split_ok(hosts[g]);
     const uint32_t classes = split ? (total_m < kLongArcs * G ? kHeads : kFewHeads) : total_m < kShortArcs ? kHeads : 1u;
+    const uint32_t fine = classes > 1 ? 0xFFFFFFFFu : hmax(grid, (uint32_t)(total_m / kFineArcs));
     // Codes: one graph with in-lists and segment words, or counted without in-lists
     // and without per-row output, and a workspace that holds their arrays (count_ws_base is
     // still enough for k_count).  Whether its hubs cover its columns well enough is
@@ -1212,13 +1215,13 @@ lstc_status count_launch(const HostGraph *hosts, uint32_t G, const GraphDev *d_t
     const uint32_t *hub_on = hub_grid ? hs.hctl + HC_ON : nullptr;
     if (total <= kSmallPlan && !hub_grid) {
         hipLaunchKernelGGL(k_plan_small, dim3(1), dim3(1024), 0, st, gs, bd, ctl, queue, d_counts, tr.small_group, grid,
-                           tr.waves, classes);
+                           tr.waves, classes, fine);
         LSTC_LAUNCHED("k_plan_small");
     } else {
         hipLaunchKernelGGL(k_plan_rows<0>, dim3(kPlanBlocks), dim3(256), 0, st, gs, bd, wcnt, queue, hs);
         LSTC_LAUNCHED("k_plan_rows<0>");
         hipLaunchKernelGGL(k_plan_scan, dim3(1), dim3(1024), 0, st, wcnt, ctl, d_counts, G, tr.small_group, grid,
-                           tr.waves, classes, hs, hub_grid);
+                           tr.waves, classes, fine, hs, hub_grid);
         LSTC_LAUNCHED("k_plan_scan");
         hipLaunchKernelGGL(k_plan_rows<1>, dim3(kPlanBlocks), dim3(256), 0, st, gs, bd, wcnt, queue, hs);
         LSTC_LAUNCHED("k_plan_rows<1>");
